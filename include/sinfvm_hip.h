@@ -170,8 +170,8 @@ int sfv_advance(sfv_handle* h, int64_t nsteps, double max_dt, double* t_io);
  * memory).  *t_io is the start time on entry and the end time on exit;
  * *dt_out (may be NULL) receives the last step's dt.  The scratch the steps
  * need (the stage right-hand side, the second state of the ping-pong pair and
- * the step-control block) is one static device array of
- * SFV_NOALLOC_SCRATCH_BYTES that each GPU the library runs on holds until the
+ * the step-control block) is static device memory, SFV_NOALLOC_SCRATCH_BYTES
+ * for the first two, that each GPU the library runs on holds until the
  * process ends: grids of at most 1,398,085 cells ghosts included (f64;
  * 2,796,170 with f32 storage) are accepted, larger ones return
  * SFV_ERR_DOMAIN.  The configuration must suit the fused RK2 kernels:

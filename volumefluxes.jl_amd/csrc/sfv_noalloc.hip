@@ -5,11 +5,11 @@
 // step, the boundary condition when the loop ends) need, besides the state
 // and the topography the caller passes, three scratch buffers: the stage
 // right-hand side (3 planes), the other state of the ping-pong pair and the
-// step-control block.  Here they live in one file-scope device array,
-// `scratch`, which every GPU the library runs on holds from module load until
-// the process ends.  Its device address is looked up once per device with
-// hipGetSymbolAddress (the array's name in host code is not a device
-// address) and cached; kernels and copies only ever see that address.
+// step-control block.  Here they live in file-scope device arrays, `scratch`
+// (the first two) and `ctl_scratch`, which every GPU the library runs on holds
+// from module load until the process ends.  Their device addresses are looked
+// up once per device with hipGetSymbolAddress (an array's name in host code is
+// not a device address) and cached; kernels and copies only ever see those.
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
@@ -21,14 +21,21 @@
 
 namespace {
 
-constexpr size_t CTL_BYTES = 256;                // StepCtl, padded to the array's alignment
-static_assert(sizeof(sfv::StepCtl) <= CTL_BYTES, "StepCtl outgrew its scratch slot");
+constexpr size_t CTL_BYTES = 256;                // ahead of the right-hand side (unused)
+constexpr size_t CTL_ARRAY = 4096;
+static_assert(sizeof(sfv::StepCtl) <= CTL_ARRAY, "StepCtl outgrew its array");
 
 static __device__ __align__(256) unsigned char scratch[SFV_NOALLOC_SCRATCH_BYTES];
+static __device__ __align__(256) unsigned char ctl_scratch[CTL_ARRAY];
 
 constexpr int MAX_DEVICES = 64;
 std::mutex g_mu;
-void* g_scratch[MAX_DEVICES] = {};               // device address of `scratch` per device
+// device addresses of `scratch` and `ctl_scratch` per device
+struct Scratch {
+    void* state = nullptr;
+    void* ctl = nullptr;
+};
+Scratch g_scratch[MAX_DEVICES];
 
 int fail(int code, const std::string& msg) {
     sfv::set_call_error(msg);          // read with sfv_create_error()
@@ -44,15 +51,16 @@ int64_t max_cells(int32_t precision) {
 
 size_t round_up(size_t b) { return (b + 255) / 256 * 256; }
 
-// The address of this device's `scratch`, looked up on the device's first call.
-int scratch_of(int dev, void** out) {
+// The addresses of this device's arrays, looked up on the device's first call.
+int scratch_of(int dev, Scratch* out) {
     std::lock_guard<std::mutex> lk(g_mu);
-    if (!g_scratch[dev]) {
-        void* p = nullptr;
-        const hipError_t e = hipGetSymbolAddress(&p, HIP_SYMBOL(scratch));
-        if (e != hipSuccess || !p)
+    if (!g_scratch[dev].state) {
+        Scratch s;
+        hipError_t e = hipGetSymbolAddress(&s.state, HIP_SYMBOL(scratch));
+        if (e == hipSuccess) e = hipGetSymbolAddress(&s.ctl, HIP_SYMBOL(ctl_scratch));
+        if (e != hipSuccess || !s.state || !s.ctl)
             return fail(SFV_ERR_HIP, std::string("hipGetSymbolAddress(scratch): ") + hipGetErrorString(e));
-        g_scratch[dev] = p;
+        g_scratch[dev] = s;
     }
     *out = g_scratch[dev];
     return SFV_OK;
@@ -65,12 +73,12 @@ int scratch_of(int dev, void** out) {
     } while (0)
 
 template <class S>
-int advance(const sfv::KParams& P, hipStream_t st, void* base, const double* B, S* U, int64_t nsteps, double max_dt,
+int advance(const sfv::KParams& P, hipStream_t st, const Scratch& scr, const double* B, S* U, int64_t nsteps, double max_dt,
             double t0, double* t_out, double* dt_out) {
     using namespace sfv;
     const size_t n3 = 3 * (size_t)P.nxT * P.nyT;
-    StepCtl* ctl = (StepCtl*)base;
-    S* RHS = (S*)((unsigned char*)base + CTL_BYTES);
+    StepCtl* ctl = (StepCtl*)scr.ctl;
+    S* RHS = (S*)((unsigned char*)scr.state + CTL_BYTES);
     S* other = (S*)((unsigned char*)RHS + round_up(n3 * sizeof(S)));
     S* buf[2] = {U, other};
     // the step control is armed by a kernel (no memset): every field a step
@@ -129,7 +137,7 @@ int sfv_advance_noalloc(const sfv_config* cfg, const double* B_dev, void* U_dev,
     int dev = 0;
     NA_TRY(hipGetDevice(&dev));
     if (dev < 0 || dev >= MAX_DEVICES) return fail(SFV_ERR_HIP, "device index out of range");
-    void* base = nullptr;
+    Scratch base;
     const int rs = scratch_of(dev, &base);
     if (rs) return rs;
     sfv::KParams P;

@@ -543,8 +543,8 @@ __global__ void __launch_bounds__(256) k_adj_tail(KParams P, const StepCtl* ctl,
 // The direction whose wave speed set dt: min(Δx/a_x, Δy/a_y) picks y on a
 // tie (simulator.jl:147-150 with Julia's minimum).
 __device__ __forceinline__ int dt_direction(const KParams& P, const StepCtl* ctl) {
-    const double ax = __longlong_as_double((long long)ctl->slot[0].wsmax[0]);
-    const double ay = __longlong_as_double((long long)ctl->slot[0].wsmax[1]);
+    const double ax = __longlong_as_double((long long)slot_wsmax(ctl->slot[0], 0));
+    const double ay = __longlong_as_double((long long)slot_wsmax(ctl->slot[0], 1));
     return (P.dx / ax < P.dy / ay) ? 0 : 1;
 }
 
@@ -588,7 +588,7 @@ __global__ void __launch_bounds__(256) k_adj_faces(KParams P, int d, const doubl
     // each face at the maximum offers its interior cells and the smallest
     // memory index wins.
     if (best && d == dt_direction(P, ctl) &&
-        (unsigned long long)__double_as_longlong(speed) == ctl->slot[0].wsmax[d]) {
+        (unsigned long long)__double_as_longlong(speed) == slot_wsmax(ctl->slot[0], d)) {
         unsigned long long c = ~0ull;
         if (c_in) c = kc;
         if (c1_in && k1 < c) c = k1;
@@ -749,15 +749,15 @@ __global__ void __launch_bounds__(256) k_adj_dtstep(KParams P, const StepCtl* ct
     *cz_total += red[1][0];
     const unsigned long long kbest = *best;
     {
-        const double ax = __longlong_as_double((long long)ctl->slot[0].wsmax[0]);
-        const double ay = __longlong_as_double((long long)ctl->slot[0].wsmax[1]);
+        const double ax = __longlong_as_double((long long)slot_wsmax(ctl->slot[0], 0));
+        const double ay = __longlong_as_double((long long)slot_wsmax(ctl->slot[0], 1));
         const bool armed = __builtin_isfinite(ax) && __builtin_isfinite(ay) && (ax > 0.0 || ay > 0.0);
         if (armed && kbest == ~0ull) *flag = 1;
     }
     const int d = dt_direction(P, ctl);
     if (kbest >= (unsigned long long)P.nxT * P.nyT) return;
     const int i = (int)(kbest % P.nxT), j = (int)(kbest / P.nxT);
-    const double ax = __longlong_as_double((long long)ctl->slot[0].wsmax[d]);
+    const double ax = __longlong_as_double((long long)slot_wsmax(ctl->slot[0], d));
     if (!(ax > 0.0) || !__builtin_isfinite(ax)) return;
     double sr, sl;
     face_speeds(P, U, B, d, i, j, sr, sl);

@@ -79,8 +79,7 @@ __device__ void prepare_ctl(const KParams& P, StepCtl* c, int slot, double t, do
     bool act = true;
     if (until_endtime) act = t < endtime;
     for (int s = 0; s < 2; ++s) {
-        c->slot[s].wsmax[0] = 0ull;
-        c->slot[s].wsmax[1] = 0ull;
+        clear_wsmax(c->slot[s]);
         c->slot[s].active = 0;
         set_rates(P, c->slot[s], t);
     }

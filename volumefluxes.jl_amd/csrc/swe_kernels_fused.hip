@@ -194,8 +194,7 @@ __device__ __forceinline__ void block_max2(unsigned long long sx, unsigned long 
             mx = red[0][w] > mx ? red[0][w] : mx;
             my = red[1][w] > my ? red[1][w] : my;
         }
-        if (mx) atomicMax(&slot->wsmax[0], mx);
-        if (my) atomicMax(&slot->wsmax[1], my);
+        raise_wsmax(slot, mx, my);
     }
 }
 

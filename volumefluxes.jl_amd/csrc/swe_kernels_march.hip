@@ -185,12 +185,9 @@ __device__ __forceinline__ unsigned long long wave_max_u64m(unsigned long long v
 // Stage 1's wave-speed maxima of one block (its 4 waves) into the step slot.
 // Every wave of the block calls this exactly once per tile, also a wave whose
 // segment lies past the grid (with zeros): the maxima meet in LDS behind a
-// barrier and one lane does the atomics.  Per-wave atomics on the slot's two
-// addresses serialised when hundreds of short waves ended together (small
-// grids); one per block is a quarter of them.  `par` alternates between
-// consecutive tiles of a persistent block so the next tile's writes never
-// meet this tile's reads.  The maxima are reached by a few blocks early on:
-// the atomic is skipped when the slot already holds at least this value.
+// barrier and one lane raises the slot's line of this XCD.  `par` alternates
+// between consecutive tiles of a persistent block so the next tile's writes
+// never meet this tile's reads.
 __device__ __forceinline__ void block_max_to_slot_m(unsigned long long smx, unsigned long long smy, StepSlot* s,
                                                     int par) {
     __shared__ unsigned long long red[2][MWAVES][2];
@@ -208,10 +205,7 @@ __device__ __forceinline__ void block_max_to_slot_m(unsigned long long smx, unsi
             smx = red[par][k][0] > smx ? red[par][k][0] : smx;
             smy = red[par][k][1] > smy ? red[par][k][1] : smy;
         }
-        const unsigned long long cx = __hip_atomic_load(&s->wsmax[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        const unsigned long long cy = __hip_atomic_load(&s->wsmax[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (smx > cx) atomicMax(&s->wsmax[0], smx);
-        if (smy > cy) atomicMax(&s->wsmax[1], smy);
+        raise_wsmax(s, smx, smy);
     }
 }
 

@@ -33,8 +33,7 @@ __device__ void block_max_to_slot(unsigned long long sx, unsigned long long sy, 
     if (tid == 0) {
         unsigned long long mx = red[0][0], my = red[1][0];
         for (int w = 1; w < nw; ++w) { mx = red[0][w] > mx ? red[0][w] : mx; my = red[1][w] > my ? red[1][w] : my; }
-        if (mx) atomicMax(&slot->wsmax[0], mx);
-        if (my) atomicMax(&slot->wsmax[1], my);
+        raise_wsmax(slot, mx, my);
     }
 }
 

@@ -213,25 +213,25 @@ int sfv_device_count(void);
 /* Select the kernels of a step for this handle: 2 = fused RK2 stage kernels,
  * one wavefront per 60-column strip marching in y (the default whenever the
  * boundary-condition sources of the ghost cells are interior cells; unless a
- * variant is set here, the first step's tuning switches to 1 when that is
- * faster for the grid); 1 = fused RK2 stage kernels tiled through LDS; 3 =
- * every right-hand side from
- * the march stage-1 kernel, the updates and boundary conditions from the
- * per-pass kernels (any stepper and boundary condition with gc >= 2: the
- * default for NeumannBC and ForwardEuler); 0 = one kernel per reference pass
- * (the device-side reference).  All give bitwise identical results.  No
- * counterpart in the reference. */
+ * variant is set here, the first step switches to 1 where that suits the
+ * grid); 1 = the same stages with one workgroup per strip segment, for grids
+ * too small to fill the device; 3 = every right-hand side from the stage-1
+ * kernel, the updates and boundary conditions from the per-pass kernels (any
+ * stepper and boundary condition with gc >= 2: the default for NeumannBC and
+ * ForwardEuler); 0 = one kernel per reference pass (the device-side
+ * reference).  All give bitwise identical results.  No counterpart in the
+ * reference. */
 int sfv_set_fused(sfv_handle* h, int32_t fused);
 /* The kernel variant a step of this handle runs (0 to 3 as above; -1 for a
  * NULL handle).  No counterpart in the reference. */
 int32_t sfv_get_fused(const sfv_handle* h);
 
 /* Rows per wave segment of the march kernels (sfv_set_fused(h, 2)).  0 (the
- * default) lets the library choose on the first step: candidate heights are
- * timed on the handle's own state and the fastest is kept for grids of that
- * size class (quarter octaves of nx and ny) on that device; the environment
- * variable SFV_AUTOTUNE=0 turns the measurement off (the height that makes
- * the launch's workgroups the fewest rounds of resident workgroups is used).
+ * default) lets the library choose on the first step (on grids that take the
+ * workgroup kernels, without a measurement): candidate heights are timed on
+ * the handle's own state and the fastest is kept for grids of that size class
+ * (quarter octaves of nx and ny) on that device; the environment variable
+ * SFV_AUTOTUNE=0 turns the measurement off (the height that makes the launch shortest by the waves it puts on each SIMD is used).
  * rows > 0 forces a height.  Results are bitwise the same for every height.
  * No counterpart in the reference. */
 int sfv_set_march_rows(sfv_handle* h, int32_t rows);

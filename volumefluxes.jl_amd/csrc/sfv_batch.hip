@@ -61,12 +61,12 @@ int BatchEngine::init(int precision, int capacity, std::string& why) {
     if (hipGetDeviceProperties(&prop, device_) == hipSuccess && prop.multiProcessorCount > 0)
         cus = prop.multiProcessorCount;
     cus_ = cus;
-    per_cu_ = std::min(march_batch_blocks_per_cu(precision, 1), march_batch_blocks_per_cu(precision, 2));
     size_grid();
     return grow(std::max(1, capacity), why);
 }
 
 void BatchEngine::size_grid() {
+    per_cu_ = std::min(march_batch_blocks_per_cu(precision_, 1, mode_), march_batch_blocks_per_cu(precision_, 2, mode_));
     const int per = share_ == Share::ALONE ? per_cu_ : share_ == Share::HOST ? std::max(1, per_cu_ - 1) : 1;
     blocks_stage_ = std::max(8, (cus_ * per + 7) / 8 * 8);
 }
@@ -328,11 +328,11 @@ int BatchEngine::capture(std::string& why) {
     for (int s = 0; s < graph_steps_ && e == hipSuccess; ++s) {
         const int lp = s & 1;
         if (precision_ == SFV_F64) {
-            e = launch_march_batch<double>(stream_, 1, d_mem_, d_hdr_, lp, blocks_stage_, fast_);
-            if (e == hipSuccess) e = launch_march_batch<double>(stream_, 2, d_mem_, d_hdr_, lp, blocks_stage_, fast_);
+            e = launch_march_batch<double>(stream_, 1, d_mem_, d_hdr_, lp, blocks_stage_, mode_);
+            if (e == hipSuccess) e = launch_march_batch<double>(stream_, 2, d_mem_, d_hdr_, lp, blocks_stage_, mode_);
         } else {
-            e = launch_march_batch<float>(stream_, 1, d_mem_, d_hdr_, lp, blocks_stage_, fast_);
-            if (e == hipSuccess) e = launch_march_batch<float>(stream_, 2, d_mem_, d_hdr_, lp, blocks_stage_, fast_);
+            e = launch_march_batch<float>(stream_, 1, d_mem_, d_hdr_, lp, blocks_stage_, mode_);
+            if (e == hipSuccess) e = launch_march_batch<float>(stream_, 2, d_mem_, d_hdr_, lp, blocks_stage_, mode_);
         }
     }
     hipGraph_t g = nullptr;
@@ -357,13 +357,16 @@ int BatchEngine::replay_begin(int k, std::string& why) {
     int rc;
     if (table_dirty_) {
         // the graph holds the specialised kernels only while every member fits them
-        bool fast = !rows_.empty();
-        for (int s : rows_) fast = fast && march_fast(slot_handle_[s]->P);
-        if (graph_ && fast != fast_) {
-            (void)hipGraphExecDestroy(graph_);
-            graph_ = nullptr;
+        int mode = rows_.empty() ? 0 : MAX_MODE;
+        for (int s : rows_) mode = std::min(mode, march_mode(slot_handle_[s]->P));
+        if (mode != mode_) {
+            mode_ = mode;
+            size_grid();                   // the kernels' residency differs
+            if (graph_) {
+                (void)hipGraphExecDestroy(graph_);
+                graph_ = nullptr;
+            }
         }
-        fast_ = fast;
         if (members_changed_) {
             members_changed_ = false;
             plan_tuning();

@@ -45,26 +45,32 @@ int step_kernels(sfv_handle* h, int slot, int cur) {
     S* U2 = (S*)h->U[cur ^ 1];
     S* RHS = (S*)h->RHS;
     if (h->fused == KV_HYBRID) {
+        // stage-1 right-hand sides from the workgroup kernels where they suit
+        // the grid and no segment height was asked for
+        auto rhs = [&](const S* X, int remap) {
+            return h->rows_forced ? launch_march<S>(st, P, h->ctl, slot, 1, X, nullptr, RHS, h->B, 0, remap)
+                                  : launch_stage<S>(st, P, h->ctl, slot, 1, X, nullptr, RHS, h->B, 0, remap);
+        };
         // the second stage-1 launch also raises this slot's wave-speed maxima,
         // after dt was taken from them; the slot is re-armed before its next use
         if (h->cfg.stepper == SFV_FORWARD_EULER && h->ghost_sources_interior()) {
             // two launches: stage 1 reads ghosts through the boundary maps and
             // the update closes the step; ghosts are filled when the loop ends
-            HIP_TRY(h, launch_march<S>(st, P, h->ctl, slot, 1, U0, nullptr, RHS, h->B, 0, 1));
+            HIP_TRY(h, rhs(U0, 1));
             HIP_TRY(h, launch_finish<S>(st, P, h->ctl, slot, 1, U0, U0, RHS, U2, h->B, 1, 1));
             return SFV_OK;
         }
         if (h->cfg.stepper == SFV_FORWARD_EULER) {
-            HIP_TRY(h, launch_march<S>(st, P, h->ctl, slot, 1, U0, nullptr, RHS, h->B));
+            HIP_TRY(h, rhs(U0, 0));
             HIP_TRY(h, launch_finish<S>(st, P, h->ctl, slot, 1, U0, U0, RHS, U2, h->B, 1));
             HIP_TRY(h, launch_bc<S>(st, P, h->ctl, slot, U2, BC_LAST_STAGE));
             return SFV_OK;
         }
         S* U1 = (S*)h->U[2];
-        HIP_TRY(h, launch_march<S>(st, P, h->ctl, slot, 1, U0, nullptr, RHS, h->B));
+        HIP_TRY(h, rhs(U0, 0));
         HIP_TRY(h, launch_finish<S>(st, P, h->ctl, slot, 1, U0, U0, RHS, U1, h->B, 1));
         HIP_TRY(h, launch_bc<S>(st, P, h->ctl, slot, U1, BC_IN_STEP));
-        HIP_TRY(h, launch_march<S>(st, P, h->ctl, slot, 1, U1, nullptr, RHS, h->B));
+        HIP_TRY(h, rhs(U1, 0));
         HIP_TRY(h, launch_finish<S>(st, P, h->ctl, slot, 2, U0, U1, RHS, U2, h->B, 1));
         HIP_TRY(h, launch_bc<S>(st, P, h->ctl, slot, U2, BC_LAST_STAGE));
         return SFV_OK;
@@ -83,8 +89,8 @@ int step_kernels(sfv_handle* h, int slot, int cur) {
         return SFV_OK;
     }
     if (h->fused == KV_TILED) {      // as the march path: ghosts through the maps, stage 2 closes
-        HIP_TRY(h, launch_stage1<S>(st, P, h->ctl, slot, U0, RHS, h->B));
-        HIP_TRY(h, launch_stage2<S>(st, P, h->ctl, slot, U0, RHS, U2, h->B, 1));
+        HIP_TRY(h, launch_block<S>(st, P, h->ctl, slot, 1, U0, nullptr, RHS, h->B, 0, 1));
+        HIP_TRY(h, launch_block<S>(st, P, h->ctl, slot, 2, U0, RHS, U2, h->B, 1));
         return SFV_OK;
     }
     S* U1 = (S*)h->U[2];
@@ -135,14 +141,14 @@ int ensure_ready(sfv_handle* h) {
 // timed on the handle itself (full steps from its current state into the
 // spare ping-pong buffer, which the next step overwrites anyway), and the
 // winner is cached per device, precision and grid size class (quarter
-// octaves of nx and ny).  A march handle whose kernel variant was not set
-// with sfv_set_fused also times the LDS-tiled kernels, which step grids of
-// roughly 200^2 to 512^2 faster (more waves, each with a shorter serial path),
-// and switches to them when they win.  Handles on the hybrid path (ForwardEuler,
-// NeumannBC) run only the stage-1 kernel, so they time it alone and keep
+// octaves of nx and ny).  Where the workgroup kernels suit the grid
+// (block_suits), nothing is measured: a march handle whose kernel variant was
+// not set with sfv_set_fused switches to them.  Handles on the hybrid path
+// (ForwardEuler, NeumannBC) run only the stage-1 kernel, so they time it alone
+// and keep
 // their own cache entries.  Every height gives bitwise the same results.
 // SFV_AUTOTUNE=0 in the environment keeps the height model's choice
-// (march_rows_per_wave: the fewest rounds of resident workgroups).
+// (march_rows_per_wave).
 struct TuneKey {
     int dev, prec, bx, by, kind;   // kind: 0 full march steps, 1 stage 1 only
     bool operator<(const TuneKey& o) const {
@@ -154,12 +160,12 @@ struct TuneKey {
     }
 };
 std::mutex g_tune_mu;
-std::map<TuneKey, int> g_tuned;   // the march height; negative: the tiled kernels won (height = its magnitude)
+std::map<TuneKey, int> g_tuned;   // the march height
 
 int size_bucket(int n) { return (int)std::lround(4.0 * std::log2((double)std::max(n, 1))); }
 
 template <class S>
-hipError_t tune_steps(sfv_handle* h, int slot, int n, bool tiled) {
+hipError_t tune_steps(sfv_handle* h, int slot, int n) {
     const KParams& P = h->P;
     const int cur = (int)(h->cur & 1);
     const S* U0 = (const S*)h->U[cur];
@@ -167,11 +173,6 @@ hipError_t tune_steps(sfv_handle* h, int slot, int n, bool tiled) {
     S* Us = (S*)h->U[cur ^ 1];
     hipError_t e = hipSuccess;
     for (int k = 0; k < n && e == hipSuccess; ++k) {
-        if (tiled) {
-            e = launch_stage1<S>(h->stream, P, h->ctl, slot, U0, R, h->B);
-            if (e == hipSuccess) e = launch_stage2<S>(h->stream, P, h->ctl, slot, U0, R, Us, h->B);   // not closing
-            continue;
-        }
         e = launch_march<S>(h->stream, P, h->ctl, slot, 1, U0, nullptr, R, h->B, 0, h->ghost_sources_interior() ? 1 : 0);
         if (h->fused == KV_HYBRID) continue;
         if (e == hipSuccess) e = launch_march<S>(h->stream, P, h->ctl, slot, 2, U0, R, Us, h->B);   // not closing
@@ -264,21 +265,19 @@ int cached_march_rows(sfv_handle* h) {
     std::lock_guard<std::mutex> lk(g_tune_mu);
     auto it = g_tuned.find(key);
     if (it == g_tuned.end()) return 0;
-    const int rows = it->second < 0 ? -it->second : it->second;
-    h->march_rows = rows;
-    h->P.rows = rows;
-    if (it->second < 0 && !h->variant_forced && h->fused == KV_MARCH) h->fused = KV_TILED;
-    return rows;
+    h->march_rows = it->second;
+    h->P.rows = it->second;
+    return it->second;
 }
 
 int tune_march_rows(sfv_handle* h, std::string& why) {
     if ((h->fused != KV_MARCH && h->fused != KV_HYBRID) || h->march_rows > 0) return SFV_OK;
-    // a march handle whose variant the caller left open also times the tiled kernels
-    const bool try_tiled = h->fused == KV_MARCH && !h->variant_forced;
+    const bool block = !h->variant_forced && block_suits(h->P);
     const int fallback = march_rows_per_wave(h->P, 1, h->cfg.precision == SFV_F64 ? 0 : 1);
-    if (!autotune_enabled()) {
+    if (block || !autotune_enabled()) {
         h->march_rows = fallback;
         h->P.rows = fallback;
+        if (block && h->fused == KV_MARCH) h->fused = KV_TILED;
         return SFV_OK;
     }
     if (cached_march_rows(h) > 0) return SFV_OK;
@@ -308,11 +307,11 @@ int tune_march_rows(sfv_handle* h, std::string& why) {
         e = launch_prepare(h->stream, h->P, h->ctl, slot, 0.0, NAN, 0, 0, 0.0, -1, 0, h->cfg.precision);
     // time n steps with `rows`; the first call also sizes n so one
     // measurement covers about a millisecond
-    auto timed = [&](int rows, int n, double& ms_out, bool tiled = false) -> hipError_t {
+    auto timed = [&](int rows, int n, double& ms_out) -> hipError_t {
         h->P.rows = rows;
-        hipError_t r = f64 ? tune_steps<double>(h, slot, 1, tiled) : tune_steps<float>(h, slot, 1, tiled);  // warm-up
+        hipError_t r = f64 ? tune_steps<double>(h, slot, 1) : tune_steps<float>(h, slot, 1);  // warm-up
         if (r == hipSuccess) r = hipEventRecord(e0, h->stream);
-        if (r == hipSuccess) r = f64 ? tune_steps<double>(h, slot, n, tiled) : tune_steps<float>(h, slot, n, tiled);
+        if (r == hipSuccess) r = f64 ? tune_steps<double>(h, slot, n) : tune_steps<float>(h, slot, n);
         if (r == hipSuccess) r = hipEventRecord(e1, h->stream);
         if (r == hipSuccess) r = hipEventSynchronize(e1);
         float ms = 0;
@@ -324,17 +323,11 @@ int tune_march_rows(sfv_handle* h, std::string& why) {
     if (e == hipSuccess) e = timed(fallback, 2, probe);
     const int n = (int)std::min(32.0, std::max(3.0, std::ceil(1.0 / std::max(probe, 1e-3))));
     std::vector<double> best(cand.size(), 1e30);
-    double best_tiled = 1e30;
     for (int sweep = 0; sweep < 2 && e == hipSuccess; ++sweep) {
         for (size_t c = 0; c < cand.size() && e == hipSuccess; ++c) {
             double ms = 0;
             e = timed(cand[c], n, ms);
             if (e == hipSuccess) best[c] = std::min(best[c], ms);
-        }
-        if (try_tiled && e == hipSuccess) {
-            double ms = 0;
-            e = timed(fallback, n, ms, true);
-            if (e == hipSuccess) best_tiled = std::min(best_tiled, ms);
         }
     }
     if (e != hipSuccess) return bail(e);
@@ -344,35 +337,29 @@ int tune_march_rows(sfv_handle* h, std::string& why) {
     // from the current state (often a state at rest), where heights close in
     // time can order differently than in the developed flow.  The model's
     // height is the measured best for grids whose waves fill at least three
-    // quarters of the device's resident wave slots (3 per SIMD), so there it
+    // quarters of the device's resident wave slots (4 per SIMD), so there it
     // must lose by 10% to be replaced; for smaller grids, where the serial
     // path of a wave decides, by 3%.
     int cus = 256;
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, h->device) != hipSuccess || cus <= 0)
         cus = 256;
     const long waves = (long)((h->cfg.nx + MARCH_COLS - 1) / MARCH_COLS) * ((h->cfg.ny + fallback - 1) / fallback);
-    const double margin = waves >= 9L * cus ? 1.10 : 1.03;
+    const double margin = waves >= 12L * cus ? 1.10 : 1.03;
     size_t fast = 0;
     for (size_t c = 1; c < cand.size(); ++c)
         if (best[c] < best[fast]) fast = c;
     int pick = cand[fast];
-    double pick_ms = best[fast];
     for (size_t c = 0; c < cand.size(); ++c)
-        if (cand[c] == fallback && best[c] <= margin * best[fast]) { pick = fallback; pick_ms = best[c]; }
+        if (cand[c] == fallback && best[c] <= margin * best[fast]) pick = fallback;
     h->march_rows = pick;
     h->P.rows = pick;
-    // the tiled kernels replace the march ones only by the same margin
-    const bool tiled_wins = try_tiled && best_tiled * margin < pick_ms;
-    if (tiled_wins) h->fused = KV_TILED;
     if (const char* dbg = std::getenv("SFV_TUNE_REPORT"); dbg && dbg[0] == '1') {
         std::fprintf(stderr, "[sfv autotune] %dx%d %s:", h->cfg.nx, h->cfg.ny, f64 ? "f64" : "f32");
         for (size_t c = 0; c < cand.size(); ++c) std::fprintf(stderr, " %d:%.4f", cand[c], best[c]);
-        if (try_tiled) std::fprintf(stderr, " tiled:%.4f", best_tiled);
-        std::fprintf(stderr, " -> %s%d (ms per step, %d steps per timing)\n", tiled_wins ? "tiled, march " : "",
-                     pick, n);
+        std::fprintf(stderr, " -> %d (ms per step, %d steps per timing)\n", pick, n);
     }
     std::lock_guard<std::mutex> lk(g_tune_mu);
-    g_tuned.emplace(key, tiled_wins ? -pick : pick);
+    g_tuned.emplace(key, pick);
     return SFV_OK;
 }
 }  // namespace sfv
@@ -661,8 +648,8 @@ int sfv_time_kernel(sfv_handle* h, const char* which, int32_t n, double* ms_out)
     auto stage = [&](int which, auto* U0, auto* R, auto* Us) -> hipError_t {
         const KParams& P = h->P;
         if (h->fused == KV_TILED)
-            return which == 1 ? launch_stage1(h->stream, P, h->ctl, slot, U0, R, h->B)
-                              : launch_stage2(h->stream, P, h->ctl, slot, U0, R, Us, h->B);
+            return which == 1 ? launch_block(h->stream, P, h->ctl, slot, 1, U0, (decltype(U0))nullptr, R, h->B, 0, 1)
+                              : launch_block(h->stream, P, h->ctl, slot, 2, U0, R, Us, h->B);
         return which == 1 ? launch_march(h->stream, P, h->ctl, slot, 1, U0, (decltype(U0))nullptr, R, h->B, 0, 1)
                           : launch_march(h->stream, P, h->ctl, slot, 2, U0, R, Us, h->B);
     };

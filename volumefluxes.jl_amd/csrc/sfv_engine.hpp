@@ -131,7 +131,7 @@ private:
     std::vector<long long> tuned_sig_;       // member sizes the kept choice was made for
     int tuned_rows_ = 0;
     hipEvent_t ev_[2] = {nullptr, nullptr};
-    bool fast_ = false;           // the captured graph uses the specialised march kernels
+    int mode_ = 0;                // march mode of the captured graph: the lowest of the members
     int cus_ = 256;
     std::vector<int> rows_;                  // slot of each table row
     std::vector<sfv_handle*> slot_handle_;   // nullptr: free slot

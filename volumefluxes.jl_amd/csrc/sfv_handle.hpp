@@ -58,12 +58,13 @@ inline void build_kparams(const sfv_config& c, KParams& p, const double* d_rain,
     ghost_maps(c.bc, c.gc, p.nxT, p.src_lo_x, p.src_hi_x, p.flip_lo_x, p.flip_hi_x);
     ghost_maps(c.bc, c.gc, p.nyT, p.src_lo_y, p.src_hi_y, p.flip_lo_y, p.flip_hi_y);
     p.rows = march_rows;
-    // central_upwind_rng's parameter conditions; SFV_RANGED=0 turns it off
+    // the ranged forms' parameter conditions (swe_physics.hpp); SFV_RANGED=0 turns them off
     auto in = [](double v, double lo, double hi) { return v >= lo && v <= hi; };
     const char* rng_env = std::getenv("SFV_RANGED");
     p.ranged = !(rng_env && rng_env[0] == '0') && (p.rec != 1 || in(c.theta, 0x1p-10, 0x1p10)) &&
                in(c.rho, 0x1p-10, 0x1p10) && in(c.g, 0x1p-10, 0x1p10) && in(c.depth_cutoff, 0x1p-39, 0x1p10) &&
-               in(c.desingularizing_kappa, 0x1p-39, 0x1p10);
+               in(c.desingularizing_kappa, 0x1p-39, 0x1p10) && in(c.dx, 0x1p-60, 0x1p100) &&
+               in(c.dy, 0x1p-60, 0x1p100) && (c.friction == 0 || c.Cz == 0.0 || in(c.Cz, 0x1p-60, 0x1p10));
 }
 }  // namespace sfv
 

@@ -89,8 +89,8 @@ int advance(const sfv::KParams& P, hipStream_t st, const Scratch& scr, const dou
         const int slot = (int)(s & 1);
         S* in = buf[s & 1];
         S* out = buf[(s + 1) & 1];
-        NA_TRY(launch_march<S>(st, P, ctl, slot, 1, in, nullptr, RHS, B, 0, 1));
-        NA_TRY(launch_march<S>(st, P, ctl, slot, 2, in, RHS, out, B, 1, 0));
+        NA_TRY(launch_stage<S>(st, P, ctl, slot, 1, in, nullptr, RHS, B, 0, 1));
+        NA_TRY(launch_stage<S>(st, P, ctl, slot, 2, in, RHS, out, B, 1, 0));
     }
     S* last = buf[nsteps & 1];
     NA_TRY(launch_bc<S>(st, P, ctl, (int)(nsteps & 1), last, BC_STANDALONE));   // the march path leaves ghosts

@@ -241,7 +241,7 @@ __device__ inline void set_rates(const KParams& P, StepSlot& s, double t) {
 
 // Close the step of `slot` with its dt: t += dt (simulator.jl:205), count
 // it, and arm the next slot (active unless the run ends here).  One thread.
-template <class S, bool NO_INFIL = false>
+template <class S, bool NO_HORTON = false>
 __device__ inline void close_step(const KParams& P, StepCtl* c, int slot) {
     const S dt = (S)c->dt;
     const S t = (S)((S)c->slot[slot].t + dt);
@@ -253,10 +253,10 @@ __device__ inline void close_step(const KParams& P, StepCtl* c, int slot) {
     StepSlot& nx = c->slot[1 - slot];
     clear_wsmax(nx);
     nx.active = act ? 1 : 0;
-    if (NO_INFIL) {             // the caller knows the run has no infiltration
+    if (NO_HORTON) {            // the caller knows the run has no Horton infiltration
         nx.t = (double)t;
         nx.rain_now = compute_rain(P, (double)t);
-        nx.infil_tfac = 0.0;
+        nx.infil_tfac = P.infil_kind == 1 ? P.infil_rate : 0.0;
     } else {
         set_rates(P, nx, (double)t);
     }
@@ -266,9 +266,9 @@ __device__ inline void close_step(const KParams& P, StepCtl* c, int slot) {
 // The same, out of line, for the persistent batch kernels (their KParams
 // live in the member table): inlined into the tile loop, the rate code
 // costs the whole loop registers.
-template <class S, bool NO_INFIL = false>
+template <class S, bool NO_HORTON = false>
 __device__ __attribute__((noinline)) void close_step_call(const KParams& P, StepCtl* c, int slot) {
-    close_step<S, NO_INFIL>(P, c, slot);
+    close_step<S, NO_HORTON>(P, c, slot);
 }
 
 // timestep_computer (simulator.jl:147-150) with the max_dt rule of

@@ -19,16 +19,6 @@ __global__ void k_prepare(KParams P, StepCtl* ctl, int slot, double t, double en
                           int has_max_timestep, double max_timestep, long long max_steps, int until_endtime,
                           int precision);
 
-// ---- fused stage kernels (swe_kernels_fused.hip)
-// Tile of interior cells per block and threads per block.
-constexpr int FT_X = 64;
-constexpr int FT_Y = 8;
-constexpr int F_THREADS = 256;
-template <class S>
-__global__ void k_stage1(KParams P, StepCtl* ctl, int slot, const S* U0, S* RHS, const double* B);
-template <class S>
-__global__ void k_stage2(KParams P, StepCtl* ctl, int slot, const S* U0, const S* RHS1, S* U2, const double* B);
-
 // ---- host launchers (one per kernel, defined beside it); each returns the
 // launch status.  BC modes: 0 inside a step, 1 last stage of a step (closes
 // the step), 2 standalone (set_current_state!, no step-control check).
@@ -47,15 +37,17 @@ hipError_t launch_prepare(hipStream_t st, const KParams& P, StepCtl* ctl, int sl
                           int until_endtime, int precision);
 // Batched kernels over a device member table (BatchMember[hdr->members]).
 // Stage kernels are persistent: `blocks` workgroups walk the batch's tiles.
-// fast: every member satisfies march_fast (the specialised kernels).
+// mode: the lowest march_mode of the members.
 template <class S>
 hipError_t launch_march_batch(hipStream_t st, int stage, const BatchMember* mem, const BatchHeader* hdr, int lp,
-                              int blocks, bool fast);
-// The configurations the specialised march kernels cover.
-bool march_fast(const KParams& P);
+                              int blocks, int mode);
+// The specialised kernels a configuration may use (MODE_* of swe_rows.hpp; a
+// lower mode always serves too): 0 to MAX_MODE.
+constexpr int MAX_MODE = 2;
+int march_mode(const KParams& P);
 hipError_t launch_prepare_batch(hipStream_t st, const BatchMember* mem, const BatchHeader* hdr, int members);
 // Resident workgroups per CU of the batched stage kernel (occupancy).
-int march_batch_blocks_per_cu(int precision, int stage);
+int march_batch_blocks_per_cu(int precision, int stage, int mode);
 int march_rows_per_wave(const KParams& P, int stage, int precision);   // precision: 0 f64, 1 f32
 constexpr int MARCH_COLS = 60;   // output columns per wave strip
 #ifndef SFV_MARCH_WAVES
@@ -82,9 +74,6 @@ hipError_t launch_copy(hipStream_t st, const void* src, void* dst, size_t bytes)
 // state -> packed.  es = element size (4 or 8).
 hipError_t launch_interior_copy(hipStream_t st, const KParams& P, const void* packed, void* state, size_t es,
                                 int to_state);
-template <class S>
-hipError_t launch_stage1(hipStream_t st, const KParams& P, StepCtl* ctl, int slot, const S* U0, S* RHS,
-                         const double* B);
 // stage = 1: U0 -> OUT = RHS1 (+ speeds); stage = 2: U0, RHS1 -> OUT = U2
 // (interior and domain corners).  Stage 2 reads halo ghost cells through the
 // boundary-condition maps; stage 1 too with remap_halo = 1 (only when the
@@ -94,8 +83,20 @@ hipError_t launch_stage1(hipStream_t st, const KParams& P, StepCtl* ctl, int slo
 template <class S>
 hipError_t launch_march(hipStream_t st, const KParams& P, StepCtl* ctl, int slot, int stage, const S* U0,
                         const S* RHS1, S* OUT, const double* B, int close = 0, int remap_halo = 0);
+// The same stages with one workgroup per strip segment (swe_kernels_block.hip).
 template <class S>
-hipError_t launch_stage2(hipStream_t st, const KParams& P, StepCtl* ctl, int slot, const S* U0, const S* RHS1, S* U2,
-                         const double* B, int close = 0);
+hipError_t launch_block(hipStream_t st, const KParams& P, StepCtl* ctl, int slot, int stage, const S* U0,
+                        const S* RHS1, S* OUT, const double* B, int close = 0, int remap_halo = 0);
+constexpr int BLOCK_MAX_ROWS = 28;   // output rows per workgroup
+// Do these kernels suit the grid (one workgroup per CU, at most
+// BLOCK_MAX_ROWS rows each), without a measurement?
+bool block_suits(const KParams& P);
+// Either kernel: the workgroup ones where they suit the grid.
+template <class S>
+hipError_t launch_stage(hipStream_t st, const KParams& P, StepCtl* ctl, int slot, int stage, const S* U0,
+                        const S* RHS1, S* OUT, const double* B, int close = 0, int remap_halo = 0) {
+    return block_suits(P) ? launch_block<S>(st, P, ctl, slot, stage, U0, RHS1, OUT, B, close, remap_halo)
+                          : launch_march<S>(st, P, ctl, slot, stage, U0, RHS1, OUT, B, close, remap_halo);
+}
 
 }  // namespace sfv

@@ -188,151 +188,6 @@ __device__ __forceinline__ double friction_scalar(int law, double Cz, double kap
 
 
 // ---------------------------------------------------------------------------
-// Branch-free forms for the fused march kernels.  Each equals the function
-// above for every input; the reference's branches become selects so that a
-// wave's face work is straight-line code the scheduler can interleave.
-
-// minmod slopes + SWE slope fix + face values, with the fix as a select.
-template <class S>
-__device__ __forceinline__ void reconstruct_cell_nb(const S l[3], const S c[3], const S r[3], double theta,
-                                                    double Bl, double Br, S L[3], S R[3]) {
-    const bool regular = __builtin_isfinite(theta) && theta != 0.0;
-    double slope[3];
-#pragma unroll
-    for (int v = 0; v < 3; ++v) {
-        const S fwd = r[v] - c[v];
-        const S bwd = c[v] - l[v];
-        const double central = (fwd + bwd) / 2.0;
-        slope[v] = minmod(theta * fwd, central, theta * bwd, regular);
-    }
-    const S w = c[0];
-    const bool fix_l = w - 0.5 * slope[0] < Bl;
-    const bool fix_r = w + 0.5 * slope[0] < Br;
-    const double sl = 2.0 * (w - Bl), sr = 2.0 * (Br - w);
-    slope[0] = fix_l ? sl : (fix_r ? sr : slope[0]);
-#pragma unroll
-    for (int v = 0; v < 3; ++v) {
-        L[v] = (S)(c[v] - 0.5 * slope[v]);
-        R[v] = (S)(c[v] + 0.5 * slope[v]);
-    }
-    L[0] = (S)(L[0] - Bl);
-    R[0] = (S)(R[0] - Br);
-}
-
-// Desingularised depths of N face sides: the |h| >= κ case (h* = h) inline,
-// the rare |h| < κ case for all of them in one branch.
-template <class S, int N>
-__device__ __forceinline__ void desingularize_n(const S* const h[N], double kappa, double hs[N]) {
-    bool slow = false;
-#pragma unroll
-    for (int k = 0; k < N; ++k) {
-        hs[k] = (double)*h[k];
-        slow |= (double)__builtin_fabs(*h[k]) < kappa;
-    }
-    if (slow) {
-#pragma unroll
-        for (int k = 0; k < N; ++k)
-            if ((double)__builtin_fabs(*h[k]) < kappa) hs[k] = desingularize(*h[k], kappa);
-    }
-}
-
-// centralupwind.jl:48-77 for direction D with the desingularised depths of
-// both sides given: both sides are evaluated and dry sides (h <= cutoff)
-// select zero flux and eigenvalues, exactly as the reference's zero(...)
-// initialisers; the degenerate |a+ - a-| < κ and both-dry cases select the
-// reference's early returns.
-template <int D, class S>
-__device__ __forceinline__ double central_upwind_nb(const S m[3], const S q[3], double hsm, double hsq,
-                                                    const PhysParams& p, double F[3]) {
-    const bool wm = m[0] > p.cutoff, wq = q[0] > p.cutoff;
-    double fm[3], fp[3], em[2], ep[2];
-    {
-        const double u = m[1] / hsm, v = m[2] / hsm;
-        const S h2 = m[0] * m[0];
-        const double c = sqrt(p.g * m[0]);
-        const double a = D == 0 ? u : v;
-        const double f0 = p.rho * m[0] * a;
-        const double f1 = D == 0 ? p.rho * m[0] * u * u + 0.5 * p.rho * p.g * h2 : p.rho * m[0] * u * v;
-        const double f2 = D == 0 ? p.rho * m[0] * u * v : p.rho * m[0] * v * v + 0.5 * p.rho * p.g * h2;
-        fm[0] = wm ? f0 : 0.0;
-        fm[1] = wm ? f1 : 0.0;
-        fm[2] = wm ? f2 : 0.0;
-        em[0] = wm ? a + c : 0.0;
-        em[1] = wm ? a - c : 0.0;
-    }
-    {
-        const double u = q[1] / hsq, v = q[2] / hsq;
-        const S h2 = q[0] * q[0];
-        const double c = sqrt(p.g * q[0]);
-        const double a = D == 0 ? u : v;
-        const double f0 = p.rho * q[0] * a;
-        const double f1 = D == 0 ? p.rho * q[0] * u * u + 0.5 * p.rho * p.g * h2 : p.rho * q[0] * u * v;
-        const double f2 = D == 0 ? p.rho * q[0] * u * v : p.rho * q[0] * v * v + 0.5 * p.rho * p.g * h2;
-        fp[0] = wq ? f0 : 0.0;
-        fp[1] = wq ? f1 : 0.0;
-        fp[2] = wq ? f2 : 0.0;
-        ep[0] = wq ? a + c : 0.0;
-        ep[1] = wq ? a - c : 0.0;
-    }
-    const double aplus = nz_max(nz_max(ep[0], em[0]), 0.0);
-    const double aminus = nz_min(nz_min(ep[1], em[1]), 0.0);
-    const double da = aplus - aminus;
-    const bool degenerate = __builtin_fabs(da) < p.kappa;
-    const double pm = (aplus * aminus) / da;
-#pragma unroll
-    for (int v = 0; v < 3; ++v) {
-        const S diff = q[v] - m[v];
-        const double f = (aplus * fm[v] - aminus * fp[v]) / da + pm * diff;
-        F[v] = degenerate ? 0.0 : f;
-    }
-    const bool both_dry = m[0] < p.cutoff && q[0] < p.cutoff;
-    const double sp = nz_max(__builtin_fabs(aplus), __builtin_fabs(aminus));
-    return (degenerate || both_dry) ? 0.0 : sp;
-}
-
-// centralupwind.jl:48-77 for direction D when both sides are wet and
-// |h| >= κ on both (so h* = h, equation.jl:56): the reference's branches are
-// all decided, and what is left is straight-line code — the two sides and the
-// four quotients by a+ - a- are independent chains.  Only the degenerate
-// |a+ - a-| < κ return remains, as a select.
-template <int D, class S>
-__device__ __forceinline__ double central_upwind_wet(const S m[3], const S q[3], const PhysParams& p, double F[3]) {
-    const double um = m[1] / (double)m[0], vm = m[2] / (double)m[0];
-    const double uq = q[1] / (double)q[0], vq = q[2] / (double)q[0];
-    const S hm2 = m[0] * m[0], hq2 = q[0] * q[0];
-    const double cm = sqrt(p.g * m[0]), cq = sqrt(p.g * q[0]);
-    const double am = D == 0 ? um : vm, aq = D == 0 ? uq : vq;
-    const double rgh = 0.5 * p.rho * p.g;
-    double fm[3], fp[3];
-    fm[0] = p.rho * m[0] * am;
-    fp[0] = p.rho * q[0] * aq;
-    if (D == 0) {
-        fm[1] = p.rho * m[0] * um * um + rgh * hm2;
-        fm[2] = p.rho * m[0] * um * vm;
-        fp[1] = p.rho * q[0] * uq * uq + rgh * hq2;
-        fp[2] = p.rho * q[0] * uq * vq;
-    } else {
-        fm[1] = p.rho * m[0] * um * vm;
-        fm[2] = p.rho * m[0] * vm * vm + rgh * hm2;
-        fp[1] = p.rho * q[0] * uq * vq;
-        fp[2] = p.rho * q[0] * vq * vq + rgh * hq2;
-    }
-    const double aplus = nz_max(nz_max(aq + cq, am + cm), 0.0);
-    const double aminus = nz_min(nz_min(aq - cq, am - cm), 0.0);
-    const double da = aplus - aminus;
-    const bool degenerate = __builtin_fabs(da) < p.kappa;
-    const double pm = (aplus * aminus) / da;
-#pragma unroll
-    for (int v = 0; v < 3; ++v) {
-        const S diff = q[v] - m[v];
-        const double f = (aplus * fm[v] - aminus * fp[v]) / da + pm * diff;
-        F[v] = degenerate ? 0.0 : f;
-    }
-    const double sp = nz_max(__builtin_fabs(aplus), __builtin_fabs(aminus));
-    return degenerate ? 0.0 : sp;
-}
-
-// ---------------------------------------------------------------------------
 // Face evaluation on operands in a proven range.
 //
 // The compiler's correctly rounded FP64 quotient x/d on gfx950 is
@@ -355,21 +210,25 @@ __device__ __forceinline__ double central_upwind_wet(const S m[3], const S q[3],
 // in [2^-767, DBL_MAX] both are no-ops, and sqrt_rng is the same steps
 // without them: 10 instructions against 17.
 //
-// central_upwind_rng is central_upwind with these forms.  It is used only by
-// a wave whose stage inputs (w, hu, hv of every cell the face stencils read)
-// and bottom corners all lie in {0} U [2^-100, 2^40] in magnitude (checked as
-// the rows arrive, in_band5, whose set is the subset {0} U [2^-100, 2^40)),
-// with θ (linear reconstruction), ρ and g in
-// [2^-10, 2^10] and depth_cutoff and κ in [2^-39, 2^10] (KParams::ranged).
-// Then (exact differences of such values are multiples of 2^-152, rounded
-// products keep their exponent sums, and cancellation in u +- c leaves at
-// least an ulp of c >= sqrt(g*cutoff)):
-//   face values:   0 or [2^-215, 2^51]; wet depths h > cutoff >= 2^-39
-//   velocity quotient hu/h*:  x in {0} U [2^-215, 2^51], d = h* in [2^-40, 2^51]
+// The *_rng functions below are the functions above with these forms.  They
+// are used only by waves whose inputs lie in band: every stage input (w, hu,
+// hv of every cell the face stencils read) and bottom corner is 0 or of
+// magnitude in [2^-120, 2^40) (checked as the rows arrive, in_band), with θ
+// (linear reconstruction), ρ and g in [2^-10, 2^10], depth_cutoff and κ in
+// [2^-39, 2^10] and the spacings in [2^-60, 2^100] (KParams::ranged).  Then
+// (exact differences of such values are multiples of 2^-172, rounded products
+// keep their exponent sums, and cancellation in u +- c leaves at least an ulp
+// of c >= sqrt(g*cutoff)):
+//   face values:   0 or [2^-235, 2^51]; wet depths h > cutoff >= 2^-39
+//   velocity quotient hu/h*:  x in {0} U [2^-235, 2^51], d = h* in [2^-40, 2^51]
 //   c = sqrt(g h):  g h in [2^-49, 2^61]
 //   a+, a-:         0 or [2^-78, 2^92];  da = a+ - a- in [κ, 2^93] unless degenerate
-//   flux quotients: numerators 0 or [2^-712, 2^336], (a+ a-) in [2^-156, 2^184]
-// which is inside the range above.  A degenerate face (|da| < κ) discards
+//   flux quotients: numerators 0 or [2^-752, 2^336], (a+ a-) in [2^-156, 2^184]
+//   h^2/(2κ) below κ: x = 0 or [2^-470, 2^20], d in [2^-38, 2^11]
+//   bottom slopes:  x = 0 or [2^-173, 2^41], d in [2^-60, 2^100]
+// which is inside the range above, or clear of every scaling condition where
+// d reaches beyond it (no operand is subnormal, |x| > 2^-969, the exponents
+// of x and d are less than 768 apart).  A degenerate face (|da| < κ) discards
 // its quotients, as the reference's early return does.
 struct Recip {
     double d, r;
@@ -399,62 +258,67 @@ __device__ __forceinline__ double sqrt_rng(double x) {
     d = __builtin_fma(-g, g, x);
     return __builtin_fma(d, h, g);
 }
-// |v| is 0 or in [2^-100, 2^40] (false for NaN, Inf and subnormals).
-__device__ __forceinline__ bool in_band(double v) {
-    const double a = __builtin_fabs(v);
-    return a == 0.0 || (a >= 0x1p-100 && a <= 0x1p40);
-}
-// Every value 0 or in [2^-100, 2^40) in magnitude (a subset of in_band's
-// set), tested through exponents: the hardware's frexp exponent e (v = m 2^e
-// with |m| in [0.5, 1); 0 for 0, the true exponent for subnormals, 0 for Inf
-// and NaN) lies in [-99, 40] exactly for 0 and the magnitudes in
-// [2^-100, 2^40), and for Inf and NaN, which make the sum non-finite.  The
-// exponents combine with integer min/max, so the test costs one lane mask
-// instead of three per value.
-__device__ __forceinline__ bool in_band5(double a, double b, double c, double d, double e) {
-    const int ea = __builtin_amdgcn_frexp_exp(a), eb = __builtin_amdgcn_frexp_exp(b),
-              ec = __builtin_amdgcn_frexp_exp(c), ed = __builtin_amdgcn_frexp_exp(d),
-              ee = __builtin_amdgcn_frexp_exp(e);
-    const int lo = min(min(min(ea, eb), min(ec, ed)), ee), hi = max(max(max(ea, eb), max(ec, ed)), ee);
-    const double s = ((a + b) + (c + d)) + e;      // finite: no value is Inf or NaN (|v| < 2^40 cannot overflow it)
-    return (unsigned)(lo + 99) <= 139u && (unsigned)(hi + 99) <= 139u && __builtin_isfinite(s);
+// Every value is 0 or of magnitude at least 2^-120, and their magnitudes add
+// up to less than 2^40 (false for NaN and Inf, whose sums are not less).  The
+// lower bound is tested through the hardware's frexp exponent e (v = m 2^e
+// with |m| in [0.5, 1); 0 for 0, the true exponent for subnormals): integer
+// minima combine it over the values, and one addition per value covers the
+// rest.
+__device__ __forceinline__ bool in_band(double a, double b, double c, double d) {
+    const int lo = min(min(__builtin_amdgcn_frexp_exp(a), __builtin_amdgcn_frexp_exp(b)),
+                       min(__builtin_amdgcn_frexp_exp(c), __builtin_amdgcn_frexp_exp(d)));
+    const double s = (__builtin_fabs(a) + __builtin_fabs(b)) + (__builtin_fabs(c) + __builtin_fabs(d));
+    return lo >= -119 && s < 0x1p40;
 }
 
-// swe_2D.jl:43-81 with the ranged quotients and square root (h > cutoff).
-template <class S>
-__device__ __forceinline__ void phys_flux_rng(int d, S h, S hu, S hv, const PhysParams& p, double f[3],
+// What the ranged forms need of a run's constants, the same on every lane:
+// refined reciprocals and products formed once per wave.
+struct RngK {
+    Recip k2, dx, dy;          // 2κ and the spacings
+    double half_kappa, hrg;    // κ/2, (0.5 ρ) g
+    double theta2;             // 2 θ
+    double bx, by;             // -g (1/Δ) / 2 (power-of-two spacings)
+};
+
+// equation.jl:56 as desingularize.
+template <class H>
+__device__ __forceinline__ double desingularize_rng(H h, double kappa, const RngK& K) {
+    const double ah = (double)__builtin_fabs(h);
+    if (!(ah < kappa)) return (double)h;
+    const H h2 = h * h;
+    return __builtin_copysign(__builtin_fmax(ah, __builtin_fmin(div_rng(h2, K.k2) + K.half_kappa, kappa)), (double)h);
+}
+
+// swe_2D.jl:43-81 for direction D with the ranged quotients and square root
+// (h > cutoff).  UNIT_RHO: ρ is 1.
+template <int D, bool UNIT_RHO, class S>
+__device__ __forceinline__ void phys_flux_rng(S h, S hu, S hv, const PhysParams& p, const RngK& K, double f[3],
                                               double e[2]) {
-    const double hs = desingularize(h, p.kappa);
-    const Recip R = recip_rng(hs);
+    const Recip R = recip_rng(desingularize_rng(h, p.kappa, K));
     const double u = div_rng(hu, R);
     const double v = div_rng(hv, R);
     const S h2 = h * h;
     const double c = sqrt_rng(p.g * h);
-    if (d == 0) {
-        f[0] = p.rho * h * u;
-        f[1] = p.rho * h * u * u + 0.5 * p.rho * p.g * h2;
-        f[2] = p.rho * h * u * v;
-        e[0] = u + c;
-        e[1] = u - c;
-    } else {
-        f[0] = p.rho * h * v;
-        f[1] = p.rho * h * u * v;
-        f[2] = p.rho * h * v * v + 0.5 * p.rho * p.g * h2;
-        e[0] = v + c;
-        e[1] = v - c;
-    }
+    const double rh = UNIT_RHO ? (double)h : p.rho * h;
+    const double ph = K.hrg * h2;
+    f[0] = rh * (D == 0 ? u : v);
+    f[1] = D == 0 ? rh * u * u + ph : rh * u * v;
+    f[2] = D == 0 ? rh * u * v : rh * v * v + ph;
+    e[0] = (D == 0 ? u : v) + c;
+    e[1] = (D == 0 ? u : v) - c;
 }
 
-// centralupwind.jl:48-77 as central_upwind, with the ranged forms.
-template <class S>
-__device__ __forceinline__ double central_upwind_rng(int d, const S m[3], const S q[3], const PhysParams& p,
+// centralupwind.jl:48-77 as central_upwind.  No NaN and no -0.0 reaches
+// max/min here (finite inputs; see nz_max), so they are the hardware's.
+template <int D, bool UNIT_RHO, class S>
+__device__ __forceinline__ double central_upwind_rng(const S m[3], const S q[3], const PhysParams& p, const RngK& K,
                                                      double F[3]) {
     double fm[3] = {0.0, 0.0, 0.0}, em[2] = {0.0, 0.0};
     double fp[3] = {0.0, 0.0, 0.0}, ep[2] = {0.0, 0.0};
-    if (m[0] > p.cutoff) phys_flux_rng(d, m[0], m[1], m[2], p, fm, em);
-    if (q[0] > p.cutoff) phys_flux_rng(d, q[0], q[1], q[2], p, fp, ep);
-    const double aplus = nz_max(nz_max(ep[0], em[0]), 0.0);
-    const double aminus = nz_min(nz_min(ep[1], em[1]), 0.0);
+    if (m[0] > p.cutoff) phys_flux_rng<D, UNIT_RHO>(m[0], m[1], m[2], p, K, fm, em);
+    if (q[0] > p.cutoff) phys_flux_rng<D, UNIT_RHO>(q[0], q[1], q[2], p, K, fp, ep);
+    const double aplus = __builtin_fmax(__builtin_fmax(ep[0], em[0]), 0.0);
+    const double aminus = __builtin_fmin(__builtin_fmin(ep[1], em[1]), 0.0);
     const double da = aplus - aminus;
     if (__builtin_fabs(da) < p.kappa) {
         F[0] = F[1] = F[2] = 0.0;
@@ -468,22 +332,63 @@ __device__ __forceinline__ double central_upwind_rng(int d, const S m[3], const 
         F[v] = div_rng(aplus * fm[v] - aminus * fp[v], R) + pm * diff;
     }
     if (m[0] < p.cutoff && q[0] < p.cutoff) return 0.0;
-    return nz_max(__builtin_fabs(aplus), __builtin_fabs(aminus));
+    return __builtin_fmax(aplus, -aminus);
 }
 
-// Both sides of a face wet with |h| >= κ: central_upwind_wet applies.
+// minmod_slope + the SWE dry-face slope fix + face values
+// (linearreconstruction.jl:37-43, 73-100) as reconstruct_cell: no NaN, and
+// scaling by a power of two is exact.  Slopes are kept doubled (s2 = 2
+// slope, theta2 = 2 θ), so (fwd + bwd)/2 needs no product, and c -+ slope/2 is
+// one fma, its product exact.  With lo = max(min(a, e), 0) and hi =
+// min(max(a, e), 0), minmod(a, b, e) is b clamped to [hi, lo]: both positive
+// gives hi = 0 and min(b, lo), both negative lo = 0 and max(b, hi), else lo =
+// hi = 0.  The added +0.0 keeps a and e from being -0.0, so a zero slope is
+// +0.0 as the reference's is.
 template <class S>
-__device__ __forceinline__ bool face_is_wet(const S m[3], const S q[3], const PhysParams& p) {
-    return m[0] > p.cutoff && q[0] > p.cutoff && (double)__builtin_fabs(m[0]) >= p.kappa &&
-           (double)__builtin_fabs(q[0]) >= p.kappa;
+__device__ __forceinline__ void reconstruct_cell_rng(const S l[3], const S c[3], const S r[3], double theta2,
+                                                     double Bl, double Br, S L[3], S R[3]) {
+    double s2[3];
+#pragma unroll
+    for (int v = 0; v < 3; ++v) {
+        const S fwd = r[v] - c[v];
+        const S bwd = c[v] - l[v];
+        const S sum = fwd + bwd;
+        const double a = __builtin_fma(theta2, (double)fwd, 0.0), e = __builtin_fma(theta2, (double)bwd, 0.0);
+        const double lo = __builtin_fmax(__builtin_fmin(a, e), 0.0), hi = __builtin_fmin(__builtin_fmax(a, e), 0.0);
+        s2[v] = __builtin_fmin(__builtin_fmax((double)sum, hi), lo);
+    }
+    // w's faces before the bottoms are taken off; the dry-face fix makes the
+    // half slope w - Bl or Br - w
+    const double w = (double)c[0];
+    double wl = __builtin_fma(-0.25, s2[0], w), wr = __builtin_fma(0.25, s2[0], w);
+    if (wl < Bl || wr < Br) {
+        const double half = wl < Bl ? w - Bl : Br - w;
+        wl = w - half;
+        wr = w + half;
+    }
+    L[0] = (S)((S)wl - Bl);
+    R[0] = (S)((S)wr - Br);
+#pragma unroll
+    for (int v = 1; v < 3; ++v) {
+        L[v] = (S)__builtin_fma(-0.25, s2[v], (double)c[v]);
+        R[v] = (S)__builtin_fma(0.25, s2[v], (double)c[v]);
+    }
 }
 
-// One face, with the straight-line evaluation when the whole wave's faces are
-// wet (a wave-uniform branch) and the general evaluation otherwise.
-template <int D, class S>
-__device__ __forceinline__ double central_upwind_auto(const S m[3], const S q[3], const PhysParams& p, double F[3]) {
-    if (__all(face_is_wet(m, q, p))) return central_upwind_wet<D>(m, q, p, F);
-    return central_upwind(D, m, q, p, F);
+// friction.jl:40-43, 62-78: the bh2021 friction scalar from a substep input in
+// band, with Cz 0 or in [2^-60, 2^10].  hs in [2^-40, 2^41], so u, v are 0 or in
+// [2^-161, 2^80], u^2 + v^2 0 or in [2^-322, 2^161], the denominator in
+// [2^-80, 2^82].  Adding 2^-700 leaves a nonzero u^2 + v^2 as it is and turns 0
+// into a speed of 2^-350: the caller's 1 - dt*fs is then 1, as it is for 0
+// (dt <= 2^100).
+template <class S>
+__device__ __forceinline__ double friction_scalar_rng(double Cz, double kappa, const RngK& K, S w, S hu, S hv,
+                                                      double Bm) {
+    const double hs = desingularize_rng(w - Bm, kappa, K);
+    const Recip R = recip_rng(hs);
+    const double u = div_rng(hu, R), v = div_rng(hv, R);
+    const double speed = sqrt_rng((u * u + v * v) + 0x1p-700);
+    return div_rng(-Cz * speed, recip_rng(hs * hs));
 }
 
 }  // namespace sfv

@@ -57,6 +57,11 @@ inline void build_kparams(const sfv_config& c, KParams& p, const double* d_rain,
     p.bc = c.bc;
     ghost_maps(c.bc, c.gc, p.nxT, p.src_lo_x, p.src_hi_x, p.flip_lo_x, p.flip_hi_x);
     ghost_maps(c.bc, c.gc, p.nyT, p.src_lo_y, p.src_hi_y, p.flip_lo_y, p.flip_hi_y);
+    auto ghost = [](int s, int gc, int N) { return s < gc || s >= N - gc; };
+    for (int g = 0; g < c.gc; ++g)
+        if (ghost(p.src_lo_x[g], c.gc, p.nxT) || ghost(p.src_hi_x[g], c.gc, p.nxT) ||
+            ghost(p.src_lo_y[g], c.gc, p.nyT) || ghost(p.src_hi_y[g], c.gc, p.nyT))
+            p.ghost_self = 1;
     p.rows = march_rows;
     // the ranged forms' parameter conditions (swe_physics.hpp); SFV_RANGED=0 turns them off
     auto in = [](double v, double lo, double hi) { return v >= lo && v <= hi; };
@@ -68,10 +73,11 @@ inline void build_kparams(const sfv_config& c, KParams& p, const double* d_rain,
 }
 }  // namespace sfv
 
-// Kernel variants of an RK2 step (all give identical results).
-// Kernel variants of a step.  KV_HYBRID: every right-hand side from the march
-// stage-1 kernel, the updates and boundary conditions from the per-pass
-// kernels (ForwardEuler and NeumannBC, whose steps the fused stage 2 cannot do).
+// Kernel variants of a step (all give identical results).  KV_MARCH: the
+// wave-march stage kernels; KV_TILED: the workgroup stage kernels; KV_HYBRID:
+// right-hand sides from the stage-1 kernels and updates from the per-pass
+// kernels, or, for ForwardEuler, both in one (ForwardEuler and NeumannBC,
+// whose steps the fused stage 2 cannot do).
 enum { KV_PER_PASS = 0, KV_TILED = 1, KV_MARCH = 2, KV_HYBRID = 3 };
 
 struct sfv_handle {
@@ -229,12 +235,29 @@ struct sfv_handle {
         return true;
     }
 
+    // The same, or a high-side ghost that is its own source (NeumannBC): the
+    // boundary condition leaves it as the update wrote it, so the maps can be
+    // read after any update without a boundary-condition pass.
+    bool ghosts_settled() const {
+        if (P.gc < 2) return false;
+        auto ok = [&](int s, const int* hi, const int* flip, int N) {
+            if (s >= P.gc && s < N - P.gc) return true;
+            return s >= N - P.gc && hi[s - (N - P.gc)] == s && !flip[s - (N - P.gc)];
+        };
+        for (int g = 0; g < P.gc; ++g) {
+            for (int s : {P.src_lo_x[g], P.src_hi_x[g]})
+                if (!ok(s, P.src_hi_x, P.flip_hi_x, P.nxT)) return false;
+            for (int s : {P.src_lo_y[g], P.src_hi_y[g]})
+                if (!ok(s, P.src_hi_y, P.flip_hi_y, P.nyT)) return false;
+        }
+        return true;
+    }
+
     // Does a step leave the output's ghost cells unwritten (they are then
-    // filled where the state leaves the stepping loop)?  The march and tiled
-    // RK2 paths and the two-launch ForwardEuler path do.
+    // filled where the state leaves the stepping loop)?  The stage kernels'
+    // RK2 paths and the hybrid paths that read ghosts through the maps do.
     bool leaves_ghosts() const {
-        return fused == KV_MARCH || fused == KV_TILED ||
-               (fused == KV_HYBRID && cfg.stepper == SFV_FORWARD_EULER && ghost_sources_interior());
+        return fused == KV_MARCH || fused == KV_TILED || (fused == KV_HYBRID && ghosts_settled());
     }
 
     // The fused stage kernels rebuild stage-1 ghost cells from their

@@ -921,11 +921,11 @@ int forward_step(sfv_handle* h, hipStream_t st, double t, const double* U0, doub
     const KParams& P = h->P;
     ATRY(launch_prepare(st, P, h->ctl, 0, t, NAN, 0, 0, 0.0, 1, 0, SFV_F64));
     ATRY(launch_stage<double>(st, P, h->ctl, 0, 1, U0, nullptr, R1, h->B));
-    ATRY(launch_finish<double>(st, P, h->ctl, 0, 1, U0, U0, R1, U1, h->B, 1, 0, R1));
+    ATRY(launch_finish<double>(st, P, h->ctl, 0, 1, U0, U0, R1, U1, h->B, 1, -1, R1));
     ATRY(hipMemcpyAsync(ctl_out, h->ctl, sizeof(StepCtl), hipMemcpyDeviceToDevice, st));
     ATRY(launch_bc<double>(st, P, h->ctl, 0, U1, BC_IN_STEP));
     ATRY(launch_stage<double>(st, P, h->ctl, 0, 1, U1, nullptr, R2, h->B));
-    ATRY(launch_finish<double>(st, P, h->ctl, 0, 2, U0, U1, R2, U2, h->B, 1, 0, R2));
+    ATRY(launch_finish<double>(st, P, h->ctl, 0, 2, U0, U1, R2, U2, h->B, 1, -1, R2));
     ATRY(launch_bc<double>(st, P, h->ctl, 0, U2, BC_LAST_STAGE));
     return SFV_OK;
 }

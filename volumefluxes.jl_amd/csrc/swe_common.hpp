@@ -46,10 +46,16 @@ struct KParams {
     // maps (NeumannBC's high side, grids narrower than gc) are exact.
     int src_lo_x[MAX_GC], src_hi_x[MAX_GC], src_lo_y[MAX_GC], src_hi_y[MAX_GC];
     int flip_lo_x[MAX_GC], flip_hi_x[MAX_GC], flip_lo_y[MAX_GC], flip_hi_y[MAX_GC];
+    // 1: some ghost's source is a ghost (one that is its own source, as on
+    // NeumannBC's high side): its value lives on in the state's memory
+    int ghost_self;
 };
 
-// Per-step flags live in two slots indexed by step parity, so the kernel that
-// finishes step n can arm step n+1 while no kernel of step n reads that slot.
+// Per-step flags live in slots the steps take in turn, so the kernel that
+// finishes step n can arm step n+1 while no kernel of step n reads that slot:
+// two slots by step parity, or three where one kernel finishes step n and
+// already raises the speeds of step n+1 (the ForwardEuler stage, STAGE 3): it
+// reads slot n mod 3, raises slot n+1 mod 3 and clears slot n+2 mod 3.
 // One step's control: the kernels of a step read only their own slot (and
 // the run-wide fields of StepCtl), and the step's last kernel arms the other
 // slot for the next step, so the step can close while its kernels still run.
@@ -57,17 +63,19 @@ struct KParams {
 // WS_LINES partial maxima, each on a cache line of its own; their maximum is
 // the step's.
 constexpr int WS_LINES = 8;
-struct StepSlot {
-    int32_t active;
-    int32_t pad;
+struct StepRates {
     double t;             // the step's start time (realtype value)
     double rain_now;      // compute_rain(rain, t)
     double infil_tfac;    // fc + (f0 - fc)*exp(-k t) for Horton, the rate for constant
+};
+struct StepSlot : StepRates {
+    int32_t active;
+    int32_t pad;
     alignas(128) unsigned long long ws[WS_LINES][16];   // [line][0]: x, [line][1]: y
 };
 
 struct StepCtl {
-    StepSlot slot[2];
+    StepSlot slot[3];
     double t;             // current time (realtype value)
     double dt;            // current_timestep (realtype value)
     double dt_stage1;     // Float64 dt of stage 1 (== dt for Float64)
@@ -217,7 +225,7 @@ __device__ inline double compute_rain(const KParams& P, double t) {
 // Non-directional sources on the w component, in source-list order
 // (system.jl:72-74): rain adds rate(t), infiltration subtracts its rate.
 template <class S>
-__device__ __forceinline__ S apply_sources(const KParams& P, const StepSlot& sl, S w, size_t k) {
+__device__ __forceinline__ S apply_sources(const KParams& P, const StepRates& sl, S w, size_t k) {
     auto infil = [&](S x) -> S {
         if (P.infil_kind == 2) return (S)(x - P.factor[k] * sl.infil_tfac);
         if (P.infil_kind == 1) return (S)(x - sl.infil_tfac);
@@ -231,18 +239,20 @@ __device__ __forceinline__ S apply_sources(const KParams& P, const StepSlot& sl,
 }
 
 // The time-dependent source rates of a step starting at t.
-__device__ inline void set_rates(const KParams& P, StepSlot& s, double t) {
+template <bool NO_HORTON = false>      // the caller knows the run has no Horton infiltration
+__device__ inline void set_rates(const KParams& P, StepRates& s, double t) {
     s.t = t;
     s.rain_now = compute_rain(P, t);
-    if (P.infil_kind == 2) s.infil_tfac = P.fc + (P.f0 - P.fc) * exp(-P.hk * t);
+    if (!NO_HORTON && P.infil_kind == 2) s.infil_tfac = P.fc + (P.f0 - P.fc) * exp(-P.hk * t);
     else if (P.infil_kind == 1) s.infil_tfac = P.infil_rate;
     else s.infil_tfac = 0.0;
 }
 
 // Close the step of `slot` with its dt: t += dt (simulator.jl:205), count
-// it, and arm the next slot (active unless the run ends here).  One thread.
+// it, and arm slot `next` (active unless the run ends here); the maxima of
+// slot `clear` restart at zero.  One thread.
 template <class S, bool NO_HORTON = false>
-__device__ inline void close_step(const KParams& P, StepCtl* c, int slot) {
+__device__ inline void close_step(const KParams& P, StepCtl* c, int slot, int next, int clear) {
     const S dt = (S)c->dt;
     const S t = (S)((S)c->slot[slot].t + dt);
     c->t = (double)t;
@@ -250,17 +260,15 @@ __device__ inline void close_step(const KParams& P, StepCtl* c, int slot) {
     if (!__builtin_isfinite((double)dt)) c->nonfinite = 1;
     bool act = c->max_steps <= 0 || c->steps < c->max_steps;
     if (c->endtime == c->endtime) act = act && (t < c->endtime);   // NaN endtime: fixed step count
-    StepSlot& nx = c->slot[1 - slot];
-    clear_wsmax(nx);
-    nx.active = act ? 1 : 0;
-    if (NO_HORTON) {            // the caller knows the run has no Horton infiltration
-        nx.t = (double)t;
-        nx.rain_now = compute_rain(P, (double)t);
-        nx.infil_tfac = P.infil_kind == 1 ? P.infil_rate : 0.0;
-    } else {
-        set_rates(P, nx, (double)t);
-    }
+    clear_wsmax(c->slot[clear]);
+    c->slot[next].active = act ? 1 : 0;
+    set_rates<NO_HORTON>(P, c->slot[next], (double)t);
 }
+template <class S, bool NO_HORTON = false>
+__device__ inline void close_step(const KParams& P, StepCtl* c, int slot) {
+    close_step<S, NO_HORTON>(P, c, slot, 1 - slot, 1 - slot);
+}
+__host__ __device__ inline int next_of_three(int slot) { return slot == 2 ? 0 : slot + 1; }
 
 
 // The same, out of line, for the persistent batch kernels (their KParams

@@ -10,7 +10,7 @@ template <class S>
 __global__ void k_flux(KParams P, StepCtl* ctl, int slot, const S* X, S* RHS, const double* B, int record);
 template <class S>
 __global__ void k_finish(KParams P, StepCtl* ctl, int slot, int stage, const S* U0, const S* X, const S* RHS, S* Out,
-                         const double* B, int rhs_interior, int close, S* ghost_rhs);
+                         const double* B, int rhs_interior, int next, S* ghost_rhs);
 
 // ---- boundary condition and step control (swe_kernels_ctl.hip)
 template <class S>
@@ -29,7 +29,7 @@ hipError_t launch_flux(hipStream_t st, const KParams& P, StepCtl* ctl, int slot,
 template <class S>
 hipError_t launch_finish(hipStream_t st, const KParams& P, StepCtl* ctl, int slot, int stage, const S* U0, const S* X,
                          const S* RHS, S* Out, const double* B,
-                         int rhs_interior = 0, int close = 0, S* ghost_rhs = nullptr);
+                         int rhs_interior = 0, int next = -1, S* ghost_rhs = nullptr);
 template <class S>
 hipError_t launch_bc(hipStream_t st, const KParams& P, StepCtl* ctl, int slot, S* U, int mode);
 hipError_t launch_prepare(hipStream_t st, const KParams& P, StepCtl* ctl, int slot, double t, double endtime,
@@ -80,13 +80,19 @@ hipError_t launch_interior_copy(hipStream_t st, const KParams& P, const void* pa
 // maps name interior cells), so U2's ghosts are left unwritten and filled
 // when something outside the march path needs them.  close = 1: stage 2 also
 // closes the step (t += dt, next slot armed), as k_bc's last stage does.
+// stage = 3 (ForwardEuler): finishes the step of `slot` from U0 and RHS1 into
+// UO (interior and domain corners), as stage 2's input, closes it into the
+// next of the three slots, and writes the next step's right-hand side to OUT
+// and its wave speeds to that slot.  Where a ghost's source is a ghost
+// (KParams::ghost_self), it writes the high-side ghosts of UO too; this
+// needs gc = 2.
 template <class S>
 hipError_t launch_march(hipStream_t st, const KParams& P, StepCtl* ctl, int slot, int stage, const S* U0,
-                        const S* RHS1, S* OUT, const double* B, int close = 0, int remap_halo = 0);
+                        const S* RHS1, S* OUT, const double* B, int close = 0, int remap_halo = 0, S* UO = nullptr);
 // The same stages with one workgroup per strip segment (swe_kernels_block.hip).
 template <class S>
 hipError_t launch_block(hipStream_t st, const KParams& P, StepCtl* ctl, int slot, int stage, const S* U0,
-                        const S* RHS1, S* OUT, const double* B, int close = 0, int remap_halo = 0);
+                        const S* RHS1, S* OUT, const double* B, int close = 0, int remap_halo = 0, S* UO = nullptr);
 constexpr int BLOCK_MAX_ROWS = 28;   // output rows per workgroup
 // Do these kernels suit the grid (one workgroup per CU, at most
 // BLOCK_MAX_ROWS rows each), without a measurement?
@@ -94,9 +100,9 @@ bool block_suits(const KParams& P);
 // Either kernel: the workgroup ones where they suit the grid.
 template <class S>
 hipError_t launch_stage(hipStream_t st, const KParams& P, StepCtl* ctl, int slot, int stage, const S* U0,
-                        const S* RHS1, S* OUT, const double* B, int close = 0, int remap_halo = 0) {
-    return block_suits(P) ? launch_block<S>(st, P, ctl, slot, stage, U0, RHS1, OUT, B, close, remap_halo)
-                          : launch_march<S>(st, P, ctl, slot, stage, U0, RHS1, OUT, B, close, remap_halo);
+                        const S* RHS1, S* OUT, const double* B, int close = 0, int remap_halo = 0, S* UO = nullptr) {
+    return block_suits(P) ? launch_block<S>(st, P, ctl, slot, stage, U0, RHS1, OUT, B, close, remap_halo, UO)
+                          : launch_march<S>(st, P, ctl, slot, stage, U0, RHS1, OUT, B, close, remap_halo, UO);
 }
 
 }  // namespace sfv

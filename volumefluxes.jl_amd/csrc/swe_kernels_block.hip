@@ -55,14 +55,17 @@ __device__ __forceinline__ int y_slot(int w, int par) { return w < BW - 1 ? w : 
 template <class S, int STAGE, int MODE, int BW>
 __device__ __forceinline__ void block_tile(const KParams& P, StepCtl* ctl, int slot, int H, int strip, int seg,
                                            const S* __restrict__ U0, const S* __restrict__ RHS1,
-                                           S* __restrict__ OUT, const double* __restrict__ B, BlockSmem<S, BW>& sm,
+                                           S* __restrict__ OUT, S* __restrict__ UO, const double* __restrict__ B,
+                                           BlockSmem<S, BW>& sm,
                                            int serial, int remap, int close) {
     const StepSlot& sl = ctl->slot[slot];
+    // the slot of the step whose speeds are found here
+    const int rslot = STAGE == 3 ? next_of_three(slot) : slot;
     const int lane = threadIdx.x & (BL - 1);
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / BL);
     const bool first = strip == 0 && seg == 0;
     if (!sl.active) {                              // the same for the whole workgroup
-        if (STAGE == 2 && close && first && threadIdx.x == 0) ctl->slot[1 - slot].active = 0;
+        if (STAGE >= 2 && close && first && threadIdx.x == 0) ctl->slot[STAGE == 3 ? rslot : 1 - slot].active = 0;
         return;
     }
     const int gc = P.gc, nxT = P.nxT, nyT = P.nyT;
@@ -78,13 +81,22 @@ __device__ __forceinline__ void block_tile(const KParams& P, StepCtl* ctl, int s
 
     double dt_d = 0.0;
     S dt_s = S(0);
-    if (STAGE == 2) {
+    if (STAGE >= 2) {
         dt_d = wave_uniform(stage1_dt<S>(P, ctl, sl));
         dt_s = (S)dt_d;
     }
+    // the source rates of the right-hand side: this step's, in STAGE 3 the
+    // next one's (close_step gives its slot the same values)
+    StepRates nrates;
+    if (STAGE == 3) {
+        set_rates<MODE != 0>(P, nrates, (double)(S)((S)sl.t + dt_s));
+        nrates.rain_now = wave_uniform(nrates.rain_now);
+        nrates.infil_tfac = wave_uniform(nrates.infil_tfac);
+    }
+    const StepRates& rates = STAGE == 3 ? nrates : static_cast<const StepRates&>(sl);
     // ghost columns read their boundary-condition source; a wall's negated
     // normal momentum flips the sign bit
-    const bool rmp = STAGE == 2 || remap;
+    const bool rmp = STAGE >= 2 || remap;
     const bool xedge = rmp && (strip == 0 || gc + strip * BCOLS + BL - 3 >= nxT - gc);
     int sci = i;
     unsigned fx = 0u;
@@ -118,10 +130,17 @@ __device__ __forceinline__ void block_tile(const KParams& P, StepCtl* ctl, int s
             b0 = Bload_row(P, B, i, r);
             n0 = Bload_row(P, B, i + 1, r);
             bool ok = true;
-            if (STAGE == 2) {
+            if (STAGE >= 2) {
                 S rr[3];
                 rr[0] = row_ld(RHS1 + ro, nxT, sci); rr[1] = row_ld(RHS1 + n + ro, nxT, sci);
                 rr[2] = row_ld(RHS1 + 2 * n + ro, nxT, sci);
+                if constexpr (STAGE == 3 && MODE == MODE_GENERAL) {
+                    // a source that is a ghost has the non-directional sources only
+                    if (P.ghost_self && in_dom && (sci >= nxT - gc || sj >= nyT - gc)) {
+                        rr[0] = apply_sources(P, sl, S(0), (size_t)sci + ro);
+                        rr[1] = rr[2] = S(0);
+                    }
+                }
                 double c0 = b0, c1 = n0;
                 if (xedge || sj != r) { c0 = Bload_row(P, B, sci, sj); c1 = Bload_row(P, B, sci + 1, sj); }
                 const double c2 = Bload_row(P, B, sci, sj + 1), c3 = Bload_row(P, B, sci + 1, sj + 1);
@@ -137,6 +156,16 @@ __device__ __forceinline__ void block_tile(const KParams& P, StepCtl* ctl, int s
             cC[1] = flip_sign(cC[1], fx);
             cC[2] = flip_sign(cC[2], fyb);
             if (STAGE == 1) ok = __all(in_band((double)cC[0], (double)cC[1], (double)cC[2], b0));
+            if constexpr (STAGE == 3 && MODE == MODE_GENERAL) {
+                // ghosts on the high sides whose values live on in memory (gc = 2)
+                const bool gx = in_dom && i >= nxT - gc && r >= j0 && r < j0 + th;
+                const bool gy = out_col && r >= nyT - gc && j0 + th == nyT - gc;
+                if (P.ghost_self && (gx || gy)) {
+                    S* urow = UO + (size_t)nxT * r;
+#pragma unroll
+                    for (int v = 0; v < 3; ++v) row_st(urow + v * n, nxT, i, cC[v]);
+                }
+            }
             const int s = u_slot<BW>(w, par);
 #pragma unroll
             for (int v = 0; v < 3; ++v) sm.u[s][v][lane] = cC[v];
@@ -194,7 +223,7 @@ __device__ __forceinline__ void block_tile(const KParams& P, StepCtl* ctl, int s
                     for (int v = 0; v < 3; ++v) Rxl[v] = shfl_up1(Rx[v]);
                     const double spx = RNG ? central_upwind_rng<0, MODE != 0>(Rxl, Lx, P.phys, K, Fxm)
                                            : central_upwind(0, Rxl, Lx, P.phys, Fxm);
-                    if (STAGE == 1) raise_speed<RNG>(smx, (double)(S)spx);
+                    if (STAGE != 2) raise_speed<RNG>(smx, (double)(S)spx);
 #pragma unroll
                     for (int v = 0; v < 3; ++v)
                         accx[v] = (S)__builtin_fma(-P.inv_dx, shfl_dn1(Fxm[v]) - Fxm[v], 0.0);   // 0 - inv*diff
@@ -216,10 +245,10 @@ __device__ __forceinline__ void block_tile(const KParams& P, StepCtl* ctl, int s
             const S Rlow[3] = {Ryp[0], Ryp[1], Ryp[2]};
             if (band) {
                 const double spy = central_upwind_rng<1, MODE != 0>(Rlow, Ly, P.phys, K, Fy);
-                if (STAGE == 1) raise_speed<true>(smy, (double)(S)spy);
+                if (STAGE != 2) raise_speed<true>(smy, (double)(S)spy);
             } else {
                 const double spy = central_upwind(1, Rlow, Ly, P.phys, Fy);
-                if (STAGE == 1) raise_speed<false>(smy, (double)(S)spy);
+                if (STAGE != 2) raise_speed<false>(smy, (double)(S)spy);
             }
             const int t = y_slot<BW>(w, par);
 #pragma unroll
@@ -239,10 +268,15 @@ __device__ __forceinline__ void block_tile(const KParams& P, StepCtl* ctl, int s
                 for (int v = 0; v < 3; ++v) acc[v] = y_part<MODE, RNG>(P, accx[v], Fy[v] - sm.fy[s][v][lane]);
                 if (P.bottom)
                     acc[2] = (S)(acc[2] + bottom_term<MODE, RNG>(P, K, 1, Bly - 0.5 * (bp + np), Ryp[0] + Ryp[3]));
-                acc[0] = MODE ? uniform_sources<S>(P, sl, acc[0]) : apply_sources(P, sl, acc[0], k);
-                if (STAGE == 1) {
+                acc[0] = MODE ? uniform_sources<S>(P, rates, acc[0]) : apply_sources(P, rates, acc[0], k);
+                if (STAGE != 2) {
 #pragma unroll
                     for (int v = 0; v < 3; ++v) row_st(orow + v * n, nxT, i, acc[v]);
+                    if (STAGE == 3) {              // the new state
+                        S* urow = UO + (size_t)nxT * p;
+#pragma unroll
+                        for (int v = 0; v < 3; ++v) row_st(urow + v * n, nxT, i, cA[v]);
+                    }
                 } else {
                     S o[3];
                     stage2_cell<S, MODE, RNG>(P, K, x0, cA, acc, bcp, dt_s, o);
@@ -254,7 +288,7 @@ __device__ __forceinline__ void block_tile(const KParams& P, StepCtl* ctl, int s
             else finish(std::false_type{});
         }
     }
-    if (STAGE == 1) {
+    if (STAGE != 2) {
         smx = wave_max_u64(face_x_ok ? smx : 0ull);
         smy = wave_max_u64(out_col ? smy : 0ull);
         if (lane == 0) { sm.red[w][0] = smx; sm.red[w][1] = smy; }
@@ -265,16 +299,17 @@ __device__ __forceinline__ void block_tile(const KParams& P, StepCtl* ctl, int s
                 smx = sm.red[k][0] > smx ? sm.red[k][0] : smx;
                 smy = sm.red[k][1] > smy ? sm.red[k][1] : smy;
             }
-            raise_wsmax(&ctl->slot[slot], smx, smy);
+            raise_wsmax(&ctl->slot[rslot], smx, smy);
         }
     }
-    if (STAGE == 2 && first && w == 0) {
+    if (STAGE >= 2 && first && w == 0) {
         if (lane == 0) {
             ctl->dt = (double)dt_s;
             ctl->dt_stage1 = dt_d;
-            if (close) close_step<S, MODE != 0>(P, ctl, slot);
+            if (STAGE == 3) close_step<S, MODE != 0>(P, ctl, slot, rslot, next_of_three(rslot));
+            else if (close) close_step<S, MODE != 0>(P, ctl, slot);
         }
-        finish_corners<S, MODE != 0>(P, sl, U0, OUT, B, dt_d, dt_s, lane, BL);
+        finish_corners<S, MODE != 0, STAGE == 3>(P, sl, U0, STAGE == 3 ? UO : OUT, B, dt_d, dt_s, lane, BL);
     }
 }
 
@@ -282,12 +317,13 @@ __device__ __forceinline__ void block_tile(const KParams& P, StepCtl* ctl, int s
 template <class S, int STAGE, int MODE, int BW>
 __global__ void __launch_bounds__(BL* BW) __attribute__((amdgpu_waves_per_eu(4)))
 k_block(KParams P, StepCtl* ctl, int slot, int H, int strips, int segs, const S* __restrict__ U0,
-        const S* __restrict__ RHS1, S* __restrict__ OUT, const double* __restrict__ B, int remap, int close) {
+        const S* __restrict__ RHS1, S* __restrict__ OUT, S* __restrict__ UO, const double* __restrict__ B, int remap,
+        int close) {
     __shared__ BlockSmem<S, BW> sm;
     if (threadIdx.x == 0) sm.bad = 0;
     __syncthreads();
     const int t = xcd_tile(blockIdx.x, strips * segs);
-    block_tile<S, STAGE, MODE, BW>(P, ctl, slot, H, t % strips, t / strips, U0, RHS1, OUT, B, sm, 1, remap, close);
+    block_tile<S, STAGE, MODE, BW>(P, ctl, slot, H, t % strips, t / strips, U0, RHS1, OUT, UO, B, sm, 1, remap, close);
 }
 
 // Rows per workgroup: the smallest height at which every workgroup has a CU
@@ -333,23 +369,23 @@ static void by_waves(int H, F&& go) {
 
 template <class S>
 hipError_t launch_block(hipStream_t st, const KParams& P, StepCtl* ctl, int slot, int stage, const S* U0,
-                        const S* RHS1, S* OUT, const double* B, int close, int remap_halo) {
+                        const S* RHS1, S* OUT, const double* B, int close, int remap_halo, S* UO) {
     int H = block_height(P);
     if (H <= 0 || H > BLOCK_MAX_ROWS) H = BLOCK_MAX_ROWS;   // asked for on a larger grid: several rounds
     const int strips = (P.nx + BCOLS - 1) / BCOLS, segs = (P.ny + H - 1) / H;
     by_waves(H, [&](auto waves) {
         constexpr int BW = decltype(waves)::value;
-        by_stage_mode(stage, march_mode(P), [&](auto stg, auto mode) {
+        by_stage_mode<3>(stage, stage == 3 && P.ghost_self ? MODE_GENERAL : march_mode(P), [&](auto stg, auto mode) {
             hipLaunchKernelGGL((k_block<S, decltype(stg)::value, decltype(mode)::value, BW>), dim3(strips * segs),
-                               dim3(BL * BW), 0, st, P, ctl, slot, H, strips, segs, U0, RHS1, OUT, B, remap_halo,
+                               dim3(BL * BW), 0, st, P, ctl, slot, H, strips, segs, U0, RHS1, OUT, UO, B, remap_halo,
                                close);
         });
     });
     return hipPeekAtLastError();
 }
 template hipError_t launch_block<double>(hipStream_t, const KParams&, StepCtl*, int, int, const double*,
-                                         const double*, double*, const double*, int, int);
+                                         const double*, double*, const double*, int, int, double*);
 template hipError_t launch_block<float>(hipStream_t, const KParams&, StepCtl*, int, int, const float*, const float*,
-                                        float*, const double*, int, int);
+                                        float*, const double*, int, int, float*);
 
 }  // namespace sfv

@@ -78,7 +78,7 @@ __device__ void prepare_ctl(const KParams& P, StepCtl* c, int slot, double t, do
     c->precision = precision;
     bool act = true;
     if (until_endtime) act = t < endtime;
-    for (int s = 0; s < 2; ++s) {
+    for (int s = 0; s < 3; ++s) {
         clear_wsmax(c->slot[s]);
         c->slot[s].active = 0;
         set_rates(P, c->slot[s], t);

@@ -154,21 +154,24 @@ __device__ __forceinline__ void march_fence() {
 template <class S, int STAGE, int MODE = MODE_GENERAL, bool BATCH = false>
 __device__ __forceinline__ void march_tile(const KParams& P, StepCtl* ctl, int slot, int my, int strip, int seg,
                                            const S* __restrict__ U0, const S* __restrict__ RHS1,
-                                           S* __restrict__ OUT, const double* __restrict__ B,
+                                           S* __restrict__ OUT, S* __restrict__ UO, const double* __restrict__ B,
                                            MarchWin<S>& win, int remap, int par = 0, int close = 0,
                                            int prio_after = 0, int prio_total = 0, int prio_cap = 3) {
     const StepSlot& sl = ctl->slot[slot];
+    // the slot of the step whose speeds are found here
+    const int rslot = STAGE == 3 ? next_of_three(slot) : slot;
     const int lane = threadIdx.x & (MW - 1);
     if (!sl.active) {                              // the same for every wave of the block
         // an inactive step passes inactivity on, so steps launched past the
         // end of a run stay no-ops
-        if (STAGE == 2 && close && strip == 0 && seg == 0 && lane == 0) ctl->slot[1 - slot].active = 0;
+        if (STAGE >= 2 && close && strip == 0 && seg == 0 && lane == 0)
+            ctl->slot[STAGE == 3 ? next_of_three(slot) : 1 - slot].active = 0;
         return;
     }
     const int gc = P.gc, nxT = P.nxT, nyT = P.nyT;
     const int j0 = gc + seg * my;
     if (j0 >= nyT - gc) {                          // whole wave: past the grid
-        if (STAGE == 1) block_max_to_slot_m(0ull, 0ull, &ctl->slot[slot], par);
+        if (STAGE != 2) block_max_to_slot_m(0ull, 0ull, &ctl->slot[rslot], par);
         return;
     }
     const int th = min(my, nyT - gc - j0);
@@ -181,10 +184,19 @@ __device__ __forceinline__ void march_tile(const KParams& P, StepCtl* ctl, int s
 
     double dt_d = 0.0;
     S dt_s = S(0);
-    if (STAGE == 2) {
+    if (STAGE >= 2) {
         dt_d = wave_uniform(stage1_dt<S>(P, ctl, sl));
         dt_s = (S)dt_d;
     }
+    // the source rates of the right-hand side: this step's, in STAGE 3 the
+    // next one's (close_step gives its slot the same values)
+    StepRates nrates;
+    if (STAGE == 3) {
+        set_rates<MODE != 0>(P, nrates, (double)(S)((S)sl.t + dt_s));
+        nrates.rain_now = wave_uniform(nrates.rain_now);
+        nrates.infil_tfac = wave_uniform(nrates.infil_tfac);
+    }
+    const StepRates& rates = STAGE == 3 ? nrates : static_cast<const StepRates&>(sl);
 
     // Ghost cells are read through the boundary-condition maps (stage 2
     // always, stage 1 with remap): a ghost's value is its source's, with the
@@ -193,7 +205,7 @@ __device__ __forceinline__ void march_tile(const KParams& P, StepCtl* ctl, int s
     // and segments hold ghost columns or rows; the test is the same for the
     // whole wave.  The lanes span columns gc + strip*MX - 2 .. +61, the rows
     // loaded are j0 - 2 .. j0 + th + 1.
-    const bool rmp = STAGE == 2 || remap;
+    const bool rmp = STAGE >= 2 || remap;
     const bool xedge = rmp && (strip == 0 || gc + strip * MX + MW - 3 >= nxT - gc);
     const bool yedge = rmp && (j0 - 2 < gc || j0 + th + 1 >= nyT - gc);
     int sci = i;
@@ -210,7 +222,7 @@ __device__ __forceinline__ void march_tile(const KParams& P, StepCtl* ctl, int s
     // a row's stage input as loaded: the state, with stage 2 the right-hand
     // side and the upper bottom corners of the source cell
     struct Raw {
-        S x[3], r[STAGE == 2 ? 3 : 1];
+        S x[3], r[STAGE >= 2 ? 3 : 1];
         double c2, c3;
         int sj;
         unsigned fyb;
@@ -227,10 +239,17 @@ __device__ __forceinline__ void march_tile(const KParams& P, StepCtl* ctl, int s
         const size_t ro = (size_t)nxT * sj;        // row sj (uniform), column sci (per lane)
 #pragma unroll
         for (int v = 0; v < 3; ++v) o.x[v] = row_ld(U0 + v * n + ro, nxT, sci);
-        if (STAGE == 2) {
+        if (STAGE >= 2) {
 #pragma unroll
             for (int v = 0; v < 3; ++v) o.r[v] = row_ld(RHS1 + v * n + ro, nxT, sci);
             Bload_row2(P, B, sci, sj + 1, o.c2, o.c3);
+        }
+        if constexpr (STAGE == 3 && MODE == MODE_GENERAL) {
+            // a source that is a ghost has the non-directional sources only
+            if (P.ghost_self && in_dom && (sci >= nxT - gc || sj >= nyT - gc)) {
+                o.r[0] = apply_sources(P, sl, S(0), (size_t)sci + ro);
+                o.r[1] = o.r[2] = S(0);
+            }
         }
     };
     Raw raw;
@@ -245,7 +264,7 @@ __device__ __forceinline__ void march_tile(const KParams& P, StepCtl* ctl, int s
 #if SFV_MARCH_TIMELINE
         if (!BATCH && r < TL_ROWS && lane == 0) {
             const int tw = blockIdx.x * MWAVES + threadIdx.x / MW;
-            if (tw < TL_WAVES) tl_rows[STAGE - 1][tw][r] = __builtin_amdgcn_s_memrealtime();
+            if (tw < TL_WAVES) tl_rows[STAGE == 1 ? 0 : 1][tw][r] = __builtin_amdgcn_s_memrealtime();
         }
 #endif
         // Issue priority by iterations left (this segment's and, in the
@@ -285,6 +304,16 @@ __device__ __forceinline__ void march_tile(const KParams& P, StepCtl* ctl, int s
         cC[1] = flip_sign(cC[1], fxb);
         cC[2] = flip_sign(cC[2], fyb);
         if (STAGE == 1) band = band && __all(in_band(cC[0], cC[1], cC[2], b0));
+        if constexpr (STAGE == 3 && MODE == MODE_GENERAL) {
+            // ghosts on the high sides whose values live on in memory (gc = 2)
+            const bool gx = in_dom && i >= nxT - gc && jr >= j0 && jr < j0 + th;
+            const bool gy = out_col && jr >= nyT - gc && j0 + th == nyT - gc;
+            if (P.ghost_self && (gx || gy)) {
+                S* urow = UO + (size_t)nxT * jr;
+#pragma unroll
+                for (int v = 0; v < 3; ++v) row_st(urow + v * n, nxT, i, cC[v]);
+            }
+        }
 #pragma unroll
         for (int v = 0; v < 3; ++v) win.u[s0][v][lane] = cC[v];
         const double Bly = 0.5 * (bm1 + nm1), Bry = 0.5 * (b0 + n0);
@@ -316,7 +345,7 @@ __device__ __forceinline__ void march_tile(const KParams& P, StepCtl* ctl, int s
                 double Fy[3], Fyp[3];
                 const double spy = RNG ? central_upwind_rng<1, MODE != 0>(Ryp, Ly, P.phys, K, Fy)
                                        : central_upwind(1, Ryp, Ly, P.phys, Fy);
-                if (STAGE == 1) raise_speed<RNG>(smy, (double)(S)spy);
+                if (STAGE != 2) raise_speed<RNG>(smy, (double)(S)spy);
 #pragma unroll
                 for (int v = 0; v < 3; ++v) { Fyp[v] = win.fy[v][lane]; win.fy[v][lane] = Fy[v]; }
                 // finish row p = jr-2: y part on top of its x part, then sources
@@ -328,11 +357,16 @@ __device__ __forceinline__ void march_tile(const KParams& P, StepCtl* ctl, int s
                     for (int v = 0; v < 3; ++v) acc[v] = y_part<MODE, RNG>(P, win.ax[v][lane], Fy[v] - Fyp[v]);
                     if (P.bottom)
                         acc[2] = (S)(acc[2] + bottom_term<MODE, RNG>(P, K, 1, Bly - Blyp, Ryp[0] + Lyp0));
-                    acc[0] = MODE ? uniform_sources<S>(P, sl, acc[0])
-                                  : apply_sources(P, sl, acc[0], (size_t)i + (size_t)nxT * p);
-                    if (STAGE == 1) {
+                    acc[0] = MODE ? uniform_sources<S>(P, rates, acc[0])
+                                  : apply_sources(P, rates, acc[0], (size_t)i + (size_t)nxT * p);
+                    if (STAGE != 2) {
 #pragma unroll
                         for (int v = 0; v < 3; ++v) row_st(orow + v * n, nxT, i, acc[v]);
+                        if (STAGE == 3) {                          // the new state, from the window
+                            S* urow = UO + (size_t)nxT * p;
+#pragma unroll
+                            for (int v = 0; v < 3; ++v) row_st(urow + v * n, nxT, i, ua[v * MW]);
+                        }
                     } else {
                         // U1 of row p from the window; U0 (output rows are
                         // interior) once more from the cache
@@ -365,7 +399,7 @@ __device__ __forceinline__ void march_tile(const KParams& P, StepCtl* ctl, int s
                     double Fxm[3];
                     const double spx = RNG ? central_upwind_rng<0, MODE != 0>(Rxl, Lx, P.phys, K, Fxm)
                                            : central_upwind(0, Rxl, Lx, P.phys, Fxm);
-                    if (STAGE == 1) raise_speed<RNG>(smx, (double)(S)spx);
+                    if (STAGE != 2) raise_speed<RNG>(smx, (double)(S)spx);
                     S ax[3];
 #pragma unroll
                     for (int v = 0; v < 3; ++v)
@@ -389,25 +423,27 @@ __device__ __forceinline__ void march_tile(const KParams& P, StepCtl* ctl, int s
         s1 = s0;
         s0 = free;
     }
-    if (STAGE == 1) {
+    if (STAGE != 2) {
         // x faces this lane evaluated (its left face) that border an output cell
         const bool face_x_ok = in_dom && lane >= 2 && lane <= MX + 2 && (lane == 2 ? i < nxT - gc : i - 1 < nxT - gc);
-        block_max_to_slot_m(face_x_ok ? smx : 0ull, out_col ? smy : 0ull, &ctl->slot[slot], par);
+        block_max_to_slot_m(face_x_ok ? smx : 0ull, out_col ? smy : 0ull, &ctl->slot[rslot], par);
     }
 
     // dt for the host and the step's closing (t += dt, next slot armed), by
     // one lane: the other waves read only this step's slot, and the next
     // slot is read only by the next launches.
-    if (STAGE == 2 && strip == 0 && seg == 0) {
+    if (STAGE >= 2 && strip == 0 && seg == 0) {
         if (lane == 0) {
             ctl->dt = (double)dt_s;
             ctl->dt_stage1 = dt_d;
-            if (close) {
+            if (STAGE == 3) {
+                close_step<S, MODE != 0>(P, ctl, slot, rslot, next_of_three(rslot));
+            } else if (close) {
                 if (BATCH) close_step_call<S, MODE != 0>(P, ctl, slot);
                 else close_step<S, MODE != 0>(P, ctl, slot);
             }
         }
-        finish_corners<S, MODE != 0>(P, sl, U0, OUT, B, dt_d, dt_s, lane, MW);
+        finish_corners<S, MODE != 0, STAGE == 3>(P, sl, U0, STAGE == 3 ? UO : OUT, B, dt_d, dt_s, lane, MW);
     }
 }
 
@@ -419,7 +455,8 @@ template <class S, int STAGE, int MODE>
 __global__ void __launch_bounds__(MW* MWAVES)
 __attribute__((amdgpu_waves_per_eu(SFV_MARCH_MIN_WAVES)))
 k_march(KParams P, StepCtl* ctl, int slot, int my, int strips, int segs, const S* __restrict__ U0,
-        const S* __restrict__ RHS1, S* __restrict__ OUT, const double* __restrict__ B, int close, int remap) {
+        const S* __restrict__ RHS1, S* __restrict__ OUT, S* __restrict__ UO, const double* __restrict__ B, int close,
+        int remap) {
     const int t = xcd_tile(blockIdx.x, march_blocks(strips, segs));
     // the same for every lane of the wave; readfirstlane tells the compiler so
 #if SFV_MARCH_LINEAR
@@ -443,12 +480,12 @@ k_march(KParams P, StepCtl* ctl, int slot, int my, int strips, int segs, const S
     const unsigned long long tl0 = __builtin_amdgcn_s_memrealtime();
 #endif
     __shared__ MarchWin<S> win[MWAVES];
-    march_tile<S, STAGE, MODE>(P, ctl, slot, my, strip, seg, U0, RHS1, OUT, B, win[threadIdx.x / MW], remap, 0, close);
+    march_tile<S, STAGE, MODE>(P, ctl, slot, my, strip, seg, U0, RHS1, OUT, UO, B, win[threadIdx.x / MW], remap, 0, close);
 #if SFV_MARCH_TIMELINE
     const unsigned long long tl1 = __builtin_amdgcn_s_memrealtime();
     const int tw = blockIdx.x * MWAVES + threadIdx.x / MW;
     if ((threadIdx.x & (MW - 1)) == 0 && tw < TL_WAVES) {
-        unsigned long long* o = tl_wave[STAGE - 1][tw];
+        unsigned long long* o = tl_wave[STAGE == 1 ? 0 : 1][tw];
         o[0] = tl0;
         o[1] = tl1;
         o[2] = __builtin_amdgcn_s_getreg((31 << 11) | 4);                       // HW_ID
@@ -501,7 +538,7 @@ k_march_batch(const BatchMember* __restrict__ mem, const BatchHeader* __restrict
         const int after = hdr->prio == 1 ? -1 : ((c1 - 1 - t) / per) * (M.my + 4);
         const int total = ntiles * (M.my + 4);
         march_tile<S, STAGE, MODE, true>(M.P, M.ctl, slot, M.my, strip, seg, U0, STAGE == 1 ? nullptr : (const S*)M.RHS,
-                                         STAGE == 1 ? (S*)M.RHS : (S*)M.U[cur ^ 1], M.B, win[threadIdx.x / MW], 1, par,
+                                         STAGE == 1 ? (S*)M.RHS : (S*)M.U[cur ^ 1], nullptr, M.B, win[threadIdx.x / MW], 1, par,
                                          1, after, total, cap);
     }
 }
@@ -566,13 +603,13 @@ int march_rows_per_wave(const KParams& P, int stage, int precision) {
 
 template <class S>
 hipError_t launch_march(hipStream_t st, const KParams& P, StepCtl* ctl, int slot, int stage, const S* U0,
-                        const S* RHS1, S* OUT, const double* B, int close, int remap_halo) {
+                        const S* RHS1, S* OUT, const double* B, int close, int remap_halo, S* UO) {
     const int my = P.rows > 0 ? P.rows : march_rows_per_wave(P, stage, std::is_same<S, float>::value ? 1 : 0);
     const int segs = (P.ny + my - 1) / my;
     const int strips = (P.nx + MX - 1) / MX;
-    by_stage_mode(stage, march_mode(P), [&](auto stg, auto mode) {
+    by_stage_mode<3>(stage, stage == 3 && P.ghost_self ? MODE_GENERAL : march_mode(P), [&](auto stg, auto mode) {
         hipLaunchKernelGGL((k_march<S, decltype(stg)::value, decltype(mode)::value>), dim3(march_blocks(strips, segs)),
-                           dim3(MW * MWAVES), 0, st, P, ctl, slot, my, strips, segs, U0, RHS1, OUT, B, close,
+                           dim3(MW * MWAVES), 0, st, P, ctl, slot, my, strips, segs, U0, RHS1, OUT, UO, B, close,
                            remap_halo);
     });
     return hipPeekAtLastError();
@@ -581,7 +618,7 @@ template <class S>
 hipError_t launch_march_batch(hipStream_t st, int stage, const BatchMember* mem, const BatchHeader* hdr, int lp,
                               int blocks, int mode) {
     if (blocks < N_XCD || blocks % N_XCD) return hipErrorInvalidValue;
-    by_stage_mode(stage, mode, [&](auto stg, auto m) {
+    by_stage_mode<2>(stage, mode, [&](auto stg, auto m) {
         hipLaunchKernelGGL((k_march_batch<S, decltype(stg)::value, decltype(m)::value>), dim3(blocks),
                            dim3(MW * MWAVES), 0, st, mem, hdr, lp);
     });
@@ -591,7 +628,7 @@ hipError_t launch_march_batch(hipStream_t st, int stage, const BatchMember* mem,
 int march_batch_blocks_per_cu(int precision, int stage, int mode) {
     int blocks = 0;
     hipError_t e = hipErrorUnknown;
-    by_stage_mode(stage, mode, [&](auto stg, auto m) {
+    by_stage_mode<2>(stage, mode, [&](auto stg, auto m) {
         constexpr int ST = decltype(stg)::value, M = decltype(m)::value;
         e = precision == 0 ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, k_march_batch<double, ST, M>, MW * MWAVES, 0)
                            : hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, k_march_batch<float, ST, M>, MW * MWAVES, 0);
@@ -604,9 +641,9 @@ template hipError_t launch_march_batch<double>(hipStream_t, int, const BatchMemb
 template hipError_t launch_march_batch<float>(hipStream_t, int, const BatchMember*, const BatchHeader*, int, int,
                                               int);
 template hipError_t launch_march<double>(hipStream_t, const KParams&, StepCtl*, int, int, const double*,
-                                         const double*, double*, const double*, int, int);
+                                         const double*, double*, const double*, int, int, double*);
 template hipError_t launch_march<float>(hipStream_t, const KParams&, StepCtl*, int, int, const float*, const float*,
-                                        float*, const double*, int, int);
+                                        float*, const double*, int, int, float*);
 
 }  // namespace sfv
 

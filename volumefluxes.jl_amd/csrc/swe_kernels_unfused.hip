@@ -125,12 +125,12 @@ __global__ void __launch_bounds__(256) k_flux(KParams P, StepCtl* ctl, int slot,
 template <class S>
 __global__ void __launch_bounds__(256) k_finish(KParams P, StepCtl* ctl, int slot, int stage, const S* __restrict__ U0,
                                                 const S* __restrict__ X, const S* RHS, S* __restrict__ Out,
-                                                const double* __restrict__ B, int rhs_interior, int close,
+                                                const double* __restrict__ B, int rhs_interior, int next,
                                                 S* ghost_rhs) {
     const StepSlot& sl = ctl->slot[slot];
-    const bool closer = close && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0 && threadIdx.y == 0;
+    const bool closer = next >= 0 && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0 && threadIdx.y == 0;
     if (!sl.active) {
-        if (closer) ctl->slot[1 - slot].active = 0;   // steps past the end of a run stay no-ops
+        if (closer) ctl->slot[next].active = 0;   // steps past the end of a run stay no-ops
         return;
     }
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -144,14 +144,14 @@ __global__ void __launch_bounds__(256) k_finish(KParams P, StepCtl* ctl, int slo
         if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0 && threadIdx.y == 0) {
             ctl->dt = (double)dt_s;
             ctl->dt_stage1 = dt_d;
-            // a one-stage step may close here (t += dt, next slot armed): the
-            // other threads read only this step's slot
-            if (close) close_step<S>(P, ctl, slot);
         }
     } else {
         dt_s = (S)ctl->dt;
         dt_d = (double)dt_s;
     }
+    // a step's last update may close it here (t += dt, slot `next` armed): the
+    // other threads read only this step's slot and dt
+    if (closer) close_step<S>(P, ctl, slot, next, next);
     if (i >= P.nxT || j >= P.nyT) return;
     const size_t n = (size_t)P.nxT * P.nyT;
     const size_t k = cid(P, i, j);
@@ -204,11 +204,11 @@ hipError_t launch_flux(hipStream_t st, const KParams& P, StepCtl* ctl, int slot,
 }
 template <class S>
 hipError_t launch_finish(hipStream_t st, const KParams& P, StepCtl* ctl, int slot, int stage, const S* U0, const S* X,
-                         const S* RHS, S* Out, const double* B, int rhs_interior, int close, S* ghost_rhs) {
+                         const S* RHS, S* Out, const double* B, int rhs_interior, int next, S* ghost_rhs) {
     const dim3 block(64, 4);
     const dim3 grid((P.nxT + 63) / 64, (P.nyT + 3) / 4);
     hipLaunchKernelGGL(k_finish<S>, grid, block, 0, st, P, ctl, slot, stage, U0, X, RHS, Out, B, rhs_interior,
-                       close, ghost_rhs);
+                       next, ghost_rhs);
     return hipPeekAtLastError();
 }
 template hipError_t launch_flux<double>(hipStream_t, const KParams&, StepCtl*, int, const double*, double*,

@@ -97,7 +97,7 @@ __device__ __forceinline__ void row_st(float* row, int len, int col, float v) {
 
 // Stage-1 result of one cell (rungekutta.jl:38-41 with the Float64 dt,
 // friction.jl:80-84 from U0 with the stored dt, timestepper.jl:53-63).
-// FAST: the friction law is none or bh2021 (march_fast).
+// FAST: the friction law is none or bh2021.
 template <class S, bool FAST = false>
 __device__ __forceinline__ void stage1_cell(const KParams& P, const S x[3], const S r[3], double Bm, double dt_d,
                                             S dt_s, S o[3]) {
@@ -118,7 +118,7 @@ __device__ __forceinline__ void stage1_cell(const KParams& P, const S x[3], cons
 // Rain and infiltration on the w component where both are uniform in space,
 // in source-list order (apply_sources).
 template <class S>
-__device__ __forceinline__ S uniform_sources(const KParams& P, const StepSlot& sl, S w) {
+__device__ __forceinline__ S uniform_sources(const KParams& P, const StepRates& sl, S w) {
     auto infil = [&](S x) -> S { return P.infil_kind ? (S)(x - sl.infil_tfac) : x; };
     auto rain = [&](S x) -> S { return P.rain_kind ? (S)(x + sl.rain_now) : x; };
     return P.rain_first ? infil(rain(w)) : rain(infil(w));
@@ -289,9 +289,10 @@ __device__ __forceinline__ float flip_sign(float v, unsigned mask) {
 // Stage 2 on the gc x gc corner cells of the domain, by `lanes` threads:
 // never written by the boundary condition (bc.jl:92-109) nor read by a
 // stencil, but part of the state; both stages run sources, RK update,
-// friction and clamp on them.
-template <class S, bool FAST>
-__device__ __forceinline__ void finish_corners(const KParams& P, const StepSlot& sl, const S* __restrict__ U0,
+// friction and clamp on them.  ONE_STAGE: the ForwardEuler step, which is the
+// first of the two.
+template <class S, bool FAST, bool ONE_STAGE>
+__device__ __forceinline__ void finish_corners(const KParams& P, const StepRates& sl, const S* __restrict__ U0,
                                                S* __restrict__ OUT, const double* __restrict__ B, double dt_d, S dt_s,
                                                int lane, int lanes) {
     const int gc = P.gc, nxT = P.nxT, nyT = P.nyT;
@@ -308,6 +309,12 @@ __device__ __forceinline__ void finish_corners(const KParams& P, const StepSlot&
         const S rs[3] = {src, S(0), S(0)};
         S u1[3];
         stage1_cell<S, FAST>(P, x, rs, Bm, dt_d, dt_s, u1);
+        if (ONE_STAGE) {
+            OUT[k] = u1[0];
+            OUT[n + k] = u1[1];
+            OUT[2 * n + k] = u1[2];
+            continue;
+        }
         S o[3];
 #pragma unroll
         for (int v = 0; v < 3; ++v) o[v] = (S)(u1[v] + dt_s * rs[v]);
@@ -339,16 +346,18 @@ __device__ __forceinline__ int xcd_tile(int L, int N) {
     return x * q + min(x, r) + k;
 }
 
-// kernel(stage, mode) for a run-time stage and mode.
-template <class F>
+// kernel(stage, mode) for a run-time stage (1 to STAGES) and mode.
+template <int STAGES, class F>
 inline void by_stage_mode(int stage, int mode, F&& go) {
     auto with = [&](auto st) {
         if (mode == MODE_POW2) go(st, std::integral_constant<int, MODE_POW2>{});
         else if (mode == MODE_FAST) go(st, std::integral_constant<int, MODE_FAST>{});
         else go(st, std::integral_constant<int, MODE_GENERAL>{});
     };
-    if (stage == 1) with(std::integral_constant<int, 1>{});
-    else with(std::integral_constant<int, 2>{});
+    if (stage == 1) return with(std::integral_constant<int, 1>{});
+    if constexpr (STAGES == 3)
+        if (stage == 3) return with(std::integral_constant<int, 3>{});
+    with(std::integral_constant<int, 2>{});
 }
 
 }  // namespace sfv

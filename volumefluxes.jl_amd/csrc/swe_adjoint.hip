@@ -10,12 +10,14 @@
 // differentiated; dt is differentiated through its maximum wave speed.
 //
 // Memory: the forward pass keeps a checkpoint every `checkpoint_every`
-// steps.  The reverse pass recomputes one segment from its checkpoint (the
-// per-pass kernels, bitwise the forward run), keeping each step's stage-1
-// state U1, right-hand sides R1 = L(U0) + sources, R2 = L(U1) + sources and
-// control block when they fit (on a second stream, overlapped with the
-// previous segment's reverse steps, when two sets fit), then walks it
-// backwards.  Per stage in reverse order a reverse step applies the
+// steps.  The reverse pass recomputes one segment from its checkpoint
+// (bitwise the forward run; the last segment is kept as the forward pass runs
+// it), keeping each step's stage-1 state U1, right-hand sides R1 = L(U0) +
+// sources, R2 = L(U1) + sources, dt and maximum speeds when they fit (on a
+// second stream, overlapped with the previous segment's reverse steps, when
+// two sets fit), then walks it backwards.  A kept step is three launches:
+// stage 1 (R1), stage 3 (U1 and R2) and k_adj_finish (U2 and the ghosts); at
+// 512^2 f64 they take 43 us where the per-pass chain of eight took 75.  Per stage in reverse order a reverse step applies the
 // boundary-condition fold (read as a gather), dry clamp, implicit friction
 // and the RK combination, then the face fluxes of both directions (the
 // central-upwind flux swept back by hand at each face) and the
@@ -126,36 +128,58 @@ __device__ __forceinline__ double desing_dh(double h, double kappa) {
     return sg * (mx_mn ? dmn : sg);
 }
 
-// One side of a face: its flux f and eigenvalues e (swe_2D.jl:43-81), zero
-// for a dry side (centralupwind.jl:51-61 leaves them at zero).
-__device__ __forceinline__ bool side_values(int d, const double s[3], const PhysParams& p, double f[3], double e[2]) {
-    for (int v = 0; v < 3; ++v) f[v] = 0.0;
-    e[0] = e[1] = 0.0;
-    if (!(s[0] > p.cutoff)) return false;
-    ad::phys<double>(d, s[0], s[1], s[2], p, f, e);
-    return true;
+// One side of a face (swe_2D.jl:43-81): its flux f and eigenvalues e, zero
+// for a dry side (centralupwind.jl:51-61 leaves them at zero), and what its
+// reverse sweep takes up again: h* = desingularize(h), the normal and
+// tangential velocities un = s_n / h* and ut = s_t / h*, and c = sqrt(g h).
+struct Side {
+    double f[3], e[2], hs, un, ut, c;
+    bool wet;
+};
+__device__ __forceinline__ Side side_values(int d, const double s[3], const PhysParams& p) {
+    Side o;
+    for (int v = 0; v < 3; ++v) o.f[v] = 0.0;
+    o.e[0] = o.e[1] = 0.0;
+    o.hs = 1.0;
+    o.un = o.ut = o.c = 0.0;
+    o.wet = s[0] > p.cutoff;
+    if (!o.wet) return o;
+    const double h = s[0];
+    o.hs = ad::desingularize<double>(h, p.kappa);
+    const double u = s[1] / o.hs, v = s[2] / o.hs;
+    o.un = d == 0 ? u : v;
+    o.ut = d == 0 ? v : u;
+    const double h2 = h * h;
+    o.c = sqrt(p.g * h);
+    if (d == 0) {
+        o.f[0] = p.rho * h * u;
+        o.f[1] = p.rho * h * u * u + 0.5 * p.rho * p.g * h2;
+        o.f[2] = p.rho * h * u * v;
+    } else {
+        o.f[0] = p.rho * h * v;
+        o.f[1] = p.rho * h * u * v;
+        o.f[2] = p.rho * h * v * v + 0.5 * p.rho * p.g * h2;
+    }
+    o.e[0] = o.un + o.c;
+    o.e[1] = o.un - o.c;
+    return o;
 }
 
 // Reverse sweep of one wet side: given the adjoints lf of its flux and le of
 // its eigenvalues, the adjoint of its state (h, hu, hv).  With the normal
-// momentum n = 1 + d and the tangential t = 2 - d, the side computes
-// un = s_n / hs, ut = s_t / hs, hs = desingularize(h), c = sqrt(g h),
+// momentum at n = 1 + d and the tangential at t = 2 - d,
 // f = [rho h un, rho h un^2 + 0.5 rho g h^2 (at n), rho h un ut (at t)],
 // e = [un + c, un - c].
-__device__ __forceinline__ void side_vjp(int d, const double s[3], const PhysParams& p, const double lf[3],
+__device__ __forceinline__ void side_vjp(int d, double h, const Side& o, const PhysParams& p, const double lf[3],
                                          const double le[2], double ls[3]) {
-    const double h = s[0];
-    const double sn = d == 0 ? s[1] : s[2], st = d == 0 ? s[2] : s[1];
     const double ln = d == 0 ? lf[1] : lf[2], lt = d == 0 ? lf[2] : lf[1];
-    const double hs = ad::desingularize<double>(h, p.kappa);
-    const double un = sn / hs, ut = st / hs;
-    const double c = sqrt(p.g * h);
+    const double un = o.un, ut = o.ut;
     const double rh = p.rho * h;
     const double l_un = lf[0] * rh + ln * (2.0 * rh * un) + lt * (rh * ut) + le[0] + le[1];
     const double l_ut = lt * (rh * un);
     double l_h = lf[0] * (p.rho * un) + ln * (p.rho * un * un + p.rho * p.g * h) + lt * (p.rho * un * ut);
-    if (c > 0.0) l_h += (le[0] - le[1]) * (p.g * (0.5 / c));
-    const double ihs = 1.0 / hs;
+    if (o.c > 0.0) l_h += (le[0] - le[1]) * (p.g * (0.5 / o.c));
+    const double ihs = 1.0 / o.hs;
     const double l_hs = -(l_un * un + l_ut * ut) * ihs;
     ls[0] = l_h + l_hs * desing_dh(h, p.kappa);
     const double l_sn = l_un * ihs, l_st = l_ut * ihs;
@@ -171,9 +195,8 @@ __device__ __forceinline__ void side_vjp(int d, const double s[3], const PhysPar
 // differentiated by hand (side_vjp).
 __device__ __forceinline__ void face_vjp(int d, const double m[3], const double q[3], const PhysParams& p, const double lF[3],
                          double lm[3], double lq[3], double& speed, double l_speed = 0.0) {
-    double fm[3], em[2], fp[3], ep[2];
-    const bool wm = side_values(d, m, p, fm, em);
-    const bool wq = side_values(d, q, p, fp, ep);
+    const Side sm = side_values(d, m, p), sq = side_values(d, q, p);
+    const double *fm = sm.f, *em = sm.e, *fp = sq.f, *ep = sq.e;
     for (int v = 0; v < 3; ++v) lm[v] = lq[v] = 0.0;
     const int pk1 = jmax_pick(ep[0], em[0]);
     const double ap1 = pk1 ? em[0] : ep[0];
@@ -225,8 +248,8 @@ __device__ __forceinline__ void face_vjp(int d, const double m[3], const double 
         else l_ep[1] += l_am;
     }
     double gm[3] = {0.0, 0.0, 0.0}, gq[3] = {0.0, 0.0, 0.0};
-    if (wm) side_vjp(d, m, p, l_fm, l_em, gm);
-    if (wq) side_vjp(d, q, p, l_fp, l_ep, gq);
+    if (sm.wet) side_vjp(d, m[0], sm, p, l_fm, l_em, gm);
+    if (sq.wet) side_vjp(d, q[0], sq, p, l_fp, l_ep, gq);
     for (int a = 0; a < 3; ++a) {
         lm[a] += gm[a];
         lq[a] += gq[a];
@@ -298,27 +321,24 @@ __device__ void recon_at(const KParams& P, const double* U, const double* B, int
     ad::reconstruct(cl, cc, cr, P.theta, Bl, Br, L, R);
 }
 
-// Face states of cell (i,j) along d, as recon_at<double> gives them, and the
-// branch each slope took (linearreconstruction.jl:28-43, 81-91): pick[v] is
-// 0 for theta*fwd, 1 for (fwd+bwd)/2, 2 for theta*bwd, 3 for minmod's zero;
-// dry is 0, or 1 for the 2(w - Bl) line, 2 for the 2(Br - w) line.  Ties
-// resolve as Julia's min/max (and djl_min/djl_max) resolve them.  Every
-// branch is linear in its stencil, and variable v's face states depend on
-// variable v only, so the picks give the reconstruction's Jacobian.
-__device__ void recon_pick(const KParams& P, const double* U, const double* B, int d, int i, int j, double L[3],
-                           double R[3], int pick[3], int& dry) {
-    const size_t n = (size_t)P.nxT * P.nyT;
-    const int di = d == 0 ? 1 : 0, dj = d == 0 ? 0 : 1;
-    const double theta = P.theta;
-    double cc[3], slope[3];
+// Face states of a cell from its stencil l, c, r along a direction and its two
+// face bottoms, as reconstruct<double> gives them, and the branch each slope
+// took (linearreconstruction.jl:28-43, 81-91) as a byte, two bits each:
+// variable v's at bit 2v is 0 for theta*fwd, 1 for (fwd+bwd)/2, 2 for
+// theta*bwd, 3 for minmod's zero; the dry fix's at bit 6 is 0, or 1 for the
+// 2(w - Bl) line, 2 for the 2(Br - w) line.  Ties resolve as Julia's min/max
+// (and djl_min/djl_max) resolve them.  Every branch is linear in its stencil,
+// and variable v's face states depend on variable v only, so the byte gives
+// the reconstruction's Jacobian.
+__device__ __forceinline__ unsigned recon_pick(const double l[3], const double cc[3], const double r[3], double theta,
+                                               double Bl, double Br, double L[3], double R[3]) {
+    unsigned code = 0;
+    double slope[3];
+#pragma unroll
     for (int v = 0; v < 3; ++v) {
-        const double l = U[v * n + cid(P, i - di, j - dj)];
-        const double c = U[v * n + cid(P, i, j)];
-        const double r = U[v * n + cid(P, i + di, j + dj)];
-        cc[v] = c;
-        const double fwd = r - c, bwd = c - l;
+        const double fwd = r[v] - cc[v], bwd = cc[v] - l[v];
         const double a = theta * fwd, b = (fwd + bwd) / 2.0, e = theta * bwd;
-        int k = 3;
+        unsigned k = 3;
         double m = 0.0;
         if (a != a || b != b || e != e) {
         } else if (a > 0 && b > 0 && e > 0) {        // djl_min(djl_min(a, b), e)
@@ -330,25 +350,37 @@ __device__ void recon_pick(const KParams& P, const double* U, const double* B, i
             m = k ? b : a;
             if (e >= m) { k = 2; m = e; }
         }
-        pick[v] = k;
+        code |= k << (2 * v);
         slope[v] = m;
     }
-    const double Bl = B_face_left(P, B, i, j, d), Br = B_face_right(P, B, i, j, d);
     const double w = cc[0];
-    dry = 0;
-    if (w - 0.5 * slope[0] < Bl) { slope[0] = 2.0 * (w - Bl); dry = 1; }
-    else if (w + 0.5 * slope[0] < Br) { slope[0] = 2.0 * (Br - w); dry = 2; }
+    if (w - 0.5 * slope[0] < Bl) { slope[0] = 2.0 * (w - Bl); code |= 1u << 6; }
+    else if (w + 0.5 * slope[0] < Br) { slope[0] = 2.0 * (Br - w); code |= 2u << 6; }
+#pragma unroll
     for (int v = 0; v < 3; ++v) {
         L[v] = cc[v] - 0.5 * slope[v];
         R[v] = cc[v] + 0.5 * slope[v];
     }
     L[0] = L[0] - Bl;
     R[0] = R[0] - Br;
+    return code;
+}
+
+// Sum of the two face depths of a cell, from w's stencil and the byte
+// recon_pick gave it (the same operations along the branch taken).
+__device__ __forceinline__ double depth_sum(double l, double c, double r, double theta, double Bl, double Br,
+                                            unsigned code) {
+    const double fwd = r - c, bwd = c - l;
+    const unsigned k = code & 3u, dry = code >> 6 & 3u;
+    double slope = k == 0 ? theta * fwd : k == 1 ? (fwd + bwd) / 2.0 : k == 2 ? theta * bwd : 0.0;
+    slope = dry == 1 ? 2.0 * (c - Bl) : dry == 2 ? 2.0 * (Br - c) : slope;
+    const double L = c - 0.5 * slope - Bl, R = c + 0.5 * slope - Br;
+    return R + L;
 }
 
 // d slope / d U at stencil position p (-1 left, 0 centre, 1 right) for the
 // branch pick (and, for w, the dry-fix line).
-__device__ __forceinline__ double slope_coef(int pick, int dry, int p, double theta) {
+__device__ __forceinline__ double slope_coef(unsigned pick, unsigned dry, int p, double theta) {
     if (dry == 1) return p == 0 ? 2.0 : 0.0;
     if (dry == 2) return p == 0 ? -2.0 : 0.0;
     if (pick == 0) return p == 1 ? theta : (p == 0 ? -theta : 0.0);
@@ -357,7 +389,73 @@ __device__ __forceinline__ double slope_coef(int pick, int dry, int p, double th
     return 0.0;
 }
 
+// What a reverse step needs of its forward step's control: dt and the
+// wave-speed maxima it came from.
+struct AdjStep {
+    double dt;
+    unsigned long long ws[2];
+    double pad;
+};
+
 // ---------------------------------------------------------------- kernels
+
+// The end of a recomputed RK2 step, every cell: U2 = clamp(friction(0.5 (U0 +
+// U1 + dt R2))) (k_finish's stage 2).  A ghost takes its boundary-condition
+// source's value, and U1's ghosts are filled likewise, so that no
+// boundary-condition pass is needed; corners have sources only.  One thread
+// keeps the step's control for the reverse pass and closes the step.
+__global__ void __launch_bounds__(256) k_adj_finish(KParams P, StepCtl* ctl, int slot, const double* __restrict__ U0,
+                                                    double* U1, const double* __restrict__ R2, double* __restrict__ U2,
+                                                    const double* __restrict__ B, AdjStep* keep) {
+    if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0 && threadIdx.y == 0) {
+        keep->dt = ctl->dt_stage1;
+        for (int d = 0; d < 2; ++d) keep->ws[d] = slot_wsmax(ctl->slot[slot], d);
+        close_step<double>(P, ctl, slot);
+    }
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    // the launchers' blocks are 64 wide, so a wave shares threadIdx.y
+    const int j = __builtin_amdgcn_readfirstlane(blockIdx.y * blockDim.y + threadIdx.y);
+    if (i >= P.nxT || j >= P.nyT) return;
+    const int gc = P.gc;
+    const size_t n = (size_t)P.nxT * P.nyT;
+    const bool gx = i < gc || i >= P.nxT - gc, gy = j < gc || j >= P.nyT - gc;
+    int si = i, sj = j;
+    double fu = 1.0, fv = 1.0;
+    if (gx && !gy) {
+        const int g = i < gc ? i : i - (P.nxT - gc);
+        si = i < gc ? P.src_lo_x[g] : P.src_hi_x[g];
+        fu = (i < gc ? P.flip_lo_x[g] : P.flip_hi_x[g]) ? -1.0 : 1.0;
+    } else if (gy && !gx) {
+        const int g = j < gc ? j : j - (P.nyT - gc);
+        sj = j < gc ? P.src_lo_y[g] : P.src_hi_y[g];
+        fv = (j < gc ? P.flip_lo_y[g] : P.flip_hi_y[g]) ? -1.0 : 1.0;
+    }
+    const size_t k = cid(P, i, j), q = cid(P, si, sj);
+    const double dt = ctl->dt;
+    double x[3], r[3] = {0.0, 0.0, 0.0}, o[3];
+    for (int v = 0; v < 3; ++v) x[v] = U1[v * n + q];
+    if (gx && gy) r[0] = apply_sources(P, ctl->slot[slot], 0.0, k);
+    else for (int v = 0; v < 3; ++v) r[v] = R2[v * n + q];
+    for (int v = 0; v < 3; ++v) {
+        o[v] = x[v] + dt * r[v];
+        o[v] = 0.5 * (U0[v * n + q] + o[v]);
+    }
+    const double Bm = B_cell(P, B, si, sj);
+    if (P.friction) sfv::apply_friction(o, dt, sfv::friction_scalar(P.friction, P.Cz, P.phys.kappa, x[0], x[1], x[2], Bm));
+    if (o[0] - Bm < P.phys.cutoff) {
+        o[0] = jl_max(o[0], Bm);
+        o[1] = 0.0;
+        o[2] = 0.0;
+    }
+    U2[k] = o[0];
+    U2[n + k] = fu < 0 ? -o[1] : o[1];
+    U2[2 * n + k] = fv < 0 ? -o[2] : o[2];
+    if (gx != gy) {
+        U1[k] = x[0];
+        U1[n + k] = fu < 0 ? -x[1] : x[1];
+        U1[2 * n + k] = fv < 0 ? -x[2] : x[2];
+    }
+}
 
 // Boundary-condition fold (adjoint of update_bc!): ghost adjoints go to the
 // cells the ghosts were copied from (sign flipped with the momentum), then
@@ -464,9 +562,9 @@ __device__ void block_sum(double v, double* part, int slot) {
 // friction (scalar from `in`), dry clamp.  Lout: adjoint of the stage
 // output, read through its boundary-condition fold (folded_adj).  Stage 2 writes Lin and LU0 for every
 // cell and resets the step's argmax search (*best); stage 1 adds to Lin.
-// Writes LR = adjoint of R, adds the B_cell adjoint, and block partial sums
-// of the dt and Cz adjoints.
-__global__ void __launch_bounds__(256) k_adj_tail(KParams P, const StepCtl* ctl, int stage, const double* __restrict__ U0,
+// Writes LR = adjoint of R (interior cells), adds the B_cell adjoint, and block
+// partial sums of the dt and Cz adjoints.  24 planes of traffic: 14 us at 512^2.
+__global__ void __launch_bounds__(256) k_adj_tail(KParams P, const AdjStep* ctl, int stage, const double* __restrict__ U0,
                                                   const double* __restrict__ Uin, const double* __restrict__ R,
                                                   const double* __restrict__ B, const double* __restrict__ Lout,
                                                   double* __restrict__ Lin, double* __restrict__ LU0,
@@ -479,10 +577,18 @@ __global__ void __launch_bounds__(256) k_adj_tail(KParams P, const StepCtl* ctl,
     const int nblk = gridDim.x * gridDim.y, bid = blockIdx.x + gridDim.x * blockIdx.y;
     if (stage == 2 && bid == 0 && threadIdx.x == 0 && threadIdx.y == 0) *best = ~0ull;
     double gdt = 0.0, gcz = 0.0;
-    if (i < P.nxT && j < P.nyT) {
+    const bool interior = i >= P.gc && i < P.nxT - P.gc && j >= P.gc && j < P.nyT - P.gc;
+    if (!interior) {
+        // the boundary condition overwrites a ghost (a corner feeds nothing):
+        // its adjoint ends here; stage 1 keeps what Lin holds
+        if (stage == 2 && i < P.nxT && j < P.nyT) {
+            const size_t n = (size_t)P.nxT * P.nyT, k = cid(P, i, j);
+            for (int v = 0; v < 3; ++v) Lin[v * n + k] = LU0[v * n + k] = 0.0;
+        }
+    } else {
         const size_t n = (size_t)P.nxT * P.nyT;
         const size_t k = cid(P, i, j);
-        const double dt = ctl->dt_stage1;
+        const double dt = ctl->dt;
         double x[3], r[3], ax[3], pre[3], lo[3];
         for (int v = 0; v < 3; ++v) {
             x[v] = Uin[v * n + k];
@@ -493,8 +599,12 @@ __global__ void __launch_bounds__(256) k_adj_tail(KParams P, const StepCtl* ctl,
         folded_adj(P, Lout, i, j, lo);
         const double Bm = Bc4(P, B, i, j);
         double fs = 0.0, D = 1.0;
+        using D5 = Dual<5>;
+        D5 fsd(0.0);                               // value and derivatives to w, hu, hv, the bottom and Cz
         if (P.friction) {
-            fs = ad::friction_scalar<double>(P.friction, P.Cz, P.phys.kappa, x[0], x[1], x[2], Bm);
+            fsd = ad::friction_scalar<D5>(P.friction, D5::var(P.Cz, 4), P.phys.kappa, D5::var(x[0], 0),
+                                          D5::var(x[1], 1), D5::var(x[2], 2), D5::var(Bm, 3));
+            fs = fsd.v;
             D = 1 - dt * fs;
         }
         double o[3] = {pre[0] * (1 - dt * 0.0), pre[1] / D, pre[2] / D};
@@ -518,9 +628,6 @@ __global__ void __launch_bounds__(256) k_adj_tail(KParams P, const StepCtl* ctl,
             const double lD = -(lo[1] * pre[1] + lo[2] * pre[2]) / (D * D);
             const double lfs = lD * (-dt);
             gdt += lD * (-fs);
-            using D5 = Dual<5>;
-            const D5 fsd = ad::friction_scalar<D5>(P.friction, D5::var(P.Cz, 4), P.phys.kappa, D5::var(x[0], 0),
-                                               D5::var(x[1], 1), D5::var(x[2], 2), D5::var(Bm, 3));
             for (int v = 0; v < 3; ++v) lin[v] += lfs * fsd.d[v];
             lBc += lfs * fsd.d[3];
             gcz += lfs * fsd.d[4];
@@ -542,69 +649,112 @@ __global__ void __launch_bounds__(256) k_adj_tail(KParams P, const StepCtl* ctl,
 
 // The direction whose wave speed set dt: min(Δx/a_x, Δy/a_y) picks y on a
 // tie (simulator.jl:147-150 with Julia's minimum).
-__device__ __forceinline__ int dt_direction(const KParams& P, const StepCtl* ctl) {
-    const double ax = __longlong_as_double((long long)slot_wsmax(ctl->slot[0], 0));
-    const double ay = __longlong_as_double((long long)slot_wsmax(ctl->slot[0], 1));
+__device__ __forceinline__ int dt_direction(const KParams& P, const AdjStep* ctl) {
+    const double ax = __longlong_as_double((long long)ctl->ws[0]);
+    const double ay = __longlong_as_double((long long)ctl->ws[1]);
     return (P.dx / ax < P.dy / ay) ? 0 : 1;
 }
 
-// Face fluxes of direction d (numericalflux.jl:21-33): face between cell c
-// and c+1 along d, c from gc-1 to nT-gc-1, other index interior.  The flux
+// Face fluxes of both directions (numericalflux.jl:21-33): face between cell
+// c and c+1 along d, c from gc-1 to nT-gc-1, other index interior.  The flux
 // adjoint is (1/Δ)(LR(c+1) - LR(c)) over interior cells; its transpose
 // through the central-upwind Jacobian gives the adjoints of c's right face
-// state and (c+1)'s left face state.
-__global__ void __launch_bounds__(256) k_adj_faces(KParams P, int d, const double* __restrict__ U,
-                                                   const double* __restrict__ B, const double* __restrict__ LR,
-                                                   double* __restrict__ LfL, double* __restrict__ LfR,
-                                                   const StepCtl* __restrict__ ctl, unsigned long long* __restrict__ best) {
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    const int nT = d == 0 ? P.nxT : P.nyT, nO = d == 0 ? P.ny : P.nx;
-    const int nf = nT - 2 * P.gc + 1;
-    if (t >= nf * nO) return;
-    // consecutive threads take consecutive i in both directions (coalesced)
-    const int s = d == 0 ? P.gc - 1 + t % nf : P.gc - 1 + t / nO;
-    const int o = d == 0 ? P.gc + t / nf : P.gc + t % nO;
-    const int i = d == 0 ? s : o, j = d == 0 ? o : s;
-    const int i1 = d == 0 ? i + 1 : i, j1 = d == 0 ? j : j + 1;
-    const size_t n = (size_t)P.nxT * P.nyT;
-    const size_t kc = cid(P, i, j), k1 = cid(P, i1, j1);
-    const double inv = d == 0 ? P.inv_dx : P.inv_dy;
-    const bool c_in = s >= P.gc, c1_in = s + 1 < nT - P.gc;
-    double lF[3];
-    for (int v = 0; v < 3; ++v) lF[v] = inv * ((c1_in ? LR[v * n + k1] : 0.0) - (c_in ? LR[v * n + kc] : 0.0));
-    double Lc[3], Rc[3], L1[3], R1[3];
-    recon_at<double>(P, U, B, d, i, j, Lc, Rc);
-    recon_at<double>(P, U, B, d, i1, j1, L1, R1);
-    double gm[3], gq[3], speed;
-    ad::face_vjp(d, Rc, L1, P.phys, lF, gm, gq, speed);
-    for (int a = 0; a < 3; ++a) {
-        LfR[a * n + kc] = gm[a];
-        LfL[a * n + k1] = gq[a];
+// state and (c+1)'s left face state.  The branches of every reconstruction
+// are kept for k_adj_recon: x's byte and y's in the two halves of `picks`.
+//
+// A workgroup is FROWS+1 waves of 64 columns, one row each: every wave
+// reconstructs its row's cells once in each direction, a face takes its left
+// cell's state from the lane to the left, or its lower cell's from the wave
+// below through LDS (so lane 0 and wave 0 only reconstruct).  FP64 issue
+// bounds it: at 512^2 25 us where one launch per direction, each thread
+// reconstructing both cells of its face and each side of a face evaluated
+// twice, took 16 us each.
+constexpr int FROWS = 4, FCOLS = 63;
+__global__ void __launch_bounds__(64 * (FROWS + 1))
+k_adj_faces(KParams P, const double* __restrict__ U, const double* __restrict__ B, const double* __restrict__ LR,
+            double* __restrict__ LfL0, double* __restrict__ LfR0, double* __restrict__ LfL1, double* __restrict__ LfR1,
+            unsigned short* __restrict__ picks, const AdjStep* __restrict__ ctl, unsigned long long* __restrict__ best) {
+    __shared__ double up[FROWS + 1][3][64];          // a row's upper face states
+    const int gc = P.gc, nxT = P.nxT, nyT = P.nyT;
+    const int lane = threadIdx.x & 63;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+    const int ci = gc - 1 + FCOLS * blockIdx.x + lane, cj = gc - 1 + FROWS * blockIdx.y + w;
+    const bool in = ci <= nxT - gc && cj <= nyT - gc;
+    // a lane past the last reconstructed cell takes that cell again (its
+    // stencil lies in the array) and writes nothing
+    const int i = ci <= nxT - gc ? ci : nxT - gc, j = cj <= nyT - gc ? cj : nyT - gc;
+    const size_t n = (size_t)nxT * nyT, k = cid(P, i, j);
+    const bool ix = i >= gc && i < nxT - gc, iy = j >= gc && j < nyT - gc;
+    double c[3], Lx[3], Rx[3], Ly[3], Ry[3];
+    unsigned code;
+    {
+        const double b00 = Bcorner(P, B, i, j), b10 = Bcorner(P, B, i + 1, j), b01 = Bcorner(P, B, i, j + 1),
+                     b11 = Bcorner(P, B, i + 1, j + 1);
+        double l[3], r[3], s[3], t[3];
+#pragma unroll
+        for (int v = 0; v < 3; ++v) {
+            c[v] = U[v * n + k];
+            l[v] = U[v * n + k - 1];
+            r[v] = U[v * n + k + 1];
+            s[v] = U[v * n + k - nxT];
+            t[v] = U[v * n + k + nxT];
+        }
+        code = recon_pick(l, c, r, P.theta, 0.5 * (b00 + b01), 0.5 * (b10 + b11), Lx, Rx);
+        code |= recon_pick(s, c, t, P.theta, 0.5 * (b00 + b10), 0.5 * (b01 + b11), Ly, Ry) << 8;
     }
-    // With best given: the face that set dt.  maximum(wavespeeds) returns the
-    // first interior cell in memory order whose wavespeed, the max of its two
-    // face speeds (numericalflux.jl:29-32), is the step's maximum; a cell's
-    // wavespeed is the maximum exactly when one of its faces' speeds is, so
-    // each face at the maximum offers its interior cells and the smallest
-    // memory index wins.
-    if (best && d == dt_direction(P, ctl) &&
-        (unsigned long long)__double_as_longlong(speed) == slot_wsmax(ctl->slot[0], d)) {
-        unsigned long long c = ~0ull;
-        if (c_in) c = kc;
-        if (c1_in && k1 < c) c = k1;
-        if (c != ~0ull) atomicMin(best, c);
+    if (in && (lane > 0 || blockIdx.x == 0) && (w > 0 || blockIdx.y == 0)) picks[k] = (unsigned short)code;
+#pragma unroll
+    for (int v = 0; v < 3; ++v) up[w][v][lane] = Ry[v];
+    double Rl[3];                                    // the left cell's right face state
+#pragma unroll
+    for (int v = 0; v < 3; ++v) Rl[v] = __shfl_up(Rx[v], 1, 64);
+    __syncthreads();
+    if (w == 0 || !in) return;
+    const int dset = best ? dt_direction(P, ctl) : -1;
+    auto face = [&](int d, const double* m, const double* q, size_t kc, bool c_in, bool c1_in, double* LfL, double* LfR) {
+        const double inv = d == 0 ? P.inv_dx : P.inv_dy;
+        double lF[3];
+#pragma unroll
+        for (int v = 0; v < 3; ++v) lF[v] = inv * ((c1_in ? LR[v * n + k] : 0.0) - (c_in ? LR[v * n + kc] : 0.0));
+        double gm[3], gq[3], speed;
+        ad::face_vjp(d, m, q, P.phys, lF, gm, gq, speed);
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            LfR[a * n + kc] = gm[a];
+            LfL[a * n + k] = gq[a];
+        }
+        // With best given: the face that set dt.  maximum(wavespeeds) returns the
+        // first interior cell in memory order whose wavespeed, the max of its two
+        // face speeds (numericalflux.jl:29-32), is the step's maximum; a cell's
+        // wavespeed is the maximum exactly when one of its faces' speeds is, so
+        // each face at the maximum offers its interior cells and the smallest
+        // memory index wins.
+        if (d == dset && (unsigned long long)__double_as_longlong(speed) == ctl->ws[d]) {
+            unsigned long long f = ~0ull;
+            if (c_in) f = kc;
+            if (c1_in && k < f) f = k;
+            if (f != ~0ull) atomicMin(best, f);
+        }
+    };
+    if (lane > 0 && iy && i >= gc) face(0, Rl, Lx, k - 1, i - 1 >= gc, ix, LfL0, LfR0);
+    if (lane > 0 && ix && j >= gc) {
+        const double Rb[3] = {up[w - 1][0][lane], up[w - 1][1][lane], up[w - 1][2][lane]};
+        face(1, Rb, Ly, k - nxT, j - 1 >= gc, iy, LfL1, LfR1);
     }
 }
 
 // Cell (i,j), direction d: adjoint of the reconstruction (and of the bottom
 // source, source_term_bottom.jl:24-41) gathered from the face-state adjoints
-// of the cell and its two neighbours along d.  Adds it to acc (has: whether
-// the cell takes part in direction d); adds the face bottom adjoints of the
-// cell to LBf (planes: x left, x right, y left, y right).
-__device__ __forceinline__ bool recon_dir(const KParams& P, int d, int i, int j, const double* __restrict__ U,
+// of the cell and its two neighbours along d, with the branches k_adj_faces
+// kept.  Adds it to acc (has: whether the cell takes part in direction d);
+// adds the face bottom adjoints of the cell to LBf (planes: x left, x right,
+// y left, y right).
+template <int d>
+__device__ __forceinline__ bool recon_dir(const KParams& P, int i, int j, const double* __restrict__ U,
                                           const double* __restrict__ B, const double* __restrict__ LR,
                                           const double* __restrict__ LfL, const double* __restrict__ LfR,
-                                          double acc[3], double* __restrict__ LBf) {
+                                          const unsigned short* __restrict__ picks, double acc[3],
+                                          double* __restrict__ LBf) {
     const int s = d == 0 ? i : j, o = d == 0 ? j : i;
     const int nT = d == 0 ? P.nxT : P.nyT, oT = d == 0 ? P.nyT : P.nxT;
     if (o < P.gc || o >= oT - P.gc) return false;
@@ -612,23 +762,11 @@ __device__ __forceinline__ bool recon_dir(const KParams& P, int d, int i, int j,
     const double g = P.phys.g;
     const double Dd = d == 0 ? P.dx : P.dy, inv = d == 0 ? P.inv_dx : P.inv_dy;
     const int pow2 = d == 0 ? P.dx_pow2 : P.dy_pow2;
-    // total adjoint of cell k's face states: flux part + bottom-source part
-    auto face_adj = [&](int kk, int ki, int kj, double aL[3], double aR[3]) {
-        const size_t q = cid(P, ki, kj);
-        for (int v = 0; v < 3; ++v) { aL[v] = LfL[v * n + q]; aR[v] = LfR[v * n + q]; }
-        if (P.bottom && kk >= P.gc && kk < nT - P.gc) {
-            const double slope = slope_div(B_face_right(P, B, ki, kj, d) - B_face_left(P, B, ki, kj, d), Dd, inv, pow2);
-            const double c = LR[(1 + d) * n + q] * (-g * slope) * 0.5;
-            aL[0] += c;
-            aR[0] += c;
-        }
-    };
-    double Lc[3], Rc[3];                              // the cell's own face states
-    int dry_c = 0;
+    double aL0[3], aR0[3];                            // the cell's own face-state adjoints
+    unsigned code0 = 0;
     // Branch-free over the three stencil offsets, so that every load can be
     // issued up front: an offset whose cell lies outside the range where face
-    // states are used is evaluated at a clamped, in-bounds cell (the stencil
-    // of a cell in [gc-1, nT-gc] stays inside the array for gc >= 2) and its
+    // states are used is evaluated at a clamped, in-bounds cell and its
     // contribution is dropped.
 #pragma unroll
     for (int off = -1; off <= 1; ++off) {
@@ -636,34 +774,47 @@ __device__ __forceinline__ bool recon_dir(const KParams& P, int d, int i, int j,
         const bool use = kr >= P.gc - 1 && kr <= nT - P.gc;
         const int kk = kr < P.gc - 1 ? P.gc - 1 : (kr > nT - P.gc ? nT - P.gc : kr);
         const int ki = d == 0 ? kk : i, kj = d == 0 ? j : kk;
+        const size_t q = cid(P, ki, kj);
+        // total adjoint of the cell's face states: flux part + bottom-source part
         double aL[3], aR[3];
-        face_adj(kk, ki, kj, aL, aR);
-        double L[3], R[3];
-        int pick[3], dry;
-        recon_pick(P, U, B, d, ki, kj, L, R, pick, dry);
+#pragma unroll
+        for (int v = 0; v < 3; ++v) { aL[v] = LfL[v * n + q]; aR[v] = LfR[v * n + q]; }
+        if (P.bottom) {
+            const double slope = slope_div(B_face_right(P, B, ki, kj, d) - B_face_left(P, B, ki, kj, d), Dd, inv, pow2);
+            const double c = LR[(1 + d) * n + q] * (-g * slope) * 0.5;
+            if (kk >= P.gc && kk < nT - P.gc) {
+                aL[0] += c;
+                aR[0] += c;
+            }
+        }
+        const unsigned code = (unsigned)picks[q] >> (8 * d);
         const int p = -off;                           // this cell's position in kk's stencil
         const double dc = p == 0 ? 1.0 : 0.0;
+#pragma unroll
         for (int v = 0; v < 3; ++v) {
-            const double cs = slope_coef(pick[v], v == 0 ? dry : 0, p, P.theta);
+            const double cs = slope_coef(code >> (2 * v) & 3u, v == 0 ? code >> 6 & 3u : 0u, p, P.theta);
             const double t = aL[v] * (dc - 0.5 * cs) + aR[v] * (dc + 0.5 * cs);
             if (use) acc[v] += t;
         }
         if (off == 0) {
-            for (int v = 0; v < 3; ++v) { Lc[v] = L[v]; Rc[v] = R[v]; }
-            dry_c = dry;
+#pragma unroll
+            for (int v = 0; v < 3; ++v) { aL0[v] = aL[v]; aR0[v] = aR[v]; }
+            code0 = code;
         }
     }
     const size_t k = cid(P, i, j);
     // the cell's own face bottoms: Bl and Br enter w's face states directly
     // (L_w -= Bl, R_w -= Br) and through the dry-fix line
     if (s >= P.gc - 1 && s <= nT - P.gc) {
-        double aL[3], aR[3];
-        face_adj(s, i, j, aL, aR);
-        const double sbl = dry_c == 1 ? -2.0 : 0.0, sbr = dry_c == 2 ? 2.0 : 0.0;   // d slope_w / d Bl, d Br
-        double lBl = aL[0] * ((0.0 - 0.5 * sbl) - 1.0) + aR[0] * (0.0 + 0.5 * sbl);
-        double lBr = aL[0] * (0.0 - 0.5 * sbr) + aR[0] * ((0.0 + 0.5 * sbr) - 1.0);
+        const unsigned dry = code0 >> 6 & 3u;
+        const double sbl = dry == 1 ? -2.0 : 0.0, sbr = dry == 2 ? 2.0 : 0.0;   // d slope_w / d Bl, d Br
+        double lBl = aL0[0] * ((0.0 - 0.5 * sbl) - 1.0) + aR0[0] * (0.0 + 0.5 * sbl);
+        double lBr = aL0[0] * (0.0 - 0.5 * sbr) + aR0[0] * ((0.0 + 0.5 * sbr) - 1.0);
         if (P.bottom && s >= P.gc && s < nT - P.gc) {   // bottom source: -g ((Br - Bl)/Δ) ((hR + hL)/2)
-            const double c = LR[(1 + d) * n + k] * (-g) * inv * ((Rc[0] + Lc[0]) / 2.0);
+            const size_t st = d == 0 ? 1 : (size_t)P.nxT;
+            const double hsum = depth_sum(U[k - st], U[k], U[k + st], P.theta, B_face_left(P, B, i, j, d),
+                                          B_face_right(P, B, i, j, d), code0);
+            const double c = LR[(1 + d) * n + k] * (-g) * inv * (hsum / 2.0);
             lBr += c;
             lBl -= c;
         }
@@ -675,21 +826,25 @@ __device__ __forceinline__ bool recon_dir(const KParams& P, int d, int i, int j,
 
 // Both directions of the reconstruction adjoint for one cell, one
 // read-modify-write of LU: LU += acc_x, then += acc_y (the x and y face-state
-// adjoints come in their own buffers).
+// adjoints come in their own buffers).  Its 30 planes of traffic bound it: at
+// 512^2 23 us (2.8 TB/s); with the six reconstructions repeated here instead
+// of read as bytes it took 34.
 __global__ void __launch_bounds__(256) k_adj_recon(KParams P, const double* __restrict__ U, const double* __restrict__ B,
                                                    const double* __restrict__ LR, const double* __restrict__ LfL0,
                                                    const double* __restrict__ LfR0, const double* __restrict__ LfL1,
-                                                   const double* __restrict__ LfR1, double* __restrict__ LU,
+                                                   const double* __restrict__ LfR1,
+                                                   const unsigned short* __restrict__ picks, double* __restrict__ LU,
                                                    double* __restrict__ LBf) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     // the launchers' blocks are 64 wide, so a wave shares threadIdx.y
     const int j = __builtin_amdgcn_readfirstlane(blockIdx.y * blockDim.y + threadIdx.y);
     if (i >= P.nxT || j >= P.nyT) return;
     double ax[3] = {0.0, 0.0, 0.0}, ay[3] = {0.0, 0.0, 0.0};
-    const bool hx = recon_dir(P, 0, i, j, U, B, LR, LfL0, LfR0, ax, LBf);
-    const bool hy = recon_dir(P, 1, i, j, U, B, LR, LfL1, LfR1, ay, LBf);
+    const bool hx = recon_dir<0>(P, i, j, U, B, LR, LfL0, LfR0, picks, ax, LBf);
+    const bool hy = recon_dir<1>(P, i, j, U, B, LR, LfL1, LfR1, picks, ay, LBf);
     if (!hx && !hy) return;
     const size_t n = (size_t)P.nxT * P.nyT, k = cid(P, i, j);
+#pragma unroll
     for (int v = 0; v < 3; ++v) {
         double lu = LU[v * n + k];
         if (hx) lu += ax[v];
@@ -706,19 +861,7 @@ __global__ void __launch_bounds__(256) k_adj_recon(KParams P, const double* __re
 // whose wavespeed is the maximum (found by the stage-1 face kernel: best =
 // its memory index), and its right face unless the left one is strictly
 // faster.
-__device__ inline void face_speeds(const KParams& P, const double* U, const double* B, int d, int i, int j, double& sr,
-                                   double& sl) {
-    const int di = d == 0 ? 1 : 0, dj = d == 0 ? 0 : 1;
-    double Lm[3], Rm[3], Ll[3], Rl[3], Lr[3], Rr[3], F[3];
-    recon_at<double>(P, U, B, d, i, j, Lm, Rm);
-    recon_at<double>(P, U, B, d, i - di, j - dj, Ll, Rl);
-    recon_at<double>(P, U, B, d, i + di, j + dj, Lr, Rr);
-    sr = ad::central_upwind<double>(d, Rm, Lr, P.phys, F);
-    sl = ad::central_upwind<double>(d, Rl, Lm, P.phys, F);
-}
-
-
-
+//
 // Once per reverse step, after the stage tails and both
 // directions' face adjoints of stage 1: (1) sum the two stages' block
 // partials of the dt and Cz adjoints in a fixed order (sums[0] = the step's
@@ -726,7 +869,11 @@ __device__ inline void face_speeds(const KParams& P, const double* U, const doub
 // finite positive wave speed must have a face reproducing that speed, else
 // the sticky flag is raised; (3) the dt adjoint goes to the face that set dt
 // (in the face buffers of its direction, d = 0: LfL0/LfR0, d = 1: LfL1/LfR1).
-__global__ void __launch_bounds__(256) k_adj_dtstep(KParams P, const StepCtl* ctl, const double* __restrict__ part_dt,
+//
+// One workgroup, and latency is all of it: the two face speeds and the face's
+// states come from two lanes of the last wave while the sums are under way
+// (10 us; 14 with one thread doing it all after the sums).
+__global__ void __launch_bounds__(256) k_adj_dtstep(KParams P, const AdjStep* ctl, const double* __restrict__ part_dt,
                                                     const double* __restrict__ part_cz, int count,
                                                     double* __restrict__ sums, double* __restrict__ cz_total,
                                                     const unsigned long long* __restrict__ best, int* __restrict__ flag,
@@ -734,44 +881,49 @@ __global__ void __launch_bounds__(256) k_adj_dtstep(KParams P, const StepCtl* ct
                                                     double* __restrict__ LfL0, double* __restrict__ LfR0,
                                                     double* __restrict__ LfL1, double* __restrict__ LfR1) {
     __shared__ double red[2][256];
+    const int tid = threadIdx.x;
+    const unsigned long long kbest = *best;
+    const double ws[2] = {__longlong_as_double((long long)ctl->ws[0]), __longlong_as_double((long long)ctl->ws[1])};
     double a = 0.0, b = 0.0;
-    for (int k = threadIdx.x; k < count; k += blockDim.x) { a += part_dt[k]; b += part_cz[k]; }
-    red[0][threadIdx.x] = a;
-    red[1][threadIdx.x] = b;
+    for (int k = tid; k < count; k += 256) { a += part_dt[k]; b += part_cz[k]; }
+    red[0][tid] = a;
+    red[1][tid] = b;
+    const int d = dt_direction(P, ctl);
+    const double amax = d == 0 ? ws[0] : ws[1];
+    const bool have = kbest < (unsigned long long)P.nxT * P.nyT && amax > 0.0 && __builtin_isfinite(amax);
+    const int di = d == 0 ? 1 : 0, dj = d == 0 ? 0 : 1;
+    int ia = 0, ja = 0;                            // the face lies between (ia,ja) and the next cell
+    double Ra[3] = {0.0, 0.0, 0.0}, Lb[3] = {0.0, 0.0, 0.0};
+    if (have && tid >= 192 && tid < 194) {
+        // lane 0 the cell's right face, lane 1 its left face
+        ia = (int)(kbest % P.nxT) - (tid == 193 ? di : 0);
+        ja = (int)(kbest / P.nxT) - (tid == 193 ? dj : 0);
+        double La[3], Rb[3], F[3];
+        recon_at<double>(P, U, B, d, ia, ja, La, Ra);
+        recon_at<double>(P, U, B, d, ia + di, ja + dj, Lb, Rb);
+        const double mine = ad::central_upwind<double>(d, Ra, Lb, P.phys, F);
+        const double other = __shfl_xor(mine, 1, 64);
+        // jl_max(sr, sl) returns sr unless sl is larger
+        const bool right = tid == 192 ? !(other > mine) : !(mine > other);
+        if (right == (tid == 193)) ia = -1;        // the other lane's face
+    }
     __syncthreads();
     for (int s = 128; s > 0; s >>= 1) {
-        if ((int)threadIdx.x < s) { red[0][threadIdx.x] += red[0][threadIdx.x + s]; red[1][threadIdx.x] += red[1][threadIdx.x + s]; }
+        if (tid < s) { red[0][tid] += red[0][tid + s]; red[1][tid] += red[1][tid + s]; }
         __syncthreads();
     }
-    if (threadIdx.x != 0) return;
     const double ldt = red[0][0];
-    sums[0] = ldt;
-    *cz_total += red[1][0];
-    const unsigned long long kbest = *best;
-    {
-        const double ax = __longlong_as_double((long long)slot_wsmax(ctl->slot[0], 0));
-        const double ay = __longlong_as_double((long long)slot_wsmax(ctl->slot[0], 1));
-        const bool armed = __builtin_isfinite(ax) && __builtin_isfinite(ay) && (ax > 0.0 || ay > 0.0);
+    if (tid == 0) {
+        sums[0] = ldt;
+        *cz_total += red[1][0];
+        const bool armed = __builtin_isfinite(ws[0]) && __builtin_isfinite(ws[1]) && (ws[0] > 0.0 || ws[1] > 0.0);
         if (armed && kbest == ~0ull) *flag = 1;
     }
-    const int d = dt_direction(P, ctl);
-    if (kbest >= (unsigned long long)P.nxT * P.nyT) return;
-    const int i = (int)(kbest % P.nxT), j = (int)(kbest / P.nxT);
-    const double ax = __longlong_as_double((long long)slot_wsmax(ctl->slot[0], d));
-    if (!(ax > 0.0) || !__builtin_isfinite(ax)) return;
-    double sr, sl;
-    face_speeds(P, U, B, d, i, j, sr, sl);
-    const bool right = !(sl > sr);                 // jl_max(sr, sl) returns sr unless sl is larger
-    const int di = d == 0 ? 1 : 0, dj = d == 0 ? 0 : 1;
-    const int ia = right ? i : i - di, ja = right ? j : j - dj;   // the face lies between (ia,ja) and the next cell
-    const int ib = ia + di, jb = ja + dj;
+    if (!have || tid < 192 || tid >= 194 || ia < 0) return;
     const double Dd = d == 0 ? P.dx : P.dy;
     // dt = cfl * Δ_d / a_d on the selected direction: d dt / d a = -cfl Δ / a^2
-    const double lspeed = ldt * P.cfl * (-Dd / (ax * ax));
+    const double lspeed = ldt * P.cfl * (-Dd / (amax * amax));
     const size_t n = (size_t)P.nxT * P.nyT;
-    double La[3], Ra[3], Lb[3], Rb[3];
-    recon_at<double>(P, U, B, d, ia, ja, La, Ra);
-    recon_at<double>(P, U, B, d, ib, jb, Lb, Rb);
     const double lF0[3] = {0.0, 0.0, 0.0};
     double gm[3], gq[3], sp;
     ad::face_vjp(d, Ra, Lb, P.phys, lF0, gm, gq, sp, lspeed);
@@ -779,7 +931,7 @@ __global__ void __launch_bounds__(256) k_adj_dtstep(KParams P, const StepCtl* ct
     double* LfR = d == 0 ? LfR0 : LfR1;
     for (int c = 0; c < 3; ++c) {
         LfR[c * n + cid(P, ia, ja)] += gm[c];
-        LfL[c * n + cid(P, ib, jb)] += gq[c];
+        LfL[c * n + cid(P, ia + di, ja + dj)] += gq[c];
     }
 }
 
@@ -836,14 +988,17 @@ namespace {
 
 using namespace sfv;
 
-// Every buffer starts at zero: the clear is queued on the handle's stream,
+// The small buffers start at zero: the clear is queued on the handle's stream,
 // ahead of every kernel of the call (the side stream's work waits for an
-// event recorded on that stream after the forward pass).
+// event recorded on that stream after the forward pass).  The states and what
+// the steps keep of themselves come from one slab (`clear` false): each is
+// written before it is read, and releasing one large allocation takes as long
+// as releasing each of its parts (270 us on an idle device).
 struct AdjBuffers {
     hipStream_t stream;
     std::vector<void*> owned;
     explicit AdjBuffers(hipStream_t s) : stream(s) {}
-    double* alloc(size_t count, std::string& why, int& rc) {
+    double* alloc(size_t count, std::string& why, int& rc, bool clear = true) {
         void* p = nullptr;
         if (rc) return nullptr;
         if (hipMalloc(&p, count * sizeof(double)) != hipSuccess) {
@@ -852,7 +1007,7 @@ struct AdjBuffers {
             return nullptr;
         }
         owned.push_back(p);
-        if (hipMemsetAsync(p, 0, count * sizeof(double), stream) != hipSuccess) {
+        if (clear && hipMemsetAsync(p, 0, count * sizeof(double), stream) != hipSuccess) {
             rc = SFV_ERR_HIP;
             why = "clearing the adjoint buffers failed";
             return nullptr;
@@ -909,24 +1064,17 @@ int march_step(sfv_handle* h, int slot, const double* U0, double* U2) {
     return SFV_OK;
 }
 
-// One forward step U0 -> U2 (bitwise the fused path), keeping the stage-1
-// state, both right-hand sides at every cell and, in ctl_out, the step's
-// control block as stage 1 leaves it (its dt and wave-speed maxima).  The
-// right-hand sides come from the march stage-1 kernel, which reads the
-// ghost cells the boundary condition filled and writes interior cells; the
-// finishing kernel stores the ghost cells' (sources only) beside them.  The
-// second march launch raises the slot's maxima again, after the copy.
-int forward_step(sfv_handle* h, hipStream_t st, double t, const double* U0, double* U1, double* R1, double* R2,
-                 double* U2, StepCtl* ctl_out) {
+// One forward step U0 -> U2 (bitwise the fused path) in step slot `slot` of a
+// prepared loop, keeping the stage-1 state (ghosts too), both right-hand sides
+// at interior cells and, in keep, the step's control.
+int forward_step(sfv_handle* h, hipStream_t st, int slot, const double* U0, double* U1, double* R1, double* R2,
+                 double* U2, ad::AdjStep* keep) {
     const KParams& P = h->P;
-    ATRY(launch_prepare(st, P, h->ctl, 0, t, NAN, 0, 0, 0.0, 1, 0, SFV_F64));
-    ATRY(launch_stage<double>(st, P, h->ctl, 0, 1, U0, nullptr, R1, h->B));
-    ATRY(launch_finish<double>(st, P, h->ctl, 0, 1, U0, U0, R1, U1, h->B, 1, -1, R1));
-    ATRY(hipMemcpyAsync(ctl_out, h->ctl, sizeof(StepCtl), hipMemcpyDeviceToDevice, st));
-    ATRY(launch_bc<double>(st, P, h->ctl, 0, U1, BC_IN_STEP));
-    ATRY(launch_stage<double>(st, P, h->ctl, 0, 1, U1, nullptr, R2, h->B));
-    ATRY(launch_finish<double>(st, P, h->ctl, 0, 2, U0, U1, R2, U2, h->B, 1, -1, R2));
-    ATRY(launch_bc<double>(st, P, h->ctl, 0, U2, BC_LAST_STAGE));
+    ATRY(launch_stage<double>(st, P, h->ctl, slot, 1, U0, nullptr, R1, h->B, 0, 1));
+    ATRY(launch_stage<double>(st, P, h->ctl, slot, 3, U0, R1, R2, h->B, 0, 1, U1));
+    hipLaunchKernelGGL(ad::k_adj_finish, dim3((P.nxT + 63) / 64, (P.nyT + 3) / 4), dim3(64, 4), 0, st, P, h->ctl, slot,
+                       U0, U1, R2, U2, h->B, keep);
+    ATRY(hipPeekAtLastError());
     return SFV_OK;
 }
 
@@ -953,8 +1101,6 @@ extern "C" int sfv_adjoint(sfv_handle* h, int64_t nsteps, int32_t checkpoint_eve
     std::string why;
     int rc = SFV_OK;
     AdjBuffers buf(st);
-    double* ck = buf.alloc(n3 * (size_t)nseg, why, rc);         // checkpoint states
-    double* seg = buf.alloc(n3 * (size_t)(ce + 1), why, rc);    // the states of one segment
     double* U1 = buf.alloc(n3, why, rc);
     double* R1 = buf.alloc(n3, why, rc);
     double* R2 = buf.alloc(n3, why, rc);
@@ -980,64 +1126,100 @@ extern "C" int sfv_adjoint(sfv_handle* h, int64_t nsteps, int32_t checkpoint_eve
     unsigned long long* best = (unsigned long long*)buf.alloc(1, why, rc);
     double* d_times = buf.alloc((size_t)nsteps + 1, why, rc);
     int* flag = (int*)buf.alloc(1, why, rc);
-    // the control block of the step being recomputed, without kept blocks
-    StepCtl* step_ctl = (StepCtl*)buf.alloc(sizeof(StepCtl) / sizeof(double) + 1, why, rc);
+    unsigned short* picks = (unsigned short*)buf.alloc((n + 3) / 4, why, rc);   // the reconstruction's branches
+    // the control of the step being recomputed, without kept ones
+    ad::AdjStep* step_ctl = (ad::AdjStep*)buf.alloc(sizeof(ad::AdjStep) / sizeof(double), why, rc);
     // The stage-1 states, right-hand sides and step controls of a segment are
     // kept from its recompute when they fit in half the free device memory;
     // otherwise each reverse step recomputes its own.
     size_t free_b = 0, total_b = 0;
-    const size_t keep_bytes = (size_t)ce * (3 * n3 * sizeof(double) + sizeof(StepCtl));
+    const size_t keep_bytes = (size_t)ce * (3 * n3 * sizeof(double) + sizeof(ad::AdjStep));
     const char* keep_env = std::getenv("SFV_ADJOINT_KEEP");      // "0": always recompute
-    const bool keep = !rc && !(keep_env && keep_env[0] == '0') && hipMemGetInfo(&free_b, &total_b) == hipSuccess &&
-                      keep_bytes < free_b / 2;
+    const size_t seg_bytes = n3 * (size_t)(ce + 1) * sizeof(double);
+    const bool known = hipMemGetInfo(&free_b, &total_b) == hipSuccess;
+    free_b -= std::min(free_b, seg_bytes + n3 * (size_t)nseg * sizeof(double));   // checkpoints and one segment
+    const bool keep = !rc && !(keep_env && keep_env[0] == '0') && known && keep_bytes < free_b / 2;
     // When two sets of them (and a second segment of states) fit as well,
     // segment sg-1 is recomputed on a second stream while the reverse steps
     // of segment sg run.
     const char* ovl_env = std::getenv("SFV_ADJOINT_OVERLAP");   // "0": one stream
-    const size_t seg_bytes = n3 * (size_t)(ce + 1) * sizeof(double);
     const bool overlap = keep && nseg > 1 && !(ovl_env && ovl_env[0] == '0') &&
                          2 * keep_bytes + seg_bytes < free_b / 2;
-    const size_t ctl_words = (size_t)ce * (sizeof(StepCtl) / sizeof(double) + 1);
+    const size_t ctl_words = (size_t)ce * (sizeof(ad::AdjStep) / sizeof(double));
     double* kU1s[2] = {nullptr, nullptr};
     double* kR1s[2] = {nullptr, nullptr};
     double* kR2s[2] = {nullptr, nullptr};
-    StepCtl* kctls[2] = {nullptr, nullptr};
-    double* segs[2] = {seg, nullptr};
-    for (int k = 0; k < (overlap ? 2 : keep ? 1 : 0); ++k) {
-        kU1s[k] = buf.alloc(n3 * (size_t)ce, why, rc);
-        kR1s[k] = buf.alloc(n3 * (size_t)ce, why, rc);
-        kR2s[k] = buf.alloc(n3 * (size_t)ce, why, rc);
-        kctls[k] = (StepCtl*)buf.alloc(ctl_words, why, rc);
-    }
-    if (overlap) segs[1] = buf.alloc(n3 * (size_t)(ce + 1), why, rc);
+    ad::AdjStep* kctls[2] = {nullptr, nullptr};
+    double* segs[2] = {nullptr, nullptr};
+    const int sets = overlap ? 2 : keep ? 1 : 0;
+    const size_t slab_words = n3 * (size_t)nseg + (overlap ? 2 : 1) * n3 * (size_t)(ce + 1) +
+                              sets * (3 * n3 * (size_t)ce + ctl_words);
+    double* slab = buf.alloc(slab_words, why, rc, false);
     if (rc) { h->err = why; return rc; }
+    auto take = [&](size_t words) {
+        double* p = slab;
+        slab += words;
+        return p;
+    };
+    double* ck = take(n3 * (size_t)nseg);                        // checkpoint states
+    for (int k = 0; k < (overlap ? 2 : 1); ++k) segs[k] = take(n3 * (size_t)(ce + 1));   // the states of one segment
+    for (int k = 0; k < sets; ++k) {
+        kU1s[k] = take(n3 * (size_t)ce);
+        kR1s[k] = take(n3 * (size_t)ce);
+        kR2s[k] = take(n3 * (size_t)ce);
+        kctls[k] = (ad::AdjStep*)take(ctl_words);
+    }
+    double* seg = segs[0];
     ATRY(hipMemcpyAsync(tgt, h_target, sizeof(double) * P.nx * P.ny, hipMemcpyHostToDevice, st));
 
+    // Step s of segment sg from its state in buffer set `set`, on stream rs: the
+    // next state, and with keep its stage-1 state, right-hand sides and control.
+    auto kept_step = [&](int64_t sg, int set, int64_t s, hipStream_t rs) -> int {
+        const size_t e = (size_t)(s - sg * ce), o = e * n3;
+        double* a = segs[set] + o;
+        return keep ? forward_step(h, rs, (int)(e & 1), a, kU1s[set] + o, kR1s[set] + o, kR2s[set] + o, a + n3,
+                                   kctls[set] + e)
+                    : forward_step(h, rs, (int)(e & 1), a, U1, R1, R2, a + n3, step_ctl);
+    };
     // forward pass with checkpoints, device-resident: one prepared loop of
-    // march steps; each step's end time is copied on the device and the
-    // times come back once
+    // march steps (with keep, the last segment's steps are kept as they run, in
+    // the buffer set its reverse reads); the times at which steps are
+    // recomputed are copied on the device and come back once
     std::vector<double> times((size_t)nsteps + 1);
+    const int last = overlap ? (int)((nseg - 1) & 1) : 0;
     double* cur = (double*)h->U[h->cur & 1];
+    double* UT = seg + (size_t)(nsteps & 1) * n3;
     ATRY(hipMemcpyAsync(seg, cur, n3 * sizeof(double), hipMemcpyDeviceToDevice, st));
     ATRY(launch_prepare(st, P, h->ctl, 0, *t_io, NAN, 0, 0, 0.0, -1, 0, SFV_F64));
     for (int64_t s = 0; s < nsteps; ++s) {
         double* a = seg + (size_t)(s & 1) * n3;
         double* b = seg + (size_t)((s + 1) & 1) * n3;
         if (s % ce == 0) {
-            // a checkpoint restarts the per-pass recompute, which reads ghosts
+            // a recompute's reverse steps read the checkpoint's ghosts
             if (s > 0) ATRY(launch_bc<double>(st, P, h->ctl, 0, a, BC_STANDALONE));
             ATRY(hipMemcpyAsync(ck + (size_t)(s / ce) * n3, a, n3 * sizeof(double), hipMemcpyDeviceToDevice, st));
         }
-        if ((rc = march_step(h, (int)(s & 1), a, b))) return rc;
-        ATRY(hipMemcpyAsync(d_times + s + 1, &h->ctl->t, sizeof(double), hipMemcpyDeviceToDevice, st));
+        if (keep && s / ce == nseg - 1) {
+            if (s % ce == 0) {
+                ATRY(hipMemcpyAsync(segs[last], ck + (size_t)(nseg - 1) * n3, n3 * sizeof(double),
+                                    hipMemcpyDeviceToDevice, st));
+                if (s & 1)      // kept steps take the slots from 0
+                    ATRY(hipMemcpyAsync(&h->ctl->slot[0], &h->ctl->slot[1], sizeof(StepSlot), hipMemcpyDeviceToDevice, st));
+                UT = segs[last] + (size_t)(nsteps - s) * n3;
+            }
+            if ((rc = kept_step(nseg - 1, last, s, st))) return rc;
+        } else {
+            if ((rc = march_step(h, (int)(s & 1), a, b))) return rc;
+            if (!keep || (s + 1) % ce == 0)
+                ATRY(hipMemcpyAsync(d_times + s + 1, &h->ctl->t, sizeof(double), hipMemcpyDeviceToDevice, st));
+        }
     }
     ATRY(hipMemcpyAsync(times.data() + 1, d_times + 1, (size_t)nsteps * sizeof(double), hipMemcpyDeviceToHost, st));
     ATRY(hipMemcpyAsync(h->ctl_host, h->ctl, sizeof(StepCtl), hipMemcpyDeviceToHost, st));
     ATRY(hipStreamSynchronize(st));
     times[0] = *t_io;
-    const double t = times[(size_t)nsteps];
+    const double t = h->ctl_host->t;
     const double last_dt = h->ctl_host->dt;
-    double* UT = seg + (size_t)(nsteps & 1) * n3;
     // the final state, ghosts filled, becomes the handle's state
     if (nsteps > 0) ATRY(launch_bc<double>(st, P, h->ctl, 0, UT, BC_STANDALONE));
     ATRY(hipMemcpyAsync(cur, UT, n3 * sizeof(double), hipMemcpyDeviceToDevice, st));
@@ -1052,10 +1234,8 @@ extern "C" int sfv_adjoint(sfv_handle* h, int64_t nsteps, int32_t checkpoint_eve
     for (double v : pj) J += v;
 
     const int bcx = (P.ny + 255) / 256, bcy = (P.nx + 4 * P.gc * P.gc + 255) / 256;
-    auto faces_grid = [&](int d) {
-        const int nT = d == 0 ? P.nxT : P.nyT, nO = d == 0 ? P.ny : P.nx;
-        return dim3((unsigned)(((nT - 2 * P.gc + 1) * nO + 255) / 256));
-    };
+    // lanes 1..63 and waves 1..FROWS of a workgroup own faces: nx + 1 by ny + 1 of them
+    const dim3 fg((P.nx + ad::FCOLS) / ad::FCOLS, (P.ny + ad::FROWS) / ad::FROWS), fb(64 * (ad::FROWS + 1));
     // Recompute of segment sg from its checkpoint into buffer set `set`, on
     // stream rs: with keep, every step's stage-1 state, right-hand sides and
     // control block are kept; without, only the states.
@@ -1063,17 +1243,10 @@ extern "C" int sfv_adjoint(sfv_handle* h, int64_t nsteps, int32_t checkpoint_eve
         const int64_t s0 = sg * ce, s1 = std::min<int64_t>(nsteps, s0 + ce);
         double* sb = segs[set];
         ATRY(hipMemcpyAsync(sb, ck + (size_t)sg * n3, n3 * sizeof(double), hipMemcpyDeviceToDevice, rs));
+        ATRY(launch_prepare(rs, P, h->ctl, 0, times[(size_t)s0], NAN, 0, 0, 0.0, -1, 0, SFV_F64));
         for (int64_t s = s0; s < (keep ? s1 : s1 - 1); ++s) {
-            double* a = sb + (size_t)(s - s0) * n3;
-            const size_t o = (size_t)(s - s0) * n3;
-            int r;
-            if (keep) {
-                if ((r = forward_step(h, rs, times[(size_t)s], a, kU1s[set] + o, kR1s[set] + o, kR2s[set] + o,
-                                      a + n3, kctls[set] + (s - s0))))
-                    return r;
-            } else if ((r = forward_step(h, rs, times[(size_t)s], a, U1, R1, R2, a + n3, step_ctl))) {
-                return r;
-            }
+            const int r = kept_step(sg, set, s, rs);
+            if (r) return r;
         }
         return SFV_OK;
     };
@@ -1084,14 +1257,15 @@ extern "C" int sfv_adjoint(sfv_handle* h, int64_t nsteps, int32_t checkpoint_eve
             const size_t o = (size_t)(s - s0) * n3;
             const double* U0 = segs[set] + o;
             const double *u1 = U1, *r1 = R1, *r2 = R2;
-            const StepCtl* cs = step_ctl;               // the step's control block (its dt and maxima)
+            const ad::AdjStep* cs = step_ctl;           // the step's control (its dt and maxima)
             if (keep) {
                 u1 = kU1s[set] + o;
                 r1 = kR1s[set] + o;
                 r2 = kR2s[set] + o;
                 cs = kctls[set] + (s - s0);
             } else {
-                const int r = forward_step(h, st, times[(size_t)s], U0, U1, R1, R2, Ut, step_ctl);
+                ATRY(launch_prepare(st, P, h->ctl, 0, times[(size_t)s], NAN, 0, 0, 0.0, -1, 0, SFV_F64));
+                const int r = forward_step(h, st, 0, U0, U1, R1, R2, Ut, step_ctl);
                 if (r) return r;
             }
             // stage 2: U2 = clamp(friction(0.5 (U0 + U1 + dt R2))); the tail
@@ -1099,23 +1273,17 @@ extern "C" int sfv_adjoint(sfv_handle* h, int64_t nsteps, int32_t checkpoint_eve
             // Lnew afresh
             hipLaunchKernelGGL(ad::k_adj_tail, cg, cb, 0, st, P, cs, 2, U0, u1, r2, h->B, L, L1, Lnew, LR, LBc,
                                part_dt, part_cz, best);
-            hipLaunchKernelGGL(ad::k_adj_faces, faces_grid(0), dim3(256), 0, st, P, 0, u1, h->B, LR, LfL, LfR, cs,
-                               nullptr);
-            hipLaunchKernelGGL(ad::k_adj_faces, faces_grid(1), dim3(256), 0, st, P, 1, u1, h->B, LR, LfL1, LfR1, cs,
-                               nullptr);
-            hipLaunchKernelGGL(ad::k_adj_recon, cg, cb, 0, st, P, u1, h->B, LR, LfL, LfR, LfL1, LfR1, L1, LBf);
+            hipLaunchKernelGGL(ad::k_adj_faces, fg, fb, 0, st, P, u1, h->B, LR, LfL, LfR, LfL1, LfR1, picks, cs, nullptr);
+            hipLaunchKernelGGL(ad::k_adj_recon, cg, cb, 0, st, P, u1, h->B, LR, LfL, LfR, LfL1, LfR1, picks, L1, LBf);
             // stage 1: U1 = clamp(friction(U0 + dt R1))
             hipLaunchKernelGGL(ad::k_adj_tail, cg, cb, 0, st, P, cs, 1, U0, U0, r1, h->B, L1, Lnew, nullptr, LR,
                                LBc, part_dt, part_cz, best);
             // stage 1's faces also find the face that set dt, as the
             // reference's maximum(ws) would
-            hipLaunchKernelGGL(ad::k_adj_faces, faces_grid(0), dim3(256), 0, st, P, 0, U0, h->B, LR, LfL, LfR, cs,
-                               best);
-            hipLaunchKernelGGL(ad::k_adj_faces, faces_grid(1), dim3(256), 0, st, P, 1, U0, h->B, LR, LfL1, LfR1, cs,
-                               best);
+            hipLaunchKernelGGL(ad::k_adj_faces, fg, fb, 0, st, P, U0, h->B, LR, LfL, LfR, LfL1, LfR1, picks, cs, best);
             hipLaunchKernelGGL(ad::k_adj_dtstep, dim3(1), dim3(256), 0, st, P, cs, part_dt, part_cz, 2 * nblk,
                                sums, sums + 1, best, flag, U0, h->B, LfL, LfR, LfL1, LfR1);
-            hipLaunchKernelGGL(ad::k_adj_recon, cg, cb, 0, st, P, U0, h->B, LR, LfL, LfR, LfL1, LfR1, Lnew, LBf);
+            hipLaunchKernelGGL(ad::k_adj_recon, cg, cb, 0, st, P, U0, h->B, LR, LfL, LfR, LfL1, LfR1, picks, Lnew, LBf);
             ATRY(hipPeekAtLastError());
             std::swap(L, Lnew);
         }
@@ -1130,12 +1298,9 @@ extern "C" int sfv_adjoint(sfv_handle* h, int64_t nsteps, int32_t checkpoint_eve
         ATRY(hipEventRecord(side.fwd, st));
         ATRY(hipStreamWaitEvent(side.s, side.fwd, 0));
         bool used[2] = {false, false};
-        const int last = (int)((nseg - 1) & 1);
-        if ((rc = recompute(nseg - 1, last, side.s))) return rc;
-        ATRY(hipEventRecord(side.ready[last], side.s));
         for (int64_t sg = nseg - 1; sg >= 0; --sg) {
             const int set = (int)(sg & 1), other = 1 - set;
-            ATRY(hipStreamWaitEvent(st, side.ready[set], 0));
+            if (sg < nseg - 1) ATRY(hipStreamWaitEvent(st, side.ready[set], 0));
             if (sg > 0) {
                 if (used[other]) ATRY(hipStreamWaitEvent(side.s, side.done[other], 0));
                 if ((rc = recompute(sg - 1, other, side.s))) return rc;
@@ -1147,7 +1312,7 @@ extern "C" int sfv_adjoint(sfv_handle* h, int64_t nsteps, int32_t checkpoint_eve
         }
     } else {
         for (int64_t sg = nseg - 1; sg >= 0; --sg) {
-            if ((rc = recompute(sg, 0, st))) return rc;
+            if ((!keep || sg < nseg - 1) && (rc = recompute(sg, 0, st))) return rc;
             if ((rc = reverse(sg, 0))) return rc;
         }
     }

@@ -10,7 +10,7 @@ template <class S>
 __global__ void k_flux(KParams P, StepCtl* ctl, int slot, const S* X, S* RHS, const double* B, int record);
 template <class S>
 __global__ void k_finish(KParams P, StepCtl* ctl, int slot, int stage, const S* U0, const S* X, const S* RHS, S* Out,
-                         const double* B, int rhs_interior, int next, S* ghost_rhs);
+                         const double* B, int rhs_interior, int next);
 
 // ---- boundary condition and step control (swe_kernels_ctl.hip)
 template <class S>
@@ -29,7 +29,7 @@ hipError_t launch_flux(hipStream_t st, const KParams& P, StepCtl* ctl, int slot,
 template <class S>
 hipError_t launch_finish(hipStream_t st, const KParams& P, StepCtl* ctl, int slot, int stage, const S* U0, const S* X,
                          const S* RHS, S* Out, const double* B,
-                         int rhs_interior = 0, int next = -1, S* ghost_rhs = nullptr);
+                         int rhs_interior = 0, int next = -1);
 template <class S>
 hipError_t launch_bc(hipStream_t st, const KParams& P, StepCtl* ctl, int slot, S* U, int mode);
 hipError_t launch_prepare(hipStream_t st, const KParams& P, StepCtl* ctl, int slot, double t, double endtime,
@@ -83,7 +83,8 @@ hipError_t launch_interior_copy(hipStream_t st, const KParams& P, const void* pa
 // stage = 3 (ForwardEuler): finishes the step of `slot` from U0 and RHS1 into
 // UO (interior and domain corners), as stage 2's input, closes it into the
 // next of the three slots, and writes the next step's right-hand side to OUT
-// and its wave speeds to that slot.  Where a ghost's source is a ghost
+// and its wave speeds to that slot; close = 0: the step stays open, the
+// right-hand side of UO is taken at its time and no speeds are raised.  Where a ghost's source is a ghost
 // (KParams::ghost_self), it writes the high-side ghosts of UO too; this
 // needs gc = 2.
 template <class S>

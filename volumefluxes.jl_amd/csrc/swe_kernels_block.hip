@@ -85,10 +85,10 @@ __device__ __forceinline__ void block_tile(const KParams& P, StepCtl* ctl, int s
         dt_d = wave_uniform(stage1_dt<S>(P, ctl, sl));
         dt_s = (S)dt_d;
     }
-    // the source rates of the right-hand side: this step's, in STAGE 3 the
-    // next one's (close_step gives its slot the same values)
-    StepRates nrates;
-    if (STAGE == 3) {
+    // the source rates of the right-hand side: this step's, where STAGE 3 closes
+    // the step the next one's (close_step gives its slot the same values)
+    StepRates nrates = {sl.t, sl.rain_now, sl.infil_tfac};
+    if (STAGE == 3 && close) {
         set_rates<MODE != 0>(P, nrates, (double)(S)((S)sl.t + dt_s));
         nrates.rain_now = wave_uniform(nrates.rain_now);
         nrates.infil_tfac = wave_uniform(nrates.infil_tfac);
@@ -288,7 +288,7 @@ __device__ __forceinline__ void block_tile(const KParams& P, StepCtl* ctl, int s
             else finish(std::false_type{});
         }
     }
-    if (STAGE != 2) {
+    if (STAGE == 1 || (STAGE == 3 && close)) {
         smx = wave_max_u64(face_x_ok ? smx : 0ull);
         smy = wave_max_u64(out_col ? smy : 0ull);
         if (lane == 0) { sm.red[w][0] = smx; sm.red[w][1] = smy; }
@@ -306,7 +306,7 @@ __device__ __forceinline__ void block_tile(const KParams& P, StepCtl* ctl, int s
         if (lane == 0) {
             ctl->dt = (double)dt_s;
             ctl->dt_stage1 = dt_d;
-            if (STAGE == 3) close_step<S, MODE != 0>(P, ctl, slot, rslot, next_of_three(rslot));
+            if (STAGE == 3 && close) close_step<S, MODE != 0>(P, ctl, slot, rslot, next_of_three(rslot));
             else if (close) close_step<S, MODE != 0>(P, ctl, slot);
         }
         finish_corners<S, MODE != 0, STAGE == 3>(P, sl, U0, STAGE == 3 ? UO : OUT, B, dt_d, dt_s, lane, BL);

@@ -171,7 +171,7 @@ __device__ __forceinline__ void march_tile(const KParams& P, StepCtl* ctl, int s
     const int gc = P.gc, nxT = P.nxT, nyT = P.nyT;
     const int j0 = gc + seg * my;
     if (j0 >= nyT - gc) {                          // whole wave: past the grid
-        if (STAGE != 2) block_max_to_slot_m(0ull, 0ull, &ctl->slot[rslot], par);
+        if (STAGE == 1 || (STAGE == 3 && close)) block_max_to_slot_m(0ull, 0ull, &ctl->slot[rslot], par);
         return;
     }
     const int th = min(my, nyT - gc - j0);
@@ -188,10 +188,10 @@ __device__ __forceinline__ void march_tile(const KParams& P, StepCtl* ctl, int s
         dt_d = wave_uniform(stage1_dt<S>(P, ctl, sl));
         dt_s = (S)dt_d;
     }
-    // the source rates of the right-hand side: this step's, in STAGE 3 the
-    // next one's (close_step gives its slot the same values)
-    StepRates nrates;
-    if (STAGE == 3) {
+    // the source rates of the right-hand side: this step's, where STAGE 3 closes
+    // the step the next one's (close_step gives its slot the same values)
+    StepRates nrates = {sl.t, sl.rain_now, sl.infil_tfac};
+    if (STAGE == 3 && close) {
         set_rates<MODE != 0>(P, nrates, (double)(S)((S)sl.t + dt_s));
         nrates.rain_now = wave_uniform(nrates.rain_now);
         nrates.infil_tfac = wave_uniform(nrates.infil_tfac);
@@ -423,7 +423,7 @@ __device__ __forceinline__ void march_tile(const KParams& P, StepCtl* ctl, int s
         s1 = s0;
         s0 = free;
     }
-    if (STAGE != 2) {
+    if (STAGE == 1 || (STAGE == 3 && close)) {
         // x faces this lane evaluated (its left face) that border an output cell
         const bool face_x_ok = in_dom && lane >= 2 && lane <= MX + 2 && (lane == 2 ? i < nxT - gc : i - 1 < nxT - gc);
         block_max_to_slot_m(face_x_ok ? smx : 0ull, out_col ? smy : 0ull, &ctl->slot[rslot], par);
@@ -436,7 +436,7 @@ __device__ __forceinline__ void march_tile(const KParams& P, StepCtl* ctl, int s
         if (lane == 0) {
             ctl->dt = (double)dt_s;
             ctl->dt_stage1 = dt_d;
-            if (STAGE == 3) {
+            if (STAGE == 3 && close) {
                 close_step<S, MODE != 0>(P, ctl, slot, rslot, next_of_three(rslot));
             } else if (close) {
                 if (BATCH) close_step_call<S, MODE != 0>(P, ctl, slot);

@@ -16,7 +16,7 @@
 // sources, R2 = L(U1) + sources, dt and maximum speeds when they fit (on a
 // second stream, overlapped with the previous segment's reverse steps, when
 // two sets fit), then walks it backwards.  A kept step is three launches:
-// stage 1 (R1), stage 3 (U1 and R2) and k_adj_finish (U2 and the ghosts); at
+// stage 1 (R1), stage 4 (U1 and R2) and k_adj_finish (U2 and the ghosts); at
 // 512^2 f64 they take 43 us where the per-pass chain of eight took 75.  Per stage in reverse order a reverse step applies the
 // boundary-condition fold (read as a gather), dry clamp, implicit friction
 // and the RK combination, then the face fluxes of both directions (the
@@ -1071,7 +1071,7 @@ int forward_step(sfv_handle* h, hipStream_t st, int slot, const double* U0, doub
                  double* U2, ad::AdjStep* keep) {
     const KParams& P = h->P;
     ATRY(launch_stage<double>(st, P, h->ctl, slot, 1, U0, nullptr, R1, h->B, 0, 1));
-    ATRY(launch_stage<double>(st, P, h->ctl, slot, 3, U0, R1, R2, h->B, 0, 1, U1));
+    ATRY(launch_stage<double>(st, P, h->ctl, slot, 4, U0, R1, R2, h->B, 0, 1, U1));
     hipLaunchKernelGGL(ad::k_adj_finish, dim3((P.nxT + 63) / 64, (P.nyT + 3) / 4), dim3(64, 4), 0, st, P, h->ctl, slot,
                        U0, U1, R2, U2, h->B, keep);
     ATRY(hipPeekAtLastError());

@@ -83,10 +83,10 @@ hipError_t launch_interior_copy(hipStream_t st, const KParams& P, const void* pa
 // stage = 3 (ForwardEuler): finishes the step of `slot` from U0 and RHS1 into
 // UO (interior and domain corners), as stage 2's input, closes it into the
 // next of the three slots, and writes the next step's right-hand side to OUT
-// and its wave speeds to that slot; close = 0: the step stays open, the
-// right-hand side of UO is taken at its time and no speeds are raised.  Where a ghost's source is a ghost
+// and its wave speeds to that slot.  Where a ghost's source is a ghost
 // (KParams::ghost_self), it writes the high-side ghosts of UO too; this
-// needs gc = 2.
+// needs gc = 2.  stage = 4: as stage 3, but the step stays open: the
+// right-hand side of UO is taken at its time and no speeds are raised.
 template <class S>
 hipError_t launch_march(hipStream_t st, const KParams& P, StepCtl* ctl, int slot, int stage, const S* U0,
                         const S* RHS1, S* OUT, const double* B, int close = 0, int remap_halo = 0, S* UO = nullptr);

@@ -85,10 +85,10 @@ __device__ __forceinline__ void block_tile(const KParams& P, StepCtl* ctl, int s
         dt_d = wave_uniform(stage1_dt<S>(P, ctl, sl));
         dt_s = (S)dt_d;
     }
-    // the source rates of the right-hand side: this step's, where STAGE 3 closes
-    // the step the next one's (close_step gives its slot the same values)
-    StepRates nrates = {sl.t, sl.rain_now, sl.infil_tfac};
-    if (STAGE == 3 && close) {
+    // the source rates of the right-hand side: this step's, in STAGE 3 the
+    // next one's (close_step gives its slot the same values)
+    StepRates nrates;
+    if (STAGE == 3) {
         set_rates<MODE != 0>(P, nrates, (double)(S)((S)sl.t + dt_s));
         nrates.rain_now = wave_uniform(nrates.rain_now);
         nrates.infil_tfac = wave_uniform(nrates.infil_tfac);
@@ -197,11 +197,6 @@ __device__ __forceinline__ void block_tile(const KParams& P, StepCtl* ctl, int s
             for (int v = 0; v < 3; ++v) sm.ry[s][v][lane] = Ry[v];
             sm.ry[s][3][lane] = Ly[0];
             if (fin) {
-                if (STAGE == 2) {                  // U0 of row p, for the RK combination
-                    const size_t ro = (size_t)nxT * (r - 2);
-#pragma unroll
-                    for (int v = 0; v < 3; ++v) x0[v] = row_ld(U0 + v * n + ro, nxT, i);
-                }
                 S Lx[3], Rx[3], Rxl[3];
                 const double Blx = 0.5 * (bp + bm), Brx = 0.5 * (np + nm);
                 bcp = bc4(bp, np, bm, nm);
@@ -223,7 +218,7 @@ __device__ __forceinline__ void block_tile(const KParams& P, StepCtl* ctl, int s
                     for (int v = 0; v < 3; ++v) Rxl[v] = shfl_up1(Rx[v]);
                     const double spx = RNG ? central_upwind_rng<0, MODE != 0>(Rxl, Lx, P.phys, K, Fxm)
                                            : central_upwind(0, Rxl, Lx, P.phys, Fxm);
-                    if (STAGE != 2) raise_speed<RNG>(smx, (double)(S)spx);
+                    if (STAGE == 1 || STAGE == 3) raise_speed<RNG>(smx, (double)(S)spx);
 #pragma unroll
                     for (int v = 0; v < 3; ++v)
                         accx[v] = (S)__builtin_fma(-P.inv_dx, shfl_dn1(Fxm[v]) - Fxm[v], 0.0);   // 0 - inv*diff
@@ -245,14 +240,19 @@ __device__ __forceinline__ void block_tile(const KParams& P, StepCtl* ctl, int s
             const S Rlow[3] = {Ryp[0], Ryp[1], Ryp[2]};
             if (band) {
                 const double spy = central_upwind_rng<1, MODE != 0>(Rlow, Ly, P.phys, K, Fy);
-                if (STAGE != 2) raise_speed<true>(smy, (double)(S)spy);
+                if (STAGE == 1 || STAGE == 3) raise_speed<true>(smy, (double)(S)spy);
             } else {
                 const double spy = central_upwind(1, Rlow, Ly, P.phys, Fy);
-                if (STAGE != 2) raise_speed<false>(smy, (double)(S)spy);
+                if (STAGE == 1 || STAGE == 3) raise_speed<false>(smy, (double)(S)spy);
             }
             const int t = y_slot<BW>(w, par);
 #pragma unroll
             for (int v = 0; v < 3; ++v) sm.fy[t][v][lane] = Fy[v];
+            if (STAGE == 2 && fin) {               // U0 of row p, for the RK combination
+                const size_t ro = (size_t)nxT * (r - 2);
+#pragma unroll
+                for (int v = 0; v < 3; ++v) x0[v] = row_ld(U0 + v * n + ro, nxT, i);
+            }
         }
         __syncthreads();
         // ---- 4. finish row p
@@ -272,7 +272,7 @@ __device__ __forceinline__ void block_tile(const KParams& P, StepCtl* ctl, int s
                 if (STAGE != 2) {
 #pragma unroll
                     for (int v = 0; v < 3; ++v) row_st(orow + v * n, nxT, i, acc[v]);
-                    if (STAGE == 3) {              // the new state
+                    if (STAGE >= 3) {              // the new state
                         S* urow = UO + (size_t)nxT * p;
 #pragma unroll
                         for (int v = 0; v < 3; ++v) row_st(urow + v * n, nxT, i, cA[v]);
@@ -288,7 +288,7 @@ __device__ __forceinline__ void block_tile(const KParams& P, StepCtl* ctl, int s
             else finish(std::false_type{});
         }
     }
-    if (STAGE == 1 || (STAGE == 3 && close)) {
+    if (STAGE == 1 || STAGE == 3) {
         smx = wave_max_u64(face_x_ok ? smx : 0ull);
         smy = wave_max_u64(out_col ? smy : 0ull);
         if (lane == 0) { sm.red[w][0] = smx; sm.red[w][1] = smy; }
@@ -306,10 +306,10 @@ __device__ __forceinline__ void block_tile(const KParams& P, StepCtl* ctl, int s
         if (lane == 0) {
             ctl->dt = (double)dt_s;
             ctl->dt_stage1 = dt_d;
-            if (STAGE == 3 && close) close_step<S, MODE != 0>(P, ctl, slot, rslot, next_of_three(rslot));
+            if (STAGE == 3) close_step<S, MODE != 0>(P, ctl, slot, rslot, next_of_three(rslot));
             else if (close) close_step<S, MODE != 0>(P, ctl, slot);
         }
-        finish_corners<S, MODE != 0, STAGE == 3>(P, sl, U0, STAGE == 3 ? UO : OUT, B, dt_d, dt_s, lane, BL);
+        finish_corners<S, MODE != 0, (STAGE >= 3)>(P, sl, U0, STAGE >= 3 ? UO : OUT, B, dt_d, dt_s, lane, BL);
     }
 }
 
@@ -375,7 +375,7 @@ hipError_t launch_block(hipStream_t st, const KParams& P, StepCtl* ctl, int slot
     const int strips = (P.nx + BCOLS - 1) / BCOLS, segs = (P.ny + H - 1) / H;
     by_waves(H, [&](auto waves) {
         constexpr int BW = decltype(waves)::value;
-        by_stage_mode<3>(stage, stage == 3 && P.ghost_self ? MODE_GENERAL : march_mode(P), [&](auto stg, auto mode) {
+        by_stage_mode<4>(stage, stage == 3 && P.ghost_self ? MODE_GENERAL : march_mode(P), [&](auto stg, auto mode) {
             hipLaunchKernelGGL((k_block<S, decltype(stg)::value, decltype(mode)::value, BW>), dim3(strips * segs),
                                dim3(BL * BW), 0, st, P, ctl, slot, H, strips, segs, U0, RHS1, OUT, UO, B, remap_halo,
                                close);

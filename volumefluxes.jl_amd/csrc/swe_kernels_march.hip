@@ -171,7 +171,7 @@ __device__ __forceinline__ void march_tile(const KParams& P, StepCtl* ctl, int s
     const int gc = P.gc, nxT = P.nxT, nyT = P.nyT;
     const int j0 = gc + seg * my;
     if (j0 >= nyT - gc) {                          // whole wave: past the grid
-        if (STAGE == 1 || (STAGE == 3 && close)) block_max_to_slot_m(0ull, 0ull, &ctl->slot[rslot], par);
+        if (STAGE == 1 || STAGE == 3) block_max_to_slot_m(0ull, 0ull, &ctl->slot[rslot], par);
         return;
     }
     const int th = min(my, nyT - gc - j0);
@@ -188,10 +188,10 @@ __device__ __forceinline__ void march_tile(const KParams& P, StepCtl* ctl, int s
         dt_d = wave_uniform(stage1_dt<S>(P, ctl, sl));
         dt_s = (S)dt_d;
     }
-    // the source rates of the right-hand side: this step's, where STAGE 3 closes
-    // the step the next one's (close_step gives its slot the same values)
-    StepRates nrates = {sl.t, sl.rain_now, sl.infil_tfac};
-    if (STAGE == 3 && close) {
+    // the source rates of the right-hand side: this step's, in STAGE 3 the
+    // next one's (close_step gives its slot the same values)
+    StepRates nrates;
+    if (STAGE == 3) {
         set_rates<MODE != 0>(P, nrates, (double)(S)((S)sl.t + dt_s));
         nrates.rain_now = wave_uniform(nrates.rain_now);
         nrates.infil_tfac = wave_uniform(nrates.infil_tfac);
@@ -345,7 +345,7 @@ __device__ __forceinline__ void march_tile(const KParams& P, StepCtl* ctl, int s
                 double Fy[3], Fyp[3];
                 const double spy = RNG ? central_upwind_rng<1, MODE != 0>(Ryp, Ly, P.phys, K, Fy)
                                        : central_upwind(1, Ryp, Ly, P.phys, Fy);
-                if (STAGE != 2) raise_speed<RNG>(smy, (double)(S)spy);
+                if (STAGE == 1 || STAGE == 3) raise_speed<RNG>(smy, (double)(S)spy);
 #pragma unroll
                 for (int v = 0; v < 3; ++v) { Fyp[v] = win.fy[v][lane]; win.fy[v][lane] = Fy[v]; }
                 // finish row p = jr-2: y part on top of its x part, then sources
@@ -362,7 +362,7 @@ __device__ __forceinline__ void march_tile(const KParams& P, StepCtl* ctl, int s
                     if (STAGE != 2) {
 #pragma unroll
                         for (int v = 0; v < 3; ++v) row_st(orow + v * n, nxT, i, acc[v]);
-                        if (STAGE == 3) {                          // the new state, from the window
+                        if (STAGE >= 3) {                          // the new state, from the window
                             S* urow = UO + (size_t)nxT * p;
 #pragma unroll
                             for (int v = 0; v < 3; ++v) row_st(urow + v * n, nxT, i, ua[v * MW]);
@@ -399,7 +399,7 @@ __device__ __forceinline__ void march_tile(const KParams& P, StepCtl* ctl, int s
                     double Fxm[3];
                     const double spx = RNG ? central_upwind_rng<0, MODE != 0>(Rxl, Lx, P.phys, K, Fxm)
                                            : central_upwind(0, Rxl, Lx, P.phys, Fxm);
-                    if (STAGE != 2) raise_speed<RNG>(smx, (double)(S)spx);
+                    if (STAGE == 1 || STAGE == 3) raise_speed<RNG>(smx, (double)(S)spx);
                     S ax[3];
 #pragma unroll
                     for (int v = 0; v < 3; ++v)
@@ -423,7 +423,7 @@ __device__ __forceinline__ void march_tile(const KParams& P, StepCtl* ctl, int s
         s1 = s0;
         s0 = free;
     }
-    if (STAGE == 1 || (STAGE == 3 && close)) {
+    if (STAGE == 1 || STAGE == 3) {
         // x faces this lane evaluated (its left face) that border an output cell
         const bool face_x_ok = in_dom && lane >= 2 && lane <= MX + 2 && (lane == 2 ? i < nxT - gc : i - 1 < nxT - gc);
         block_max_to_slot_m(face_x_ok ? smx : 0ull, out_col ? smy : 0ull, &ctl->slot[rslot], par);
@@ -436,14 +436,14 @@ __device__ __forceinline__ void march_tile(const KParams& P, StepCtl* ctl, int s
         if (lane == 0) {
             ctl->dt = (double)dt_s;
             ctl->dt_stage1 = dt_d;
-            if (STAGE == 3 && close) {
+            if (STAGE == 3) {
                 close_step<S, MODE != 0>(P, ctl, slot, rslot, next_of_three(rslot));
             } else if (close) {
                 if (BATCH) close_step_call<S, MODE != 0>(P, ctl, slot);
                 else close_step<S, MODE != 0>(P, ctl, slot);
             }
         }
-        finish_corners<S, MODE != 0, STAGE == 3>(P, sl, U0, STAGE == 3 ? UO : OUT, B, dt_d, dt_s, lane, MW);
+        finish_corners<S, MODE != 0, (STAGE >= 3)>(P, sl, U0, STAGE >= 3 ? UO : OUT, B, dt_d, dt_s, lane, MW);
     }
 }
 
@@ -607,7 +607,7 @@ hipError_t launch_march(hipStream_t st, const KParams& P, StepCtl* ctl, int slot
     const int my = P.rows > 0 ? P.rows : march_rows_per_wave(P, stage, std::is_same<S, float>::value ? 1 : 0);
     const int segs = (P.ny + my - 1) / my;
     const int strips = (P.nx + MX - 1) / MX;
-    by_stage_mode<3>(stage, stage == 3 && P.ghost_self ? MODE_GENERAL : march_mode(P), [&](auto stg, auto mode) {
+    by_stage_mode<4>(stage, stage == 3 && P.ghost_self ? MODE_GENERAL : march_mode(P), [&](auto stg, auto mode) {
         hipLaunchKernelGGL((k_march<S, decltype(stg)::value, decltype(mode)::value>), dim3(march_blocks(strips, segs)),
                            dim3(MW * MWAVES), 0, st, P, ctl, slot, my, strips, segs, U0, RHS1, OUT, UO, B, close,
                            remap_halo);

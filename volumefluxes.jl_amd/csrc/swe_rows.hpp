@@ -355,8 +355,10 @@ inline void by_stage_mode(int stage, int mode, F&& go) {
         else go(st, std::integral_constant<int, MODE_GENERAL>{});
     };
     if (stage == 1) return with(std::integral_constant<int, 1>{});
-    if constexpr (STAGES == 3)
+    if constexpr (STAGES == 4) {
         if (stage == 3) return with(std::integral_constant<int, 3>{});
+        if (stage == 4) return with(std::integral_constant<int, 4>{});
+    }
     with(std::integral_constant<int, 2>{});
 }
 

@@ -607,15 +607,14 @@ int sfv_get_state(sfv_handle* h, void* U, int32_t layout) {
     const size_t es = h->elem;
     const void* src = h->U[h->cur];
     if (layout == SFV_LAYOUT_FULL) {
-        HIP_TRY(h, hipMemcpyAsync(U, src, 3 * h->ncell * es, hipMemcpyDeviceToHost, h->stream));
+        HIP_TRY(h, copy_to_host(U, src, 3 * h->ncell * es, h->stream));
     } else if (layout == SFV_LAYOUT_INTERIOR) {
         // device gather into the right-hand-side buffer, one contiguous download
         HIP_TRY(h, launch_interior_copy(h->stream, P, h->RHS, const_cast<void*>(src), es, 0));
-        HIP_TRY(h, hipMemcpyAsync(U, h->RHS, 3 * (size_t)P.nx * P.ny * es, hipMemcpyDeviceToHost, h->stream));
+        HIP_TRY(h, copy_to_host(U, h->RHS, 3 * (size_t)P.nx * P.ny * es, h->stream));
     } else {
         return fail(h, SFV_ERR_ARGUMENT, "unknown layout");
     }
-    HIP_TRY(h, hipStreamSynchronize(h->stream));
     return SFV_OK;
 }
 

@@ -12,6 +12,7 @@
 
 #include "../../include/sinfvm_hip.h"
 #include "sfv_pool.hpp"
+#include "sfv_transfer.hpp"
 #include "swe_kernels.hpp"
 
 namespace sfv {
@@ -109,6 +110,7 @@ struct sfv_handle {
     bool rows_forced = false;           // set by sfv_set_march_rows
     bool variant_forced = false;        // set by sfv_set_fused: the tuner keeps the variant
     std::string err;
+    bool staging = false;               // holds the process's staging memory (sfv_transfer.hpp)
     // Owner-supplied pool (server handles): device blocks (class-rounded),
     // the stream and the pinned mirror come from it and go back to it.
     sfv::DevicePool* pool = nullptr;
@@ -152,6 +154,8 @@ struct sfv_handle {
 
     int init(const sfv_config& c, std::string& why) {
         cfg = c;
+        if (!staging) sfv::staging_retain();
+        staging = true;
         if (c.rain == SFV_RAIN_TIME_TABLE) {
             rain_rates.assign(c.rain_table_rates, c.rain_table_rates + c.rain_table_len);
             rain_times.assign(c.rain_table_times, c.rain_table_times + c.rain_table_len);
@@ -266,6 +270,7 @@ struct sfv_handle {
 
     ~sfv_handle() {
         if (stream) (void)hipStreamSynchronize(stream);
+        if (staging) sfv::staging_release();
         if (pool) {
             for (auto& b : pooled) pool->put(b.first, b.second);
             if (ctl_host) pool->put_pinned(ctl_host);

@@ -1,0 +1,190 @@
+// sfv_transfer.hip — device-to-host copies into pageable memory.
+//
+// hipMemcpy to pageable memory runs at 18 GB/s where the destination's pages
+// are mapped and at 4.4 GB/s where they are fresh (a new array's pages are
+// mapped one fault at a time), against 57 GB/s into pinned memory.  A copy
+// here goes through a ring of pinned slots: the calling thread queues the DMA
+// of the next chunks while worker threads empty the slots that have arrived,
+// so the copies and page faults of several threads overlap with the DMA.
+// Measured, us for the plain copy and this one: 4 MB mapped 251 and 180, fresh
+// 943 and 400; 36 MB 2080 and 1000, fresh 8500 and 2250; 100 MB 5920 and 2630,
+// fresh 23700 and 5140.
+//
+// The slots belong to a lane, one lane per copy under way.  At most MAX_LANES
+// lanes exist in the process (64 MB); they are made on first use, kept while
+// any handle lives and freed with the last one.  A copy that finds none free
+// is a plain one, as is one below MIN_STAGED: a 64x48 state (85 KB) took 20 us
+// longer through a slot.
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <atomic>
+#include <cstring>
+#include <mutex>
+#include <thread>
+
+#include "sfv_transfer.hpp"
+
+namespace sfv {
+namespace {
+
+constexpr int SLOTS = 8, MAX_LANES = 4, MAX_WORKERS = 8;
+constexpr size_t SLOT_BYTES = (size_t)2 << 20, MIN_CHUNK = (size_t)256 << 10;
+constexpr size_t MIN_STAGED = (size_t)2 << 20;
+
+struct Lane {
+    int device = -1;                    // -1: not made yet
+    bool busy = false;
+    char* slot[SLOTS] = {};             // pinned, allocated as copies need them
+    hipEvent_t arrived[SLOTS] = {};
+    // the first `count` slots exist after this; false if memory is short
+    bool reserve(int count) {
+        for (int k = 0; k < count; ++k) {
+            if (!slot[k] && hipHostMalloc((void**)&slot[k], SLOT_BYTES, hipHostMallocDefault) != hipSuccess) {
+                slot[k] = nullptr;
+                (void)hipGetLastError();
+                return false;
+            }
+            if (!arrived[k] && hipEventCreateWithFlags(&arrived[k], hipEventDisableTiming) != hipSuccess) {
+                arrived[k] = nullptr;
+                (void)hipGetLastError();
+                return false;
+            }
+        }
+        return true;
+    }
+    void release() {
+        for (int k = 0; k < SLOTS; ++k) {
+            if (slot[k]) (void)hipHostFree(slot[k]);
+            if (arrived[k]) (void)hipEventDestroy(arrived[k]);
+            slot[k] = nullptr;
+            arrived[k] = nullptr;
+        }
+        device = -1;
+    }
+};
+
+std::mutex g_mu;
+Lane g_lanes[MAX_LANES];
+int g_users = 0;
+
+// A free lane of this device (an event serves its own device's streams only),
+// or nullptr.
+Lane* take_lane(int device) {
+    std::lock_guard<std::mutex> lk(g_mu);
+    for (Lane& l : g_lanes)
+        if (!l.busy && l.device == device) {
+            l.busy = true;
+            return &l;
+        }
+    for (Lane& l : g_lanes)
+        if (!l.busy && l.device < 0) {
+            l.busy = true;
+            l.device = device;
+            return &l;
+        }
+    return nullptr;
+}
+void give_lane(Lane* l) {
+    std::lock_guard<std::mutex> lk(g_mu);
+    l->busy = false;
+}
+
+hipError_t plain(void* dst, const void* src, size_t n, hipStream_t st) {
+    const hipError_t e = hipMemcpyAsync(dst, src, n, hipMemcpyDeviceToHost, st);
+    const hipError_t s = hipStreamSynchronize(st);
+    return e != hipSuccess ? e : s;
+}
+
+// Chunk c travels through slot c mod SLOTS.  `arrived` counts the chunks whose
+// DMA has completed, emptied[s] those copied out of slot s.
+hipError_t staged(Lane& L, char* dst, const char* src, size_t n, hipStream_t st, size_t chunk, int want) {
+    const long chunks = (long)((n + chunk - 1) / chunk);
+    std::atomic<long> arrived{0}, next{0};
+    std::atomic<bool> stop{false};
+    std::atomic<long> emptied[SLOTS];
+    for (auto& e : emptied) e.store(0);
+    auto bytes = [&](long c) { return std::min(chunk, n - (size_t)c * chunk); };
+    auto empty_slot = [&](long c) {
+        std::memcpy(dst + (size_t)c * chunk, L.slot[c % SLOTS], bytes(c));
+        emptied[c % SLOTS].store(c / SLOTS + 1, std::memory_order_release);
+    };
+    auto work = [&] {
+        for (;;) {
+            const long c = next.fetch_add(1);
+            if (c >= chunks) return;
+            while (arrived.load(std::memory_order_acquire) <= c) {
+                if (stop.load()) return;
+                std::this_thread::yield();
+            }
+            empty_slot(c);
+        }
+    };
+    auto slot_free = [&](long c) { return emptied[c % SLOTS].load(std::memory_order_acquire) >= c / SLOTS; };
+    hipError_t e = hipSuccess;
+    long queued = 0;
+    auto queue = [&] {
+        const int s = (int)(queued % SLOTS);
+        e = hipMemcpyAsync(L.slot[s], src + (size_t)queued * chunk, bytes(queued), hipMemcpyDeviceToHost, st);
+        if (e == hipSuccess) e = hipEventRecord(L.arrived[s], st);
+        ++queued;
+    };
+    while (e == hipSuccess && queued < chunks && queued < SLOTS) queue();
+    std::thread workers[MAX_WORKERS];
+    int running = 0;
+    try {
+        for (; e == hipSuccess && running < want; ++running) workers[running] = std::thread(work);
+    } catch (...) {                     // no more threads: those there are, or this one, do it
+    }
+    for (long c = 0; c < chunks && e == hipSuccess; ++c) {
+        e = hipEventSynchronize(L.arrived[c % SLOTS]);
+        if (e != hipSuccess) break;
+        if (running) arrived.store(c + 1, std::memory_order_release);
+        else empty_slot(c);
+        while (e == hipSuccess && queued < chunks && slot_free(queued)) queue();
+        // nothing under way: the next chunk's slot must be emptied first
+        while (e == hipSuccess && queued == c + 1 && queued < chunks) {
+            if (slot_free(queued)) queue();
+            else std::this_thread::yield();
+        }
+    }
+    if (e != hipSuccess) {
+        stop.store(true);
+        (void)hipStreamSynchronize(st);  // no DMA into a slot outlives the copy
+    }
+    for (int k = 0; k < running; ++k) workers[k].join();
+    return e;
+}
+
+}  // namespace
+
+void staging_retain() {
+    std::lock_guard<std::mutex> lk(g_mu);
+    ++g_users;
+}
+void staging_release() {
+    std::lock_guard<std::mutex> lk(g_mu);
+    if (--g_users > 0) return;
+    for (Lane& l : g_lanes)
+        if (!l.busy) l.release();
+}
+
+hipError_t copy_to_host(void* dst, const void* src, size_t n, hipStream_t st) {
+    int device = 0;
+    if (n < MIN_STAGED || hipGetDevice(&device) != hipSuccess) return plain(dst, src, n, st);
+    Lane* lane = take_lane(device);
+    if (!lane) return plain(dst, src, n, st);
+    // eight chunks, each from MIN_CHUNK up to a slot
+    const size_t chunk = std::min(SLOT_BYTES, std::max(MIN_CHUNK, (n + SLOTS - 1) / SLOTS));
+    const long chunks = (long)((n + chunk - 1) / chunk);
+    const int cpus = std::max(1, (int)std::thread::hardware_concurrency());
+    // a worker for every slot's worth: starting one takes 15 us, copying 2 MB 200
+    const int want = (int)std::min({(long)(n / SLOT_BYTES), (long)MAX_WORKERS, (long)std::max(1, cpus / 2)});
+    hipError_t e;
+    if (lane->reserve((int)std::min(chunks, (long)SLOTS))) e = staged(*lane, (char*)dst, (const char*)src, n, st, chunk, want);
+    else e = plain(dst, src, n, st);
+    give_lane(lane);
+    return e;
+}
+
+}  // namespace sfv

@@ -1,0 +1,19 @@
+// sfv_transfer.hpp — device-to-host copies into pageable memory
+// (sfv_transfer.hip).
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include <cstddef>
+
+namespace sfv {
+
+// Copy n bytes from the current device to dst after the work queued on st;
+// returns when they are there.  Any number of threads may copy at once.
+hipError_t copy_to_host(void* dst, const void* src, size_t n, hipStream_t st);
+
+// Each handle holds the staging memory; it is freed with the last of them.
+void staging_retain();
+void staging_release();
+
+}  // namespace sfv

@@ -222,22 +222,23 @@ bool BatchEngine::finished(int slot) const {
 // per SIMD (the default if none does).  Heights set with sfv_set_march_rows
 // are kept.  No height changes any result.  The online tuner (set_autotune)
 // times this choice against its neighbours.
+long BatchEngine::wave_segments(int r) const {
+    long w = 0;
+    for (int s : rows_) {
+        const sfv_handle* h = slot_handle_[s];
+        const int rr = h->rows_forced ? h->march_rows : std::min(r, h->P.ny);
+        w += (long)((h->P.nx + MARCH_COLS - 1) / MARCH_COLS) * ((h->P.ny + rr - 1) / rr);
+    }
+    return w;
+}
+
 int BatchEngine::rule_rows() const {
     const int R0 = SFV_BATCH_DEFAULT_ROWS;
     const long slots = (long)blocks_stage_ * MARCH_WAVES, simds = 4L * cus_;
-    auto waves = [&](int r) {
-        long w = 0;
-        for (int s : rows_) {
-            const sfv_handle* h = slot_handle_[s];
-            const int rr = h->rows_forced ? h->march_rows : std::min(r, h->P.ny);
-            w += (long)((h->P.nx + MARCH_COLS - 1) / MARCH_COLS) * ((h->P.ny + rr - 1) / rr);
-        }
-        return w;
-    };
     int r = R0;
-    if (waves(R0) < slots)
+    if (wave_segments(R0) < slots)
         for (int c : {1, 2, 3, 4, 6, 8})
-            if (waves(c) <= simds) { r = c; break; }
+            if (wave_segments(c) <= simds) { r = c; break; }
     return r;
 }
 
@@ -272,7 +273,11 @@ std::vector<long long> BatchEngine::signature() const {
 
 // After a membership change: reuse the kept choice for the same member sizes,
 // else line up the timed trials: the rule's height, the next lower and the
-// three next higher candidates, the rule's height again.
+// two next higher candidates, the least height at which the batch's segments
+// fit the resident wave slots in one round (in place of a third higher
+// candidate; 16 grids of 128 to 1024 squared: 55.8 ms a run at 20 rows, 59.2 at
+// 12, whose one and a half rounds leave half the slots idle at the end), the
+// rule's height again.
 void BatchEngine::plan_tuning() {
     trials_.clear();
     trial_ms_.clear();
@@ -293,7 +298,10 @@ void BatchEngine::plan_tuning() {
     if (i0 > 0) trials_.push_back(C[i0 - 1]);
     if (i0 < n - 1) trials_.push_back(C[i0 + 1]);
     if (i0 < n - 2) trials_.push_back(C[i0 + 2]);
-    if (i0 < n - 3) trials_.push_back(C[i0 + 3]);
+    int fit = r0;
+    while (fit < C[n - 1] && wave_segments(fit) > (long)blocks_stage_ * MARCH_WAVES) ++fit;
+    if (fit == r0 && i0 < n - 3) fit = C[i0 + 3];
+    if (std::find(trials_.begin(), trials_.end(), fit) == trials_.end()) trials_.push_back(fit);
     trials_.push_back(r0);
     trial_ms_.assign(trials_.size(), 0.f);
     rows_override_ = trials_[0];

@@ -98,6 +98,7 @@ private:
     int grow(int capacity, std::string& why);
     int upload_table(std::string& why);
     void choose_rows();
+    long wave_segments(int rows) const;    // of all members at this height
     int rule_rows() const;
     void plan_tuning();
     std::vector<long long> signature() const;

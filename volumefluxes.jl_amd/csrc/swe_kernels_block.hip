@@ -56,18 +56,13 @@ template <class S, int STAGE, int MODE, int BW>
 __device__ __forceinline__ void block_tile(const KParams& P, StepCtl* ctl, int slot, int H, int strip, int seg,
                                            const S* __restrict__ U0, const S* __restrict__ RHS1,
                                            S* __restrict__ OUT, S* __restrict__ UO, const double* __restrict__ B,
-                                           BlockSmem<S, BW>& sm,
-                                           int serial, int remap, int close) {
+                                           BlockSmem<S, BW>& sm, int serial, int remap) {
     const StepSlot& sl = ctl->slot[slot];
     // the slot of the step whose speeds are found here
     const int rslot = STAGE == 3 ? next_of_three(slot) : slot;
     const int lane = threadIdx.x & (BL - 1);
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / BL);
-    const bool first = strip == 0 && seg == 0;
-    if (!sl.active) {                              // the same for the whole workgroup
-        if (STAGE >= 2 && close && first && threadIdx.x == 0) ctl->slot[STAGE == 3 ? rslot : 1 - slot].active = 0;
-        return;
-    }
+    if (!sl.active) return;                        // the same for the whole workgroup
     const int gc = P.gc, nxT = P.nxT, nyT = P.nyT;
     const int j0 = gc + seg * H;
     const int th = min(H, nyT - gc - j0);          // >= 1: the launch has no empty segments
@@ -302,15 +297,6 @@ __device__ __forceinline__ void block_tile(const KParams& P, StepCtl* ctl, int s
             raise_wsmax(&ctl->slot[rslot], smx, smy);
         }
     }
-    if (STAGE >= 2 && first && w == 0) {
-        if (lane == 0) {
-            ctl->dt = (double)dt_s;
-            ctl->dt_stage1 = dt_d;
-            if (STAGE == 3) close_step<S, MODE != 0>(P, ctl, slot, rslot, next_of_three(rslot));
-            else if (close) close_step<S, MODE != 0>(P, ctl, slot);
-        }
-        finish_corners<S, MODE != 0, (STAGE >= 3)>(P, sl, U0, STAGE >= 3 ? UO : OUT, B, dt_d, dt_s, lane, BL);
-    }
 }
 
 // Grid of strips x segs workgroups in XCD-contiguous order, strips fastest.
@@ -320,14 +306,20 @@ k_block(KParams P, StepCtl* ctl, int slot, int H, int strips, int segs, const S*
         const S* __restrict__ RHS1, S* __restrict__ OUT, S* __restrict__ UO, const double* __restrict__ B, int remap,
         int close) {
     __shared__ BlockSmem<S, BW> sm;
+    // stages 2 to 4: the last block closes, the others are tiles
+    if (STAGE >= 2 && (int)blockIdx.x == strips * segs) {
+        if (threadIdx.x < BL) close_stage<S, STAGE, MODE != 0>(P, ctl, slot, U0, STAGE >= 3 ? UO : OUT, B, close);
+        return;
+    }
     if (threadIdx.x == 0) sm.bad = 0;
     __syncthreads();
     const int t = xcd_tile(blockIdx.x, strips * segs);
-    block_tile<S, STAGE, MODE, BW>(P, ctl, slot, H, t % strips, t / strips, U0, RHS1, OUT, UO, B, sm, 1, remap, close);
+    block_tile<S, STAGE, MODE, BW>(P, ctl, slot, H, t % strips, t / strips, U0, RHS1, OUT, UO, B, sm, 1, remap);
 }
 
-// Rows per workgroup: the smallest height at which every workgroup has a CU
-// of its own (0: the strips alone are more than the CUs).
+// Rows per workgroup: the smallest height at which every workgroup, the
+// closing one of stages 2 to 4 included, has a CU of its own (0: the strips
+// alone are more than the CUs).
 static int block_height(const KParams& P) {
     static int cus = 0;
     static std::once_flag once;
@@ -339,7 +331,7 @@ static int block_height(const KParams& P) {
         if (cus <= 0) cus = 256;
     });
     const int strips = (P.nx + BCOLS - 1) / BCOLS;
-    return strips > cus ? 0 : (P.ny + cus / strips - 1) / (cus / strips);
+    return strips >= cus ? 0 : (P.ny + (cus - 1) / strips - 1) / ((cus - 1) / strips);
 }
 
 // These kernels against the wave-march kernels, us per step (f64, same box):
@@ -376,7 +368,7 @@ hipError_t launch_block(hipStream_t st, const KParams& P, StepCtl* ctl, int slot
     by_waves(H, [&](auto waves) {
         constexpr int BW = decltype(waves)::value;
         by_stage_mode<4>(stage, stage == 3 && P.ghost_self ? MODE_GENERAL : march_mode(P), [&](auto stg, auto mode) {
-            hipLaunchKernelGGL((k_block<S, decltype(stg)::value, decltype(mode)::value, BW>), dim3(strips * segs),
+            hipLaunchKernelGGL((k_block<S, decltype(stg)::value, decltype(mode)::value, BW>), dim3(strips * segs + (decltype(stg)::value >= 2 ? 1 : 0)),
                                dim3(BL * BW), 0, st, P, ctl, slot, H, strips, segs, U0, RHS1, OUT, UO, B, remap_halo,
                                close);
         });

@@ -163,9 +163,8 @@ __device__ __forceinline__ void march_tile(const KParams& P, StepCtl* ctl, int s
     const int lane = threadIdx.x & (MW - 1);
     if (!sl.active) {                              // the same for every wave of the block
         // an inactive step passes inactivity on, so steps launched past the
-        // end of a run stay no-ops
-        if (STAGE >= 2 && close && strip == 0 && seg == 0 && lane == 0)
-            ctl->slot[STAGE == 3 ? next_of_three(slot) : 1 - slot].active = 0;
+        // end of a run stay no-ops (close_stage in a launch of one grid)
+        if (BATCH && STAGE == 2 && close && strip == 0 && seg == 0 && lane == 0) ctl->slot[1 - slot].active = 0;
         return;
     }
     const int gc = P.gc, nxT = P.nxT, nyT = P.nyT;
@@ -429,21 +428,16 @@ __device__ __forceinline__ void march_tile(const KParams& P, StepCtl* ctl, int s
         block_max_to_slot_m(face_x_ok ? smx : 0ull, out_col ? smy : 0ull, &ctl->slot[rslot], par);
     }
 
-    // dt for the host and the step's closing (t += dt, next slot armed), by
-    // one lane: the other waves read only this step's slot, and the next
-    // slot is read only by the next launches.
-    if (STAGE >= 2 && strip == 0 && seg == 0) {
+    // a batch member's dt for the host and its step's closing (t += dt, next
+    // slot armed), by one lane: the other waves read only this step's slot, and
+    // the next slot is read only by the next launches
+    if (BATCH && STAGE == 2 && strip == 0 && seg == 0) {
         if (lane == 0) {
             ctl->dt = (double)dt_s;
             ctl->dt_stage1 = dt_d;
-            if (STAGE == 3) {
-                close_step<S, MODE != 0>(P, ctl, slot, rslot, next_of_three(rslot));
-            } else if (close) {
-                if (BATCH) close_step_call<S, MODE != 0>(P, ctl, slot);
-                else close_step<S, MODE != 0>(P, ctl, slot);
-            }
+            if (close) close_step_call<S, MODE != 0>(P, ctl, slot);
         }
-        finish_corners<S, MODE != 0, (STAGE >= 3)>(P, sl, U0, STAGE >= 3 ? UO : OUT, B, dt_d, dt_s, lane, MW);
+        finish_corners<S, MODE != 0, false>(P, sl, U0, OUT, B, dt_d, dt_s, lane, MW);
     }
 }
 
@@ -457,6 +451,11 @@ __attribute__((amdgpu_waves_per_eu(SFV_MARCH_MIN_WAVES)))
 k_march(KParams P, StepCtl* ctl, int slot, int my, int strips, int segs, const S* __restrict__ U0,
         const S* __restrict__ RHS1, S* __restrict__ OUT, S* __restrict__ UO, const double* __restrict__ B, int close,
         int remap) {
+    // stages 2 to 4: the last block closes, the others are tiles
+    if (STAGE >= 2 && (int)blockIdx.x == march_blocks(strips, segs)) {
+        if (threadIdx.x < MW) close_stage<S, STAGE, MODE != 0>(P, ctl, slot, U0, STAGE >= 3 ? UO : OUT, B, close);
+        return;
+    }
     const int t = xcd_tile(blockIdx.x, march_blocks(strips, segs));
     // the same for every lane of the wave; readfirstlane tells the compiler so
 #if SFV_MARCH_LINEAR
@@ -608,7 +607,7 @@ hipError_t launch_march(hipStream_t st, const KParams& P, StepCtl* ctl, int slot
     const int segs = (P.ny + my - 1) / my;
     const int strips = (P.nx + MX - 1) / MX;
     by_stage_mode<4>(stage, stage == 3 && P.ghost_self ? MODE_GENERAL : march_mode(P), [&](auto stg, auto mode) {
-        hipLaunchKernelGGL((k_march<S, decltype(stg)::value, decltype(mode)::value>), dim3(march_blocks(strips, segs)),
+        hipLaunchKernelGGL((k_march<S, decltype(stg)::value, decltype(mode)::value>), dim3(march_blocks(strips, segs) + (decltype(stg)::value >= 2 ? 1 : 0)),
                            dim3(MW * MWAVES), 0, st, P, ctl, slot, my, strips, segs, U0, RHS1, OUT, UO, B, close,
                            remap_halo);
     });

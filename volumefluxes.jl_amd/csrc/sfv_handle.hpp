@@ -98,7 +98,7 @@ struct sfv_handle {
     double* d_factor = nullptr;        // Horton factor field
     double* d_rain_field = nullptr;    // FunctionalRain rates per cell
     sfv::StepCtl* ctl = nullptr;       // device step-control block
-    sfv::StepCtl* ctl_host = nullptr;  // pinned mirror
+    sfv::StepCtl* ctl_host = nullptr;  // pinned mirror, and behind it what steps report
     int64_t cur = 0;                   // index of the current state buffer
     int64_t step_parity = 0;           // parity of the next step's slot
     int64_t device_bytes = 0;
@@ -135,6 +135,9 @@ struct sfv_handle {
         device_bytes += (int64_t)bytes;
         return SFV_OK;
     }
+
+    static constexpr size_t MIRROR_BYTES = sizeof(sfv::StepCtl) + sizeof(sfv::StepReport);
+    sfv::StepReport* report() const { return (sfv::StepReport*)(ctl_host + 1); }
 
     // Device bytes init() allocates for a configuration (ctl block included;
     // the per-pass scratch state U[2] is not: it is allocated on first use),
@@ -180,11 +183,11 @@ struct sfv_handle {
         if ((rc = alloc(&RHS, 3 * ncell * elem, why))) return rc;
         if ((rc = alloc((void**)&B, (size_t)(nxT + 1) * (nyT + 1) * sizeof(double), why))) return rc;
         if ((rc = alloc((void**)&ctl, sizeof(sfv::StepCtl), why))) return rc;
-        if (pool) ctl_host = (sfv::StepCtl*)pool->get_pinned(sizeof(sfv::StepCtl));
-        else if (hipHostMalloc((void**)&ctl_host, sizeof(sfv::StepCtl), hipHostMallocDefault) != hipSuccess)
+        if (pool) ctl_host = (sfv::StepCtl*)pool->get_pinned(MIRROR_BYTES);
+        else if (hipHostMalloc((void**)&ctl_host, MIRROR_BYTES, hipHostMallocDefault) != hipSuccess)
             ctl_host = nullptr;
         if (!ctl_host) { why = "hipHostMalloc failed"; return SFV_ERR_OUT_OF_MEMORY; }
-        std::memset(ctl_host, 0, sizeof(sfv::StepCtl));
+        std::memset((void*)ctl_host, 0, MIRROR_BYTES);
         for (int s = 0; s < 2; ++s) (void)hipMemsetAsync(U[s], 0, 3 * ncell * elem, stream);
         (void)hipMemsetAsync(RHS, 0, 3 * ncell * elem, stream);
         (void)hipMemsetAsync(B, 0, (size_t)(nxT + 1) * (nyT + 1) * sizeof(double), stream);

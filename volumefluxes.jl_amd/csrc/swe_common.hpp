@@ -74,6 +74,13 @@ struct StepSlot : StepRates {
     alignas(128) unsigned long long ws[WS_LINES][16];   // [line][0]: x, [line][1]: y
 };
 
+// What the device reports to the host while a loop runs, in pinned host memory
+// the host polls.
+struct StepReport {
+    unsigned long long word;   // 2 * steps + (the run goes on)
+    double t, dt;              // of a finished single step, stored before the word
+};
+
 struct StepCtl {
     StepSlot slot[3];
     double t;             // current time (realtype value)
@@ -87,6 +94,7 @@ struct StepCtl {
     int64_t max_steps;    // <= 0: unlimited
     int32_t nonfinite;    // a step produced a NaN/Inf dt
     int32_t precision;
+    StepReport* report;   // where closing steps report their number (or NULL)
 };
 
 // One member of a batch as the batched kernels see it (a device array of
@@ -263,6 +271,9 @@ __device__ inline void close_step(const KParams& P, StepCtl* c, int slot, int ne
     clear_wsmax(c->slot[clear]);
     c->slot[next].active = act ? 1 : 0;
     set_rates<NO_HORTON>(P, c->slot[next], (double)t);
+    if (c->report)
+        __hip_atomic_store(&c->report->word, 2ull * (unsigned long long)c->steps + (act ? 1 : 0), __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_SYSTEM);
 }
 template <class S, bool NO_HORTON = false>
 __device__ inline void close_step(const KParams& P, StepCtl* c, int slot) {

@@ -14,10 +14,10 @@ __global__ void k_finish(KParams P, StepCtl* ctl, int slot, int stage, const S* 
 
 // ---- boundary condition and step control (swe_kernels_ctl.hip)
 template <class S>
-__global__ void k_bc(KParams P, StepCtl* ctl, int slot, S* U, int mode);
+__global__ void k_bc(KParams P, StepCtl* ctl, int slot, S* U, int mode, StepReport* report);
 __global__ void k_prepare(KParams P, StepCtl* ctl, int slot, double t, double endtime, int match_endtime,
                           int has_max_timestep, double max_timestep, long long max_steps, int until_endtime,
-                          int precision);
+                          int precision, StepReport* report);
 
 // ---- host launchers (one per kernel, defined beside it); each returns the
 // launch status.  BC modes: 0 inside a step, 1 last stage of a step (closes
@@ -31,10 +31,11 @@ hipError_t launch_finish(hipStream_t st, const KParams& P, StepCtl* ctl, int slo
                          const S* RHS, S* Out, const double* B,
                          int rhs_interior = 0, int next = -1);
 template <class S>
-hipError_t launch_bc(hipStream_t st, const KParams& P, StepCtl* ctl, int slot, S* U, int mode);
+hipError_t launch_bc(hipStream_t st, const KParams& P, StepCtl* ctl, int slot, S* U, int mode,
+                     StepReport* report = nullptr);   // report: BC_STANDALONE after a closed step
 hipError_t launch_prepare(hipStream_t st, const KParams& P, StepCtl* ctl, int slot, double t, double endtime,
                           int match_endtime, int has_max_timestep, double max_timestep, long long max_steps,
-                          int until_endtime, int precision);
+                          int until_endtime, int precision, StepReport* report = nullptr);
 // Batched kernels over a device member table (BatchMember[hdr->members]).
 // Stage kernels are persistent: `blocks` workgroups walk the batch's tiles.
 // mode: the lowest march_mode of the members.

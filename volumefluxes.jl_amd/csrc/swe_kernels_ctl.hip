@@ -58,7 +58,16 @@ __device__ __forceinline__ void bc_line(const KParams& P, StepCtl* ctl, int slot
 }
 
 template <class S>
-__global__ void __launch_bounds__(256) k_bc(KParams P, StepCtl* ctl, int slot, S* __restrict__ U, int mode) {
+__global__ void __launch_bounds__(256) k_bc(KParams P, StepCtl* ctl, int slot, S* __restrict__ U, int mode,
+                                            StepReport* report) {
+    // the launches before this one are done: a single step's time and dt can go
+    // to the host while the ghosts are filled
+    if (report && blockIdx.x == 0 && threadIdx.x == 0) {
+        __hip_atomic_store(&report->t, ctl->t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        __hip_atomic_store(&report->dt, ctl->dt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        __hip_atomic_store(&report->word, 2ull * (unsigned long long)ctl->steps, __ATOMIC_RELEASE,
+                           __HIP_MEMORY_SCOPE_SYSTEM);
+    }
     bc_line<S>(P, ctl, slot, U, mode, blockIdx.x * blockDim.x + threadIdx.x);
 }
 
@@ -66,8 +75,9 @@ __global__ void __launch_bounds__(256) k_bc(KParams P, StepCtl* ctl, int slot, S
 // a fixed number of steps (endtime is then NaN and never ends the loop).
 __device__ void prepare_ctl(const KParams& P, StepCtl* c, int slot, double t, double endtime, int match_endtime,
                             int has_max_timestep, double max_timestep, long long max_steps, int until_endtime,
-                            int precision) {
+                            int precision, StepReport* report) {
     c->t = t;
+    c->report = report;
     c->endtime = until_endtime ? endtime : __builtin_nan("");
     c->match_endtime = match_endtime;
     c->has_max_timestep = has_max_timestep;
@@ -88,10 +98,10 @@ __device__ void prepare_ctl(const KParams& P, StepCtl* c, int slot, double t, do
 
 __global__ void k_prepare(KParams P, StepCtl* ctl, int slot, double t, double endtime, int match_endtime,
                           int has_max_timestep, double max_timestep, long long max_steps, int until_endtime,
-                          int precision) {
+                          int precision, StepReport* report) {
     if (threadIdx.x != 0 || blockIdx.x != 0) return;
     prepare_ctl(P, ctl, slot, t, endtime, match_endtime, has_max_timestep, max_timestep, max_steps, until_endtime,
-                precision);
+                precision, report);
 }
 
 // Batched prepare: one thread per member, with the member's run parameters.
@@ -100,7 +110,7 @@ __global__ void k_prepare_batch(const BatchMember* __restrict__ mem, const Batch
     if (m >= hdr->members) return;
     const BatchMember& M = mem[m];
     prepare_ctl(M.P, M.ctl, M.slot0 & 1, M.t0, M.endtime, M.match_endtime, M.has_max_timestep, M.max_timestep,
-                M.max_steps, M.until_endtime, M.precision);
+                M.max_steps, M.until_endtime, M.precision, nullptr);
 }
 
 hipError_t launch_prepare_batch(hipStream_t st, const BatchMember* mem, const BatchHeader* hdr, int members) {
@@ -109,16 +119,16 @@ hipError_t launch_prepare_batch(hipStream_t st, const BatchMember* mem, const Ba
 }
 
 template <class S>
-hipError_t launch_bc(hipStream_t st, const KParams& P, StepCtl* ctl, int slot, S* U, int mode) {
+hipError_t launch_bc(hipStream_t st, const KParams& P, StepCtl* ctl, int slot, S* U, int mode, StepReport* report) {
     const int nthreads = P.nx + P.ny;
-    hipLaunchKernelGGL(k_bc<S>, dim3((nthreads + 255) / 256), dim3(256), 0, st, P, ctl, slot, U, mode);
+    hipLaunchKernelGGL(k_bc<S>, dim3((nthreads + 255) / 256), dim3(256), 0, st, P, ctl, slot, U, mode, report);
     return hipPeekAtLastError();
 }
 hipError_t launch_prepare(hipStream_t st, const KParams& P, StepCtl* ctl, int slot, double t, double endtime,
                           int match_endtime, int has_max_timestep, double max_timestep, long long max_steps,
-                          int until_endtime, int precision) {
+                          int until_endtime, int precision, StepReport* report) {
     hipLaunchKernelGGL(k_prepare, dim3(1), dim3(64), 0, st, P, ctl, slot, t, endtime, match_endtime, has_max_timestep,
-                       max_timestep, max_steps, until_endtime, precision);
+                       max_timestep, max_steps, until_endtime, precision, report);
     return hipPeekAtLastError();
 }
 // A plain device copy of `words` 4-byte words (16 bytes per thread and
@@ -176,7 +186,7 @@ hipError_t launch_interior_copy(hipStream_t st, const KParams& P, const void* pa
     return hipPeekAtLastError();
 }
 
-template hipError_t launch_bc<double>(hipStream_t, const KParams&, StepCtl*, int, double*, int);
-template hipError_t launch_bc<float>(hipStream_t, const KParams&, StepCtl*, int, float*, int);
+template hipError_t launch_bc<double>(hipStream_t, const KParams&, StepCtl*, int, double*, int, StepReport*);
+template hipError_t launch_bc<float>(hipStream_t, const KParams&, StepCtl*, int, float*, int, StepReport*);
 
 }  // namespace sfv

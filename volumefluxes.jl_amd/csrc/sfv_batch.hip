@@ -35,7 +35,7 @@ BatchEngine::~BatchEngine() {
     if (d_ctl_) (void)hipFree(d_ctl_);
     if (h_mem_) (void)hipHostFree(h_mem_);
     if (h_hdr_) (void)hipHostFree(h_hdr_);
-    if (h_ctl_) (void)hipHostFree(h_ctl_);
+    if (h_rep_) (void)hipHostFree(h_rep_);
     if (stream_) (void)hipStreamDestroy(stream_);
 }
 
@@ -88,11 +88,11 @@ int BatchEngine::grow(int capacity, std::string& why) {
     BatchMember* dm = nullptr;
     StepCtl* dc = nullptr;
     BatchMember* hm = nullptr;
-    StepCtl* hc = nullptr;
+    BatchReport* hc = nullptr;
     if (hipMalloc((void**)&dm, sizeof(BatchMember) * capacity) != hipSuccess ||
         hipMalloc((void**)&dc, sizeof(StepCtl) * capacity) != hipSuccess ||
         hipHostMalloc((void**)&hm, sizeof(BatchMember) * capacity, hipHostMallocDefault) != hipSuccess ||
-        hipHostMalloc((void**)&hc, sizeof(StepCtl) * capacity, hipHostMallocDefault) != hipSuccess) {
+        hipHostMalloc((void**)&hc, sizeof(BatchReport) * capacity, hipHostMallocDefault) != hipSuccess) {
         if (dm) (void)hipFree(dm);
         if (dc) (void)hipFree(dc);
         if (hm) (void)hipHostFree(hm);
@@ -100,17 +100,17 @@ int BatchEngine::grow(int capacity, std::string& why) {
         why = "allocation of the batch tables failed";
         return SFV_ERR_OUT_OF_MEMORY;
     }
-    std::memset(hc, 0, sizeof(StepCtl) * capacity);
+    std::memset(hc, 0, sizeof(BatchReport) * capacity);
     if (d_ctl_) {   // members keep their step control across the move
         ETRY(hipMemcpyAsync(dc, d_ctl_, sizeof(StepCtl) * capacity_, hipMemcpyDeviceToDevice, stream_));
-        std::memcpy(hc, h_ctl_, sizeof(StepCtl) * capacity_);
+        std::memcpy(hc, h_rep_, sizeof(BatchReport) * capacity_);
         ETRY(hipStreamSynchronize(stream_));
         (void)hipFree(d_mem_);
         (void)hipFree(d_ctl_);
         (void)hipHostFree(h_mem_);
-        (void)hipHostFree(h_ctl_);
+        (void)hipHostFree(h_rep_);
     }
-    d_mem_ = dm; d_ctl_ = dc; h_mem_ = hm; h_ctl_ = hc;
+    d_mem_ = dm; d_ctl_ = dc; h_mem_ = hm; h_rep_ = hc;
     capacity_ = capacity;
     slot_handle_.resize(capacity, nullptr);
     slot_row_.resize(capacity);
@@ -183,7 +183,7 @@ void BatchEngine::remove(int slot) {
     sfv_handle* h = slot_handle_[slot];
     if (!h) return;
     if (ran_[slot]) {
-        const StepCtl& c = h_ctl_[slot];
+        const BatchReport& c = h_rep_[slot];
         h->cur = (h->cur + c.steps) & 1;
         h->step_parity = (h->step_parity + c.steps) & 1;
         if (c.steps > 0) {
@@ -209,7 +209,7 @@ void BatchEngine::remove(int slot) {
 bool BatchEngine::finished(int slot) const {
     if (!ran_[slot]) return false;
     // replays end on launch parity 0, where the member's next slot is slot0
-    return h_ctl_[slot].slot[slot_row_[slot].slot0].active == 0;
+    return h_rep_[slot].active == 0;
 }
 
 // Segment heights of the members for the current membership.  When the
@@ -386,7 +386,9 @@ int BatchEngine::replay_begin(int k, std::string& why) {
     if (timed_k_) ETRY(hipEventRecord(ev_[0], stream_));
     for (int r = 0; r < k; ++r) ETRY(hipGraphLaunch(graph_, stream_));
     if (timed_k_) ETRY(hipEventRecord(ev_[1], stream_));
-    ETRY(hipMemcpyAsync(h_ctl_, d_ctl_, sizeof(StepCtl) * capacity_, hipMemcpyDeviceToHost, stream_));
+    // a few words per member go straight to pinned memory: a control block is
+    // mostly wave-speed lines (3.6 KB)
+    if (!rows_.empty()) ETRY(launch_report_batch(stream_, d_mem_, d_ctl_, h_rep_, members()));
     return SFV_OK;
 }
 
@@ -562,7 +564,7 @@ int sfv_batch_run(sfv_batch* b, const double* t_end, int32_t match_endtime, doub
     }
     int status = SFV_OK;
     for (int i = 0; i < n; ++i) {
-        const sfv::StepCtl& c = b->engine.ctl(slots[i]);
+        const sfv::BatchReport& c = b->engine.report(slots[i]);
         t_io[i] = c.t;
         if (steps_out) steps_out[i] = c.steps;
         if (c.nonfinite && status == SFV_OK)

@@ -57,8 +57,8 @@ public:
     int replay(int k, std::string& why);
     // The same in two halves, so the host can work while the device steps:
     // replay_begin queues the replays and the step-control copy; replay_end
-    // waits for them.  Between the two, add / remove / finished / ctl must
-    // not be called (they use the table and the step-control mirror).
+    // waits for them.  Between the two, add / remove / finished / report must
+    // not be called (they use the table and the members' reports).
     int replay_begin(int k, std::string& why);
     int replay_end(std::string& why);
     // Without waiting: has the work queued by replay_begin finished?  (Also
@@ -89,7 +89,7 @@ public:
     int members() const { return (int)rows_.size(); }
     // After replay: has the member in `slot` finished its run?
     bool finished(int slot) const;
-    const StepCtl& ctl(int slot) const { return h_ctl_[slot]; }
+    const BatchReport& report(int slot) const { return h_rep_[slot]; }
     sfv_handle* handle(int slot) const { return slot_handle_[slot]; }
     hipStream_t stream() const { return stream_; }
     int graph_steps() const { return graph_steps_; }
@@ -118,7 +118,7 @@ private:
     BatchMember* h_mem_ = nullptr;
     BatchHeader* h_hdr_ = nullptr;
     StepCtl* d_ctl_ = nullptr;
-    StepCtl* h_ctl_ = nullptr;
+    BatchReport* h_rep_ = nullptr;    // pinned, by slot; written after the replays
     hipGraphExec_t graph_ = nullptr;
     bool table_dirty_ = true;
     bool members_changed_ = false;

@@ -207,7 +207,7 @@ void sfv_server::work() {
         std::vector<Request*> still;
         for (Request* r : run[e]) {
             if (!engs[e].finished(r->slot)) { still.push_back(r); continue; }
-            const sfv::StepCtl& c = engs[e].ctl(r->slot);
+            const sfv::BatchReport& c = engs[e].report(r->slot);
             r->t = c.t;
             r->steps = c.steps;
             r->error = c.nonfinite != 0 ? SFV_ERR_NONFINITE_DT : SFV_OK;

@@ -119,6 +119,13 @@ struct BatchMember {
     long long max_steps;
     int match_endtime, has_max_timestep, until_endtime, precision;
 };
+// What the host reads of a member after replays.
+struct BatchReport {
+    double t, dt;
+    long long steps;
+    int nonfinite;
+    int active;           // of the member's next slot
+};
 // Batch-wide counts, in device memory beside the member table.
 struct BatchHeader {
     int members;

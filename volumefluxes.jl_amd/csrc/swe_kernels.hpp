@@ -47,6 +47,9 @@ hipError_t launch_march_batch(hipStream_t st, int stage, const BatchMember* mem,
 constexpr int MAX_MODE = 2;
 int march_mode(const KParams& P);
 hipError_t launch_prepare_batch(hipStream_t st, const BatchMember* mem, const BatchHeader* hdr, int members);
+// Every member's report to out[its control block's index from base] (pinned).
+hipError_t launch_report_batch(hipStream_t st, const BatchMember* mem, const StepCtl* base, BatchReport* out,
+                               int members);
 // Resident workgroups per CU of the batched stage kernel (occupancy).
 int march_batch_blocks_per_cu(int precision, int stage, int mode);
 int march_rows_per_wave(const KParams& P, int stage, int precision);   // precision: 0 f64, 1 f32

@@ -113,6 +113,19 @@ __global__ void k_prepare_batch(const BatchMember* __restrict__ mem, const Batch
                 M.max_steps, M.until_endtime, M.precision, nullptr);
 }
 
+// After an even number of steps the member's next slot is slot0 again.
+__global__ void k_report_batch(const BatchMember* __restrict__ mem, const StepCtl* base, BatchReport* __restrict__ out,
+                               int members) {
+    const int m = blockIdx.x * blockDim.x + threadIdx.x;
+    if (m >= members) return;
+    const StepCtl* c = mem[m].ctl;
+    out[c - base] = BatchReport{c->t, c->dt, (long long)c->steps, c->nonfinite, c->slot[mem[m].slot0 & 1].active};
+}
+hipError_t launch_report_batch(hipStream_t st, const BatchMember* mem, const StepCtl* base, BatchReport* out,
+                               int members) {
+    hipLaunchKernelGGL(k_report_batch, dim3((members + 63) / 64), dim3(64), 0, st, mem, base, out, members);
+    return hipPeekAtLastError();
+}
 hipError_t launch_prepare_batch(hipStream_t st, const BatchMember* mem, const BatchHeader* hdr, int members) {
     hipLaunchKernelGGL(k_prepare_batch, dim3((members + 63) / 64), dim3(64), 0, st, mem, hdr);
     return hipPeekAtLastError();

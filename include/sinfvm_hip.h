@@ -215,10 +215,10 @@ int sfv_device_count(void);
  * boundary-condition sources of the ghost cells are interior cells; unless a
  * variant is set here, the first step switches to 1 where that suits the
  * grid); 1 = the same stages with one workgroup per strip segment, for grids
- * too small to fill the device; 3 = every right-hand side from the stage-1
- * kernel, the updates and boundary conditions from the per-pass kernels (any
- * stepper and boundary condition with gc >= 2: the default for NeumannBC and
- * ForwardEuler); 0 = one kernel per reference pass (the device-side
+ * too small to fill the device; 3 = right-hand sides from the stage kernels,
+ * updates from the per-pass kernels, or for ForwardEuler both in one launch a
+ * step (any stepper and boundary condition with gc >= 2: the default for
+ * NeumannBC and ForwardEuler); 0 = one kernel per reference pass (the device-side
  * reference).  All give bitwise identical results.  No counterpart in the
  * reference. */
 int sfv_set_fused(sfv_handle* h, int32_t fused);
@@ -231,7 +231,8 @@ int32_t sfv_get_fused(const sfv_handle* h);
  * workgroup kernels, without a measurement): candidate heights are timed on
  * the handle's own state and the fastest is kept for grids of that size class
  * (quarter octaves of nx and ny) on that device; the environment variable
- * SFV_AUTOTUNE=0 turns the measurement off (the height that makes the launch shortest by the waves it puts on each SIMD is used).
+ * SFV_AUTOTUNE=0 turns the measurement off (the model's height is used: the
+ * one that makes the launch shortest by the waves it puts on each SIMD).
  * rows > 0 forces a height.  Results are bitwise the same for every height.
  * No counterpart in the reference. */
 int sfv_set_march_rows(sfv_handle* h, int32_t rows);

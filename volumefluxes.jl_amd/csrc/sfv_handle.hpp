@@ -212,8 +212,9 @@ struct sfv_handle {
         return SFV_OK;
     }
 
-    // U[2] is allocated on first use: only the per-pass and hybrid RK2 paths (their stage-1
-    // state) and kernel timing (a scratch output) need it.
+    // U[2] is allocated on first use: the per-pass and hybrid RK2 paths (their stage-1
+    // state), the ForwardEuler loop (its second right-hand side) and kernel timing (a
+    // scratch output) need it.
     int ensure_scratch(std::string& why) {
         if (U[2]) return SFV_OK;
         return alloc(&U[2], 3 * ncell * elem, why);

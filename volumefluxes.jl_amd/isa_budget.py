@@ -3,8 +3,8 @@
 Reads the AMD assembly of this build with line tables (the `isa-budget`
 target of the Makefile: hipcc -gline-tables-only --cuda-device-only -S of
 csrc/swe_kernels_march.hip, same flags as the library), finds the row loops
-of k_march<double, 1, true> and k_march<double, 2, true> (the kernels of
-the f64 terrain workload), and attributes every instruction of each loop to
+of k_march<double, 1, MODE_POW2> and k_march<double, 2, MODE_POW2> (the
+kernels of the f64 terrain workload), and attributes every instruction of each loop to
 the source function or row phase its line-table entry names.  The counts
 are static: one loop iteration is one row of a wave, and both sides of a
 branch are counted (the general face path, for example, runs only in waves
@@ -20,14 +20,14 @@ import re
 import sys
 
 KERNELS = {
-    "stage 1": "_ZN3sfv7k_marchIdLi1ELb1E",
-    "stage 2": "_ZN3sfv7k_marchIdLi2ELb1E",
+    "stage 1": "_ZN3sfv7k_marchIdLi1ELi2E",
+    "stage 2": "_ZN3sfv7k_marchIdLi2ELi2E",
 }
 
 # source function -> phase
 PHASE = {
     "reconstruct_cell": "reconstruction (minmod slopes, face values)",
-    "reconstruct_cell_nb": "reconstruction (minmod slopes, face values)",
+    "reconstruct_cell_rng": "reconstruction (minmod slopes, face values)",
     "minmod": "reconstruction (minmod slopes, face values)",
     "central_upwind_rng": "faces: central-upwind flux, ranged quotients",
     "phys_flux_rng": "faces: central-upwind flux, ranged quotients",
@@ -37,43 +37,46 @@ PHASE = {
     "central_upwind": "faces: general path (waves out of band)",
     "phys_flux": "faces: general path (waves out of band)",
     "desingularize": "desingularisation (faces and friction)",
+    "desingularize_rng": "desingularisation (faces and friction)",
     "friction_scalar": "friction (scalar and implicit update)",
     "friction_law": "friction (scalar and implicit update)",
+    "friction_scalar_rng": "friction (scalar and implicit update)",
     "apply_friction": "friction (scalar and implicit update)",
     "stage1_cell": "U1 rebuild: RK stage 1 and dry clamp",
+    "stage1_cell_rng": "U1 rebuild: RK stage 1 and dry clamp",
+    "stage1_any": "U1 rebuild: RK stage 1 and dry clamp",
+    "stage2_cell": "RK2 combination and output clamp",
+    "bottom_term": "bottom source",
+    "y_part": "y flux difference",
+    "raise_speed": "faces: dispatch and wave-speed maxima",
     "in_band": "band checks and votes",
-    "in_band5": "band checks and votes",
     "set_issue_priority": "issue priority (rows left)",
     "dpp_shift": "lane shifts (DPP)",
     "shfl_dn1": "lane shifts (DPP)",
     "shfl_up1": "lane shifts (DPP)",
-    "next_col": "lane shifts (DPP)",
     "row_rsrc": "row loads and stores (descriptors, offsets)",
     "rsrc_ld": "row loads and stores (descriptors, offsets)",
     "row_ld": "row loads and stores (descriptors, offsets)",
     "row_st": "row loads and stores (descriptors, offsets)",
     "Bload_row": "row loads and stores (descriptors, offsets)",
     "fetch": "row loads and stores (descriptors, offsets)",
-    "fetch_b": "row loads and stores (descriptors, offsets)",
+    "Bload_row2": "row loads and stores (descriptors, offsets)",
+    "row_ld2": "row loads and stores (descriptors, offsets)",
     "jl_max": "Julia max/min (NaN-propagating selects)",
     "jl_min": "Julia max/min (NaN-propagating selects)",
     "nz_max": "Julia max/min (NaN-propagating selects)",
     "nz_min": "Julia max/min (NaN-propagating selects)",
-    "sdiv": "x flux difference and bottom source",
-    "bc4": "cell bottoms",
+    "cell_bottom": "cell bottoms",
     "bcell4": "cell bottoms",
-    "face_y": "faces: dispatch and wave-speed maxima",
-    "face_x": "faces: dispatch and wave-speed maxima",
-    "sources": "sources (rain)",
+    "uniform_sources": "sources (rain)",
     "apply_sources": "sources (rain)",
 }
-# row phases inside march_tile's `body` lambda, by the comment that opens them
+# row phases inside march_tile's `work` lambda, by the comment that opens them
 BODY_MARKERS = [
-    ("// 1. y reconstruction", "row glue: reconstruction inputs and face bottoms"),
-    ("// 2. the faces", "faces: dispatch and wave-speed maxima"),
-    ("// 3. x part", "x flux difference and bottom source"),
-    ("// 4. finish row", "y flux difference, RK2 combination, output clamp"),
-    ("// shift the windows", "window shifts (register moves)"),
+    ("// y reconstruction of row", "row glue: reconstruction inputs and face bottoms"),
+    ("// the y face between", "faces: dispatch and wave-speed maxima"),
+    ("// finish row p", "y flux difference, RK2 combination, output clamp"),
+    ("// x part of row q", "x flux difference and bottom source"),
 ]
 DEF_RE = re.compile(r"(?:__device__[^(;]*?\b(\w+)\s*\(|auto\s+(\w+)\s*=\s*\[)")
 
@@ -116,7 +119,7 @@ def phase_of(defs, lines, line):
     if inner is None:
         return "other"
     name = inner[2]
-    if name == "body":
+    if name == "work":
         label = "row glue: loop control"
         for k in range(inner[0], line + 1):
             for marker, lab in BODY_MARKERS:
@@ -133,8 +136,8 @@ def phase_of(defs, lines, line):
 # functions whose phase absorbs the helpers they call (desingularisation,
 # square roots, quotients, NaN-propagating selects): a helper's instructions
 # count under the innermost of these on its inlining chain
-MAJOR = {"reconstruct_cell", "reconstruct_cell_nb", "central_upwind_rng", "phys_flux_rng", "central_upwind",
-         "phys_flux", "friction_scalar", "friction_law", "apply_friction", "stage1_cell"}
+MAJOR = {"reconstruct_cell", "reconstruct_cell_rng", "central_upwind_rng", "phys_flux_rng", "central_upwind",
+         "phys_flux", "friction_scalar", "friction_scalar_rng", "friction_law", "apply_friction", "stage1_cell"}
 FRAME_RE = re.compile(r"([\w./-]+\.(?:hpp|hip|h)):(\d+):\d+")
 
 

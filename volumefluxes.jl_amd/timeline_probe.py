@@ -28,7 +28,7 @@ import volumefluxes as VF  # noqa: E402
 from volumefluxes import _capi as C  # noqa: E402
 from volumefluxes.scenarios import terrain_workload  # noqa: E402
 
-TL_WAVES, TL_ROWS, SLOTS_PER_SIMD = 16384, 32, 3
+TL_WAVES, TL_ROWS, SLOTS_PER_SIMD = 16384, 32, 4
 
 
 def record(sim, L):

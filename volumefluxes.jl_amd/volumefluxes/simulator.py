@@ -144,10 +144,10 @@ class Simulator:
     KERNELS = {"per-pass": 0, "tiled": 1, "march": 2, "hybrid": 3}
 
     def set_kernels(self, variant: str) -> None:
-        """Choose the kernels of a step: "march" (the RK2 default), "tiled",
-        "hybrid" (march stage-1 right-hand sides with per-pass updates: the
-        default for ForwardEuler and NeumannBC) or "per-pass".  All give
-        bitwise identical results."""
+        """Choose the kernels of a step: "march" (one wave per strip segment),
+        "tiled" (one workgroup per strip segment; the first step picks it on
+        small grids), "hybrid" (the default for ForwardEuler and NeumannBC) or
+        "per-pass".  All give bitwise identical results."""
         C.check(self._h, C.lib().sfv_set_fused(self._h, self.KERNELS[variant]))
 
     @property

@@ -30,7 +30,7 @@ def _fill(sim, seed):
 
 
 # nx, ny with 4 ghost rows and columns: bytes = 3 * 8 * (nx + 4) * (ny + 4)
-@pytest.mark.parametrize("nx,ny", [(291, 292), (292, 292), (508, 508), (509, 508), (1020, 1020), (1021, 1020), (509, 1363),
+@pytest.mark.parametrize("nx,ny", [(508, 508), (587, 587), (588, 587), (1020, 1020), (1021, 1020), (509, 1363),
                                    (1277, 1399)])
 def test_bytes(nx, ny):
     sim = _sim(nx, ny)
@@ -49,7 +49,7 @@ def test_float32_and_interior():
 
 
 def test_threads():
-    sims = [_sim(400 + 40 * k, 500) for k in range(7)]
+    sims = [_sim(700 + 40 * k, 500) for k in range(7)]
     states = [_fill(s, k) for k, s in enumerate(sims)]
     bad = []
 

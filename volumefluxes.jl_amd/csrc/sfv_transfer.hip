@@ -6,15 +6,15 @@
 // here goes through a ring of pinned slots: the calling thread queues the DMA
 // of the next chunks while worker threads empty the slots that have arrived,
 // so the copies and page faults of several threads overlap with the DMA.
-// Measured, us for the plain copy and this one: 4 MB mapped 251 and 180, fresh
-// 943 and 400; 36 MB 2080 and 1000, fresh 8500 and 2250; 100 MB 5920 and 2630,
+// Measured, us for the plain copy and this one: 12 MB mapped 700 and 390, fresh
+// 2810 and 1150; 36 MB 2080 and 1000, fresh 8500 and 2250; 100 MB 5920 and 2630,
 // fresh 23700 and 5140.
 //
 // The slots belong to a lane, one lane per copy under way.  At most MAX_LANES
 // lanes exist in the process (64 MB); they are made on first use, kept while
 // any handle lives and freed with the last one.  A copy that finds none free
-// is a plain one, as is one below MIN_STAGED: a 64x48 state (85 KB) took 20 us
-// longer through a slot.
+// is a plain one, as is one below MIN_STAGED: 6 MB gain 0.1 ms at most, and the
+// slots cost 1 ms when a process's first handles (a server's) make them.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -29,36 +29,38 @@ namespace sfv {
 namespace {
 
 constexpr int SLOTS = 8, MAX_LANES = 4, MAX_WORKERS = 8;
-constexpr size_t SLOT_BYTES = (size_t)2 << 20, MIN_CHUNK = (size_t)256 << 10;
-constexpr size_t MIN_STAGED = (size_t)2 << 20;
+constexpr size_t SLOT_BYTES = (size_t)2 << 20;
+constexpr size_t MIN_STAGED = (size_t)8 << 20;
 
 struct Lane {
     int device = -1;                    // -1: not made yet
     bool busy = false;
-    char* slot[SLOTS] = {};             // pinned, allocated as copies need them
+    // pinned, SLOTS slots of SLOT_BYTES, in one allocation made by the first copy
+    // (eight allocations and their release took 2 ms each)
+    char* memory = nullptr;
     hipEvent_t arrived[SLOTS] = {};
-    // the first `count` slots exist after this; false if memory is short
-    bool reserve(int count) {
-        for (int k = 0; k < count; ++k) {
-            if (!slot[k] && hipHostMalloc((void**)&slot[k], SLOT_BYTES, hipHostMallocDefault) != hipSuccess) {
-                slot[k] = nullptr;
-                (void)hipGetLastError();
-                return false;
-            }
-            if (!arrived[k] && hipEventCreateWithFlags(&arrived[k], hipEventDisableTiming) != hipSuccess) {
-                arrived[k] = nullptr;
-                (void)hipGetLastError();
-                return false;
-            }
+    char* slot(long c) const { return memory + (size_t)(c % SLOTS) * SLOT_BYTES; }
+    // false if memory is short
+    bool reserve() {
+        if (!memory && hipHostMalloc((void**)&memory, SLOTS * SLOT_BYTES, hipHostMallocDefault) != hipSuccess) {
+            memory = nullptr;
+            (void)hipGetLastError();
+            return false;
         }
+        for (hipEvent_t& e : arrived)
+            if (!e && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) {
+                e = nullptr;
+                (void)hipGetLastError();
+                return false;
+            }
         return true;
     }
     void release() {
-        for (int k = 0; k < SLOTS; ++k) {
-            if (slot[k]) (void)hipHostFree(slot[k]);
-            if (arrived[k]) (void)hipEventDestroy(arrived[k]);
-            slot[k] = nullptr;
-            arrived[k] = nullptr;
+        if (memory) (void)hipHostFree(memory);
+        memory = nullptr;
+        for (hipEvent_t& e : arrived) {
+            if (e) (void)hipEventDestroy(e);
+            e = nullptr;
         }
         device = -1;
     }
@@ -106,7 +108,7 @@ hipError_t staged(Lane& L, char* dst, const char* src, size_t n, hipStream_t st,
     for (auto& e : emptied) e.store(0);
     auto bytes = [&](long c) { return std::min(chunk, n - (size_t)c * chunk); };
     auto empty_slot = [&](long c) {
-        std::memcpy(dst + (size_t)c * chunk, L.slot[c % SLOTS], bytes(c));
+        std::memcpy(dst + (size_t)c * chunk, L.slot(c), bytes(c));
         emptied[c % SLOTS].store(c / SLOTS + 1, std::memory_order_release);
     };
     auto work = [&] {
@@ -125,7 +127,7 @@ hipError_t staged(Lane& L, char* dst, const char* src, size_t n, hipStream_t st,
     long queued = 0;
     auto queue = [&] {
         const int s = (int)(queued % SLOTS);
-        e = hipMemcpyAsync(L.slot[s], src + (size_t)queued * chunk, bytes(queued), hipMemcpyDeviceToHost, st);
+        e = hipMemcpyAsync(L.slot(queued), src + (size_t)queued * chunk, bytes(queued), hipMemcpyDeviceToHost, st);
         if (e == hipSuccess) e = hipEventRecord(L.arrived[s], st);
         ++queued;
     };
@@ -174,14 +176,13 @@ hipError_t copy_to_host(void* dst, const void* src, size_t n, hipStream_t st) {
     if (n < MIN_STAGED || hipGetDevice(&device) != hipSuccess) return plain(dst, src, n, st);
     Lane* lane = take_lane(device);
     if (!lane) return plain(dst, src, n, st);
-    // eight chunks, each from MIN_CHUNK up to a slot
-    const size_t chunk = std::min(SLOT_BYTES, std::max(MIN_CHUNK, (n + SLOTS - 1) / SLOTS));
-    const long chunks = (long)((n + chunk - 1) / chunk);
+    // at least eight chunks, of at most a slot
+    const size_t chunk = std::min(SLOT_BYTES, (n + SLOTS - 1) / SLOTS);
     const int cpus = std::max(1, (int)std::thread::hardware_concurrency());
     // a worker for every slot's worth: starting one takes 15 us, copying 2 MB 200
     const int want = (int)std::min({(long)(n / SLOT_BYTES), (long)MAX_WORKERS, (long)std::max(1, cpus / 2)});
     hipError_t e;
-    if (lane->reserve((int)std::min(chunks, (long)SLOTS))) e = staged(*lane, (char*)dst, (const char*)src, n, st, chunk, want);
+    if (lane->reserve()) e = staged(*lane, (char*)dst, (const char*)src, n, st, chunk, want);
     else e = plain(dst, src, n, st);
     give_lane(lane);
     return e;

@@ -9,7 +9,8 @@
 namespace sfv {
 
 // Copy n bytes from the current device to dst after the work queued on st;
-// returns when they are there.  Any number of threads may copy at once.
+// returns when they are there.  dst may be any memory a plain copy could write,
+// pinned and device memory included.  Any number of threads may copy at once.
 hipError_t copy_to_host(void* dst, const void* src, size_t n, hipStream_t st);
 
 // Each handle holds the staging memory; it is freed with the last of them.

@@ -74,6 +74,74 @@ int pinned_destination() {
     return known_destination((char*)p, false);
 }
 
+// The caller's stream only waits: the copies run on another.
+int callers_stream() {
+    sfv::staging_retain();
+    Source s(20 * MB);
+    StubStream st;
+    s.queue_on(&st);
+    std::vector<char> out(s.n);
+    CHECK(sfv::copy_to_host(out.data(), s.dev, s.n, &st) == hipSuccess);
+    CHECK(std::memcmp(out.data(), s.want.data(), s.n) == 0);
+    CHECK(stub::copies >= 10);                    // staged
+    CHECK(st.copies == 0 && st.events == 0);
+    sfv::staging_release();
+    return 0;
+}
+
+// Handles made, read and destroyed one after the other share one lane; the
+// first that goes without having read as much gives it back.
+int one_after_the_other() {
+    for (int k = 0; k < 5; ++k) {
+        sfv::staging_retain();
+        CHECK(bytes_of(12 * MB) == 0);
+        sfv::staging_release();
+        CHECK(stub::host_allocs == 1 && stub::host_live == 1 && stub::streams_live == 1);
+    }
+    sfv::staging_retain();
+    CHECK(bytes_of(MB) == 0);
+    CHECK(stub::host_live == 1);
+    sfv::staging_release();
+    CHECK(stub::host_live == 0 && stub::streams_live == 0 && stub::events_live == 0);
+    return 0;
+}
+
+// Threads that copy at once have at most MAX_LANES lanes; one is left at most.
+int many_at_once() {
+    constexpr int T = 9;
+    for (int k = 0; k < T; ++k) sfv::staging_retain();
+    std::atomic<int> bad{0};
+    std::vector<std::thread> threads;
+    for (int k = 0; k < T; ++k)
+        threads.emplace_back([&] {
+            for (int r = 0; r < 3; ++r) bad += bytes_of(17 * MB + 1);
+        });
+    for (auto& t : threads) t.join();
+    CHECK(bad == 0);
+    CHECK(stub::host_live <= 4 && stub::streams_live <= 4);
+    for (int k = 0; k < T; ++k) sfv::staging_release();
+    CHECK(stub::host_live <= 1 && stub::streams_live <= 1);
+    return 0;
+}
+
+// A copy that fails ends with its error, with no thread left, and the next works.
+int failing() {
+    sfv::staging_retain();
+    Source s(40 * MB);
+    StubStream st;
+    s.queue_on(&st);
+    std::vector<char> out(s.n);
+    for (long k : {0L, 3L, 8L, 19L}) {
+        stub::fail_copy = k;
+        CHECK(sfv::copy_to_host(out.data(), s.dev, s.n, &st) == hipErrorUnknown);
+    }
+    stub::fail_copy = -1;
+    CHECK(sfv::copy_to_host(out.data(), s.dev, s.n, &st) == hipSuccess);
+    CHECK(std::memcmp(out.data(), s.want.data(), s.n) == 0);
+    sfv::staging_release();
+    return 0;
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -81,6 +149,10 @@ int main(int argc, char** argv) {
     if (what == "pageable") return pageable();
     if (what == "device_destination") return device_destination();
     if (what == "pinned_destination") return pinned_destination();
+    if (what == "callers_stream") return callers_stream();
+    if (what == "one_after_the_other") return one_after_the_other();
+    if (what == "many_at_once") return many_at_once();
+    if (what == "failing") return failing();
     std::printf("unknown scenario\n");
     return 2;
 }

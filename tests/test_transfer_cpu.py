@@ -19,7 +19,8 @@ def program(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("scenario", ["pageable", "device_destination", "pinned_destination"])
+@pytest.mark.parametrize("scenario", ["pageable", "device_destination", "pinned_destination", "callers_stream",
+                                      "one_after_the_other", "many_at_once", "failing"])
 def test_copy_to_host(program, scenario):
     r = subprocess.run([program, scenario], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, (r.returncode, r.stdout, r.stderr)

@@ -6,16 +6,28 @@
 // here goes through a ring of pinned slots: the calling thread queues the DMA
 // of the next chunks while worker threads empty the slots that have arrived,
 // so the copies and page faults of several threads overlap with the DMA.
-// Measured, us for the plain copy and this one: 12 MB mapped 700 and 390, fresh
-// 2810 and 1150; 36 MB 2080 and 1000, fresh 8500 and 2250; 100 MB 5920 and 2630,
-// fresh 23700 and 5140.
+// Measured, us for the plain copy and this one: 9 MB mapped 535 and 330; 20 MB
+// 1100 and 550; 35 MB 2000 and 920, fresh 3500 and 1350; 101 MB 5800 and 2550,
+// fresh 9800 and 2900.
 //
-// The slots belong to a lane, one lane per copy under way.  At most MAX_LANES
-// lanes exist in the process (64 MB); they are made on first use, kept while
-// any handle lives and freed with the last one.  A copy that finds none free
-// is a plain one, as is one into memory of the runtime's own and one below MIN_STAGED: 6 MB gain 0.1 ms at most, and the
-// slots cost 1 ms when a process's first handles (a server's) make them.
+// The slots belong to a lane, one lane per copy under way, with a stream of its
+// own; at most MAX_LANES lanes exist in the process (64 MB), made on first use.
+// A copy that finds none free is a plain one, as is one into memory of the
+// runtime's own and one below MIN_STAGED: 6 MB gain 0.1 ms at most.
+//
+// A copy leaves nothing behind on the caller's stream, and no mapping of the
+// process changes: the runtime gives the queue of a destroyed stream to the next
+// one only if it is idle for good, and a new queue costs 1.1 ms and its first
+// uploads run at 2.6 GB/s.  With the DMAs on the caller's stream, or with
+// default-size stacks for eight threads (64 MB, more than the C library keeps
+// for reuse, so that every copy unmapped some), that met most handles made
+// after one was read and destroyed; making the lane again cost as much.  For a
+// handle made, stepped twice, read and destroyed, ms (plain copies; as it was;
+// now): 9 MB 1.4, 8.6, 1.3; 20 MB 3.0, 11, 2.4; 54 MB 7.9, 12, 6.5.  So one lane
+// also outlives the last handle, and is freed when a later last handle goes
+// without one of its generation having needed it.
 #include <hip/hip_runtime.h>
+#include <pthread.h>
 
 #include <algorithm>
 #include <atomic>
@@ -31,10 +43,12 @@ namespace {
 constexpr int SLOTS = 8, MAX_LANES = 4, MAX_WORKERS = 8;
 constexpr size_t SLOT_BYTES = (size_t)2 << 20;
 constexpr size_t MIN_STAGED = (size_t)8 << 20;
+constexpr size_t WORKER_STACK = (size_t)256 << 10;
 
 struct Lane {
     int device = -1;                    // -1: not made yet
     bool busy = false;
+    hipStream_t stream = nullptr;
     // pinned, SLOTS slots of SLOT_BYTES, in one allocation made by the first copy
     // (eight allocations and their release took 2 ms each)
     char* memory = nullptr;
@@ -42,6 +56,11 @@ struct Lane {
     char* slot(long c) const { return memory + (size_t)(c % SLOTS) * SLOT_BYTES; }
     // false if memory is short
     bool reserve() {
+        if (!stream && hipStreamCreateWithFlags(&stream, hipStreamNonBlocking) != hipSuccess) {
+            stream = nullptr;
+            (void)hipGetLastError();
+            return false;
+        }
         if (!memory && hipHostMalloc((void**)&memory, SLOTS * SLOT_BYTES, hipHostMallocDefault) != hipSuccess) {
             memory = nullptr;
             (void)hipGetLastError();
@@ -62,6 +81,8 @@ struct Lane {
             if (e) (void)hipEventDestroy(e);
             e = nullptr;
         }
+        if (stream) (void)hipStreamDestroy(stream);
+        stream = nullptr;
         device = -1;
     }
 };
@@ -69,11 +90,13 @@ struct Lane {
 std::mutex g_mu;
 Lane g_lanes[MAX_LANES];
 int g_users = 0;
+bool g_needed = false;                  // a lane was taken since the first of these users came
 
 // A free lane of this device (an event serves its own device's streams only),
 // or nullptr.
 Lane* take_lane(int device) {
     std::lock_guard<std::mutex> lk(g_mu);
+    g_needed = true;
     for (Lane& l : g_lanes)
         if (!l.busy && l.device == device) {
             l.busy = true;
@@ -110,7 +133,8 @@ bool runtime_memory(const void* p) {
 
 // Chunk c travels through slot c mod SLOTS.  `arrived` counts the chunks whose
 // DMA has completed, emptied[s] those copied out of slot s.
-hipError_t staged(Lane& L, char* dst, const char* src, size_t n, hipStream_t st, size_t chunk, int want) {
+hipError_t staged(Lane& L, char* dst, const char* src, size_t n, size_t chunk, int want) {
+    const hipStream_t st = L.stream;
     const long chunks = (long)((n + chunk - 1) / chunk);
     std::atomic<long> arrived{0}, next{0};
     std::atomic<bool> stop{false};
@@ -142,11 +166,18 @@ hipError_t staged(Lane& L, char* dst, const char* src, size_t n, hipStream_t st,
         ++queued;
     };
     while (e == hipSuccess && queued < chunks && queued < SLOTS) queue();
-    std::thread workers[MAX_WORKERS];
+    pthread_t workers[MAX_WORKERS];
     int running = 0;
-    try {
-        for (; e == hipSuccess && running < want; ++running) workers[running] = std::thread(work);
-    } catch (...) {                     // no more threads: those there are, or this one, do it
+    auto entry = [](void* w) -> void* {
+        (*static_cast<decltype(work)*>(w))();
+        return nullptr;
+    };
+    pthread_attr_t attr;
+    if (pthread_attr_init(&attr) == 0) {
+        (void)pthread_attr_setstacksize(&attr, WORKER_STACK);
+        // no more threads: those there are, or this one, do it
+        while (e == hipSuccess && running < want && pthread_create(&workers[running], &attr, entry, &work) == 0) ++running;
+        (void)pthread_attr_destroy(&attr);
     }
     for (long c = 0; c < chunks && e == hipSuccess; ++c) {
         e = hipEventSynchronize(L.arrived[c % SLOTS]);
@@ -164,7 +195,7 @@ hipError_t staged(Lane& L, char* dst, const char* src, size_t n, hipStream_t st,
         stop.store(true);
         (void)hipStreamSynchronize(st);  // no DMA into a slot outlives the copy
     }
-    for (int k = 0; k < running; ++k) workers[k].join();
+    for (int k = 0; k < running; ++k) (void)pthread_join(workers[k], nullptr);
     return e;
 }
 
@@ -177,8 +208,13 @@ void staging_retain() {
 void staging_release() {
     std::lock_guard<std::mutex> lk(g_mu);
     if (--g_users > 0) return;
-    for (Lane& l : g_lanes)
-        if (!l.busy) l.release();
+    bool keep = g_needed;               // one, for the next user
+    g_needed = false;
+    for (Lane& l : g_lanes) {
+        if (l.busy) continue;
+        if (keep && l.memory) keep = false;
+        else l.release();
+    }
 }
 
 hipError_t copy_to_host(void* dst, const void* src, size_t n, hipStream_t st) {
@@ -192,8 +228,12 @@ hipError_t copy_to_host(void* dst, const void* src, size_t n, hipStream_t st) {
     // a worker for every slot's worth: starting one takes 15 us, copying 2 MB 200
     const int want = (int)std::min({(long)(n / SLOT_BYTES), (long)MAX_WORKERS, (long)std::max(1, cpus / 2)});
     hipError_t e;
-    if (lane->reserve()) e = staged(*lane, (char*)dst, (const char*)src, n, st, chunk, want);
-    else e = plain(dst, src, n, st);
+    if (lane->reserve()) {
+        e = hipStreamSynchronize(st);
+        if (e == hipSuccess) e = staged(*lane, (char*)dst, (const char*)src, n, chunk, want);
+    } else {
+        e = plain(dst, src, n, st);
+    }
     give_lane(lane);
     return e;
 }

@@ -13,7 +13,8 @@ namespace sfv {
 // pinned and device memory included.  Any number of threads may copy at once.
 hipError_t copy_to_host(void* dst, const void* src, size_t n, hipStream_t st);
 
-// Each handle holds the staging memory; it is freed with the last of them.
+// Each handle holds the staging memory; what the last of them leaves is one
+// lane at most (sfv_transfer.hip).
 void staging_retain();
 void staging_release();
 

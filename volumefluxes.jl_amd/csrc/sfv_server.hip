@@ -75,6 +75,11 @@ struct sfv_server {
     sfv::DevicePool pool;              // worker-owned: device blocks, streams, pinned mirrors of finished requests
     std::chrono::steady_clock::time_point start = std::chrono::steady_clock::now();
 
+    // Its requests' handles come and go: the memory their downloads are staged
+    // through stays as long as the server.
+    sfv_server() { sfv::staging_retain(); }
+    ~sfv_server() { sfv::staging_release(); }
+
     double now() const {
         return std::chrono::duration<double>(std::chrono::steady_clock::now() - start).count();
     }

@@ -217,6 +217,13 @@ void staging_release() {
     }
 }
 
+int staging_lanes() {
+    std::lock_guard<std::mutex> lk(g_mu);
+    int n = 0;
+    for (const Lane& l : g_lanes) n += l.memory != nullptr;
+    return n;
+}
+
 hipError_t copy_to_host(void* dst, const void* src, size_t n, hipStream_t st) {
     int device = 0;
     if (n < MIN_STAGED || hipGetDevice(&device) != hipSuccess || runtime_memory(dst)) return plain(dst, src, n, st);

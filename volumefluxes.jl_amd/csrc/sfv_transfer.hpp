@@ -13,9 +13,11 @@ namespace sfv {
 // pinned and device memory included.  Any number of threads may copy at once.
 hipError_t copy_to_host(void* dst, const void* src, size_t n, hipStream_t st);
 
-// Each handle holds the staging memory; what the last of them leaves is one
+// Each handle and each server holds the staging memory; what the last of them leaves is one
 // lane at most (sfv_transfer.hip).
 void staging_retain();
 void staging_release();
+// Lanes that hold memory at present.
+int staging_lanes();
 
 }  // namespace sfv

@@ -194,7 +194,9 @@ int sfv_synchronize(sfv_handle* h);
 
 /* Bytes of device memory the handle holds (for budgeting). */
 int64_t sfv_device_bytes(const sfv_handle* h);
-/* Bytes of device memory a handle with this configuration would hold. */
+/* Bytes of device memory a handle with this configuration would hold once it
+ * has run (ForwardEuler handles, and RungeKutta2 ones with NeumannBC, take a
+ * fourth state-sized buffer with their first steps). */
 int64_t sfv_device_bytes_for(const sfv_config* cfg);
 
 /* Kernel-timing hook for measurement: run n RK2 steps' kernels from the

@@ -464,7 +464,7 @@ int run_loop(sfv_handle* h, double t0, double endtime, int match_endtime, int ha
     const bool euler = h->fused == KV_HYBRID && h->cfg.stepper == SFV_FORWARD_EULER && h->ghosts_settled();
     // a second right-hand side is needed; without the memory for it each step
     // takes two launches
-    bool piped = euler && max_steps != 1 && (!h->P.ghost_self || h->P.gc == 2);
+    bool piped = euler && max_steps != 1 && h->euler_piped();
     if (piped) {
         std::string why;
         if (h->ensure_scratch(why) != SFV_OK) {
@@ -588,17 +588,20 @@ int64_t sfv_device_bytes_for(const sfv_config* c) {
     if (!c) return -1;
     const int64_t nxT = c->nx + 2 * (int64_t)c->gc, nyT = c->ny + 2 * (int64_t)c->gc;
     const int64_t elem = c->precision == SFV_F32_STORAGE ? 4 : 8;
-    // ping-pong pair + right-hand side (+ the stage-1 state of the per-pass
-    // path, which RK2 grids the fused kernels cannot take use)
+    // ping-pong pair + right-hand side, and U[2] where the default kernels use
+    // it: the stage-1 state of RK2 grids the fused kernels cannot take, the
+    // second right-hand side of ForwardEuler loops
     int64_t nstate = 3;
-    if (c->stepper == SFV_RUNGE_KUTTA2) {
+    if (c->gc >= 1 && c->gc <= MAX_GC && c->nx >= 1 && c->ny >= 1) {
         sfv_handle probe;
         probe.cfg = *c;
         probe.build_params();
-        if (!probe.fusable()) nstate = 4;
+        if (probe.uses_scratch()) nstate = 4;
     }
-    int64_t b = nstate * 3 * nxT * nyT * elem + (nxT + 1) * (nyT + 1) * 8 + 4096;
+    int64_t b = nstate * 3 * nxT * nyT * elem + (nxT + 1) * (nyT + 1) * 8 + 4096;   // the last: the step control
     if (c->infiltration == SFV_INFILTRATION_HORTON) b += nxT * nyT * 8;
+    if (c->rain == SFV_RAIN_FIELD) b += nxT * nyT * 8;
+    if (c->rain == SFV_RAIN_TIME_TABLE && c->rain_table_len > 0) b += 2 * (int64_t)c->rain_table_len * 8;
     return b;
 }
 

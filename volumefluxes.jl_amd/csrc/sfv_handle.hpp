@@ -272,6 +272,17 @@ struct sfv_handle {
     // boundary-condition sources, which must then be interior cells.
     bool fusable() const { return cfg.stepper == SFV_RUNGE_KUTTA2 && ghost_sources_interior(); }
 
+    // ForwardEuler loops of more than one step take one launch a step where
+    // ghosts can be read through the maps; where a ghost is its own source the
+    // stage writes it too, which it does for gc = 2.  (A FunctionalRain handle
+    // takes single steps only.)
+    bool euler_piped() const {
+        return cfg.stepper == SFV_FORWARD_EULER && cfg.rain != SFV_RAIN_FIELD && ghosts_settled() &&
+               (!P.ghost_self || P.gc == 2);
+    }
+    // Do the default kernels of a configuration hold U[2]?
+    bool uses_scratch() const { return cfg.stepper == SFV_RUNGE_KUTTA2 ? !fusable() : euler_piped(); }
+
     ~sfv_handle() {
         if (stream) (void)hipStreamSynchronize(stream);
         if (staging) sfv::staging_release();

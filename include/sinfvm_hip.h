@@ -125,7 +125,11 @@ int sfv_set_topography(sfv_handle* h, const double* B, int64_t nbx, int64_t nby)
 /* set_current_state! (simulator.jl:119-135).  SFV_LAYOUT_INTERIOR: U is
  * (nx, ny, 3); the interior is written and the boundary condition applied,
  * other ghost cells keep their values.  SFV_LAYOUT_FULL: U is (nxT, nyT, 3)
- * and is copied verbatim (a checkpoint restore).  Element type is double for
+ * and is copied verbatim (a checkpoint restore).  Ghost cells that differ from
+ * what the boundary condition would give are taken as they are by the next
+ * step's right-hand side with NeumannBC and wherever the per-pass or hybrid
+ * kernels run; the fused RungeKutta2 kernels, and ForwardEuler with WallBC or
+ * PeriodicBC, take the boundary condition's.  Element type is double for
  * SFV_F64 and float for SFV_F32_STORAGE. */
 int sfv_set_state(sfv_handle* h, const void* U, int32_t layout);
 /* collect(current_state(sim)) / current_interior_state (simulator.jl:98-113). */
@@ -221,8 +225,9 @@ int sfv_device_count(void);
  * updates from the per-pass kernels, or for ForwardEuler both in one launch a
  * step (any stepper and boundary condition with gc >= 2: the default for
  * NeumannBC and ForwardEuler); 0 = one kernel per reference pass (the device-side
- * reference).  All give bitwise identical results.  No counterpart in the
- * reference. */
+ * reference).  All give bitwise identical results from a state whose ghost cells
+ * agree with the boundary condition (sfv_set_state has the other case).  No
+ * counterpart in the reference. */
 int sfv_set_fused(sfv_handle* h, int32_t fused);
 /* The kernel variant a step of this handle runs (0 to 3 as above; -1 for a
  * NULL handle).  No counterpart in the reference. */

@@ -40,8 +40,10 @@ int fail(sfv_handle* h, int code, const std::string& msg) {
             return fail((h), SFV_ERR_HIP, std::string(#expr) + ": " + hipGetErrorString(e_));        \
     } while (0)
 
+// One step; first: of its loop, when the state's ghosts are still in memory as
+// they were given.
 template <class S>
-int step_kernels(sfv_handle* h, int slot, int cur) {
+int step_kernels(sfv_handle* h, int slot, int cur, bool first) {
     const KParams& P = h->P;
     hipStream_t st = h->stream;
     S* U0 = (S*)h->U[cur];
@@ -64,9 +66,11 @@ int step_kernels(sfv_handle* h, int slot, int cur) {
         // after dt was taken from them; the slot is re-armed before its next use
         S* U1 = (S*)h->U[2];
         if (h->ghosts_settled()) {
-            // both right-hand sides read ghosts through the boundary maps and
-            // the second update closes the step; ghosts are filled when the loop ends
-            HIP_TRY(h, rhs(U0, 1));
+            // right-hand sides read ghosts through the boundary maps, but for the
+            // loop's first, which takes them as given (a state restored verbatim may
+            // hold others), and the second update closes the step; ghosts are filled
+            // when the loop ends
+            HIP_TRY(h, rhs(U0, first ? 0 : 1));
             HIP_TRY(h, launch_finish<S>(st, P, h->ctl, slot, 1, U0, U0, RHS, U1, h->B, 1));
             HIP_TRY(h, rhs(U1, 1));
             HIP_TRY(h, launch_finish<S>(st, P, h->ctl, slot, 2, U0, U1, RHS, U2, h->B, 1, 1 - slot));
@@ -110,7 +114,7 @@ int step_kernels(sfv_handle* h, int slot, int cur) {
 
 // ForwardEuler steps first .. first+n-1 of a loop that was prepared for slot 0
 // and ends after max_steps (<= 0: open), ghosts read through the boundary
-// maps.  piped: step 0's right-hand side comes from stage 1, then every launch
+// maps (but for a NeumannBC loop's first step, which takes them as given).  piped: step 0's right-hand side comes from stage 1, then every launch
 // finishes its step and finds the next one's right-hand side (stage 3) until
 // the loop's last step, which the update closes.  Otherwise each step is
 // stage 1 and the update.  One launch a step instead of two (three with
@@ -120,24 +124,25 @@ int step_kernels(sfv_handle* h, int slot, int cur) {
 template <class S>
 int euler_steps(sfv_handle* h, int64_t first, int64_t n, int64_t max_steps, bool piped) {
     const KParams& P = h->P;
-    auto stage = [&](int which, int slot, const S* U0, const S* R, S* out, S* uo) {
-        return h->rows_forced ? launch_march<S>(h->stream, P, h->ctl, slot, which, U0, R, out, h->B, 1, 1, uo)
-                              : launch_stage<S>(h->stream, P, h->ctl, slot, which, U0, R, out, h->B, 1, 1, uo);
+    auto stage = [&](int which, int slot, const S* U0, const S* R, S* out, S* uo, int remap = 1) {
+        return h->rows_forced ? launch_march<S>(h->stream, P, h->ctl, slot, which, U0, R, out, h->B, 1, remap, uo)
+                              : launch_stage<S>(h->stream, P, h->ctl, slot, which, U0, R, out, h->B, 1, remap, uo);
     };
+    const int first_remap = h->ghost_sources_interior() ? 1 : 0;
     for (int64_t s = first; s < first + n; ++s) {
         const int slot = (int)(s % 3);
         const S* U0 = (const S*)h->U[(h->cur + s) & 1];
         S* U1 = (S*)h->U[(h->cur + s + 1) & 1];
         S* R = (S*)(piped && (s & 1) ? h->U[2] : h->RHS);
         S* Rn = (S*)(s & 1 ? h->RHS : h->U[2]);
-        if (!piped || s == 0) HIP_TRY(h, stage(1, slot, U0, nullptr, R, nullptr));
+        if (!piped || s == 0) HIP_TRY(h, stage(1, slot, U0, nullptr, R, nullptr, s == 0 ? first_remap : 1));
         if (piped && s != max_steps - 1) HIP_TRY(h, stage(3, slot, U0, R, Rn, U1));
         else HIP_TRY(h, launch_finish<S>(h->stream, P, h->ctl, slot, 1, U0, U0, R, U1, h->B, 1, next_of_three(slot)));
     }
     return SFV_OK;
 }
 
-int launch_steps(sfv_handle* h, int64_t nsteps) {
+int launch_steps(sfv_handle* h, int64_t nsteps, bool first) {
     if (h->cfg.stepper == SFV_RUNGE_KUTTA2 && (h->fused == KV_PER_PASS || h->fused == KV_HYBRID)) {
         std::string why;
         const int rc = h->ensure_scratch(why);
@@ -146,8 +151,8 @@ int launch_steps(sfv_handle* h, int64_t nsteps) {
     for (int64_t s = 0; s < nsteps; ++s) {
         const int slot = (int)((h->step_parity + s) & 1);
         const int cur = (int)((h->cur + s) & 1);
-        const int rc = h->cfg.precision == SFV_F64 ? step_kernels<double>(h, slot, cur)
-                                                   : step_kernels<float>(h, slot, cur);
+        const int rc = h->cfg.precision == SFV_F64 ? step_kernels<double>(h, slot, cur, first && s == 0)
+                                                   : step_kernels<float>(h, slot, cur, first && s == 0);
         if (rc) return rc;
     }
     return SFV_OK;
@@ -499,7 +504,7 @@ int run_loop(sfv_handle* h, double t0, double endtime, int match_endtime, int ha
             const int64_t save_cur = h->cur, save_par = h->step_parity;
             h->cur = (save_cur + launched) & 1;
             h->step_parity = (save_par + launched) & 1;
-            rc = launch_steps(h, nb);
+            rc = launch_steps(h, nb, launched == 0);
             h->cur = save_cur;
             h->step_parity = save_par;
         }

@@ -1052,15 +1052,24 @@ struct SideStream {
         }                                                                                            \
     } while (0)
 
-// One step U0 -> U2 of the forward pass with the march kernels, in step
+// A stage of a step with the kernels the handle's steps take: a variant or a
+// segment height that was set on the handle holds here too, otherwise the
+// workgroup kernels where they suit the grid, as in an open handle's steps.
+hipError_t stage(sfv_handle* h, hipStream_t st, int slot, int which, const double* U0, const double* R, double* out,
+                 int close, int remap, double* UO = nullptr) {
+    const bool march = h->rows_forced || (h->variant_forced && h->fused == KV_MARCH);
+    const bool block = h->variant_forced && h->fused == KV_TILED;
+    auto launch = block ? launch_block<double> : march ? launch_march<double> : launch_stage<double>;
+    return launch(st, h->P, h->ctl, slot, which, U0, R, out, h->B, close, remap, UO);
+}
+
+// One step U0 -> U2 of the forward pass with the stage kernels, in step
 // slot `slot` of a loop prepared once (stage 2 advances t and arms the next
 // slot; U2's ghost cells are left unwritten and filled where a state leaves
-// the march path).  The adjoint accepts only handles the march path serves.
+// those kernels).  The adjoint accepts only handles that they serve.
 int march_step(sfv_handle* h, int slot, const double* U0, double* U2) {
-    const KParams& P = h->P;
-    hipStream_t st = h->stream;
-    ATRY(launch_stage<double>(st, P, h->ctl, slot, 1, U0, nullptr, (double*)h->RHS, h->B, 0, 1));
-    ATRY(launch_stage<double>(st, P, h->ctl, slot, 2, U0, (const double*)h->RHS, U2, h->B, 1));
+    ATRY(stage(h, h->stream, slot, 1, U0, nullptr, (double*)h->RHS, 0, 1));
+    ATRY(stage(h, h->stream, slot, 2, U0, (const double*)h->RHS, U2, 1, 0));
     return SFV_OK;
 }
 
@@ -1070,8 +1079,8 @@ int march_step(sfv_handle* h, int slot, const double* U0, double* U2) {
 int forward_step(sfv_handle* h, hipStream_t st, int slot, const double* U0, double* U1, double* R1, double* R2,
                  double* U2, ad::AdjStep* keep) {
     const KParams& P = h->P;
-    ATRY(launch_stage<double>(st, P, h->ctl, slot, 1, U0, nullptr, R1, h->B, 0, 1));
-    ATRY(launch_stage<double>(st, P, h->ctl, slot, 4, U0, R1, R2, h->B, 0, 1, U1));
+    ATRY(stage(h, st, slot, 1, U0, nullptr, R1, 0, 1));
+    ATRY(stage(h, st, slot, 4, U0, R1, R2, 0, 1, U1));
     hipLaunchKernelGGL(ad::k_adj_finish, dim3((P.nxT + 63) / 64, (P.nyT + 3) / 4), dim3(64, 4), 0, st, P, h->ctl, slot,
                        U0, U1, R2, U2, h->B, keep);
     ATRY(hipPeekAtLastError());

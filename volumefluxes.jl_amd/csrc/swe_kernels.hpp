@@ -90,7 +90,8 @@ hipError_t launch_interior_copy(hipStream_t st, const KParams& P, const void* pa
 // and its wave speeds to that slot.  Where a ghost's source is a ghost
 // (KParams::ghost_self), it writes the high-side ghosts of UO too; this
 // needs gc = 2.  stage = 4: as stage 3, but the step stays open: the
-// right-hand side of UO is taken at its time and no speeds are raised.
+// right-hand side of UO is taken at its time and no speeds are raised (double
+// only: hipErrorInvalidValue for float).
 template <class S>
 hipError_t launch_march(hipStream_t st, const KParams& P, StepCtl* ctl, int slot, int stage, const S* U0,
                         const S* RHS1, S* OUT, const double* B, int close = 0, int remap_halo = 0, S* UO = nullptr);

@@ -362,12 +362,13 @@ static void by_waves(int H, F&& go) {
 template <class S>
 hipError_t launch_block(hipStream_t st, const KParams& P, StepCtl* ctl, int slot, int stage, const S* U0,
                         const S* RHS1, S* OUT, const double* B, int close, int remap_halo, S* UO) {
+    if (stage > LAUNCH_STAGES<S>) return hipErrorInvalidValue;
     int H = block_height(P);
     if (H <= 0 || H > BLOCK_MAX_ROWS) H = BLOCK_MAX_ROWS;   // asked for on a larger grid: several rounds
     const int strips = (P.nx + BCOLS - 1) / BCOLS, segs = (P.ny + H - 1) / H;
     by_waves(H, [&](auto waves) {
         constexpr int BW = decltype(waves)::value;
-        by_stage_mode<4>(stage, stage == 3 && P.ghost_self ? MODE_GENERAL : march_mode(P), [&](auto stg, auto mode) {
+        by_stage_mode<LAUNCH_STAGES<S>>(stage, stage == 3 && P.ghost_self ? MODE_GENERAL : march_mode(P), [&](auto stg, auto mode) {
             hipLaunchKernelGGL((k_block<S, decltype(stg)::value, decltype(mode)::value, BW>), dim3(strips * segs + (decltype(stg)::value >= 2 ? 1 : 0)),
                                dim3(BL * BW), 0, st, P, ctl, slot, H, strips, segs, U0, RHS1, OUT, UO, B, remap_halo,
                                close);

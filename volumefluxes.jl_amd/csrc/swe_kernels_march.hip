@@ -603,10 +603,11 @@ int march_rows_per_wave(const KParams& P, int stage, int precision) {
 template <class S>
 hipError_t launch_march(hipStream_t st, const KParams& P, StepCtl* ctl, int slot, int stage, const S* U0,
                         const S* RHS1, S* OUT, const double* B, int close, int remap_halo, S* UO) {
+    if (stage > LAUNCH_STAGES<S>) return hipErrorInvalidValue;
     const int my = P.rows > 0 ? P.rows : march_rows_per_wave(P, stage, std::is_same<S, float>::value ? 1 : 0);
     const int segs = (P.ny + my - 1) / my;
     const int strips = (P.nx + MX - 1) / MX;
-    by_stage_mode<4>(stage, stage == 3 && P.ghost_self ? MODE_GENERAL : march_mode(P), [&](auto stg, auto mode) {
+    by_stage_mode<LAUNCH_STAGES<S>>(stage, stage == 3 && P.ghost_self ? MODE_GENERAL : march_mode(P), [&](auto stg, auto mode) {
         hipLaunchKernelGGL((k_march<S, decltype(stg)::value, decltype(mode)::value>), dim3(march_blocks(strips, segs) + (decltype(stg)::value >= 2 ? 1 : 0)),
                            dim3(MW * MWAVES), 0, st, P, ctl, slot, my, strips, segs, U0, RHS1, OUT, UO, B, close,
                            remap_halo);

@@ -383,11 +383,15 @@ inline void by_stage_mode(int stage, int mode, F&& go) {
         else go(st, std::integral_constant<int, MODE_GENERAL>{});
     };
     if (stage == 1) return with(std::integral_constant<int, 1>{});
-    if constexpr (STAGES == 4) {
+    if constexpr (STAGES >= 3)
         if (stage == 3) return with(std::integral_constant<int, 3>{});
+    if constexpr (STAGES >= 4)
         if (stage == 4) return with(std::integral_constant<int, 4>{});
-    }
     with(std::integral_constant<int, 2>{});
 }
+// The stages a launch of storage type S has: the adjoint, whose steps take
+// stage 4, is double only.
+template <class S>
+constexpr int LAUNCH_STAGES = std::is_same<S, double>::value ? 4 : 3;
 
 }  // namespace sfv

@@ -419,9 +419,11 @@ int fill_ghosts(sfv_handle* h, StepReport* report = nullptr) {
 
 // Wait until the steps of this loop that the device has reported done are more
 // than `done`, or the run has ended: done and active follow the word the
-// closing kernels write (StepReport).  Where the stream runs dry first,
-// the control block itself is read.
-int await_progress(sfv_handle* h, int64_t& done, bool& active) {
+// closing kernels write (StepReport).  Where the stream runs dry first, the
+// control block itself is read: every launched step has closed or passed its
+// inactivity on, so the run goes on if next_slot, the slot of the step after
+// them, is active (a finished step's own slot stays so).
+int await_progress(sfv_handle* h, int next_slot, int64_t& done, bool& active) {
     const auto began = std::chrono::steady_clock::now();
     for (long spin = 0;; ++spin) {
         const unsigned long long p = __atomic_load_n(&h->report()->word, __ATOMIC_ACQUIRE);
@@ -447,7 +449,7 @@ int await_progress(sfv_handle* h, int64_t& done, bool& active) {
         done = h->ctl_host->steps;
         h->report()->t = h->ctl_host->t;
         h->report()->dt = h->ctl_host->dt;
-        active = h->ctl_host->slot[0].active || h->ctl_host->slot[1].active || h->ctl_host->slot[2].active;
+        active = h->ctl_host->slot[next_slot].active != 0;
         return SFV_OK;
     }
 }
@@ -487,9 +489,10 @@ int run_loop(sfv_handle* h, double t0, double endtime, int match_endtime, int ha
                               (long long)max_steps, until_endtime, h->cfg.precision,
                               until_endtime ? h->report() : nullptr));
     int64_t launched = 0, done = 0;
+    auto next_slot = [&] { return (int)(euler ? launched % 3 : (slot0 + launched) & 1); };
     while (active && (max_steps <= 0 || launched < max_steps)) {
         if (until_endtime && launched - done >= AHEAD) {
-            const int rc = await_progress(h, done, active);
+            const int rc = await_progress(h, next_slot(), done, active);
             if (rc) return rc;
             continue;
         }
@@ -522,7 +525,7 @@ int run_loop(sfv_handle* h, double t0, double endtime, int match_endtime, int ha
         h->step_parity = (h->step_parity + 1) & 1;
         const int rf = fill_ghosts(h, h->report());
         if (rf) return rf;
-        const int rc = await_progress(h, done, active);
+        const int rc = await_progress(h, next_slot(), done, active);
         if (rc) return rc;
         t = h->report()->t;
         dt = h->report()->dt;

@@ -311,7 +311,8 @@ int cached_march_rows(sfv_handle* h) {
 
 int tune_march_rows(sfv_handle* h, std::string& why) {
     if ((h->fused != KV_MARCH && h->fused != KV_HYBRID) || h->march_rows > 0) return SFV_OK;
-    const bool block = !h->variant_forced && block_suits(h->P);
+    // (the hybrid kernels' launches choose by the grid alone)
+    const bool block = (h->fused == KV_HYBRID || !h->variant_forced) && block_suits(h->P);
     const int fallback = march_rows_per_wave(h->P, 1, h->cfg.precision == SFV_F64 ? 0 : 1);
     if (block || !autotune_enabled()) {
         h->march_rows = fallback;

@@ -183,13 +183,14 @@ int ensure_ready(sfv_handle* h) {
 // octaves of nx and ny).  Where the workgroup kernels suit the grid
 // (block_suits), nothing is measured: a march handle whose kernel variant was
 // not set with sfv_set_fused switches to them.  Handles on the hybrid path
-// (ForwardEuler, NeumannBC) run only the stage-1 kernel, so they time it alone
-// and keep
-// their own cache entries.  Every height gives bitwise the same results.
+// time the one stage kernel of their steps and have their own cache entries:
+// stage 1 (RungeKutta2 with NeumannBC, single ForwardEuler steps), or stage 3
+// for ForwardEuler loops.  Every height gives bitwise the same results.
 // SFV_AUTOTUNE=0 in the environment keeps the height model's choice
 // (march_rows_per_wave).
+enum { TUNE_STEPS = 0, TUNE_STAGE1 = 1, TUNE_STAGE3 = 2 };   // what is timed
 struct TuneKey {
-    int dev, prec, bx, by, kind;   // kind: 0 full march steps, 1 stage 1 only
+    int dev, prec, bx, by, kind;
     bool operator<(const TuneKey& o) const {
         if (dev != o.dev) return dev < o.dev;
         if (prec != o.prec) return prec < o.prec;
@@ -204,17 +205,20 @@ std::map<TuneKey, int> g_tuned;   // the march height
 int size_bucket(int n) { return (int)std::lround(4.0 * std::log2((double)std::max(n, 1))); }
 
 template <class S>
-hipError_t tune_steps(sfv_handle* h, int slot, int n) {
+hipError_t tune_steps(sfv_handle* h, int kind, int slot, int n) {
     const KParams& P = h->P;
     const int cur = (int)(h->cur & 1);
     const S* U0 = (const S*)h->U[cur];
     S* R = (S*)h->RHS;
     S* Us = (S*)h->U[cur ^ 1];
     hipError_t e = hipSuccess;
-    for (int k = 0; k < n && e == hipSuccess; ++k) {
+    for (int k = 0; k < n && e == hipSuccess; ++k) {           // none closes its step
+        if (kind == TUNE_STAGE3) {
+            e = launch_march<S>(h->stream, P, h->ctl, slot, 3, U0, R, (S*)h->U[2], h->B, 0, 1, Us);
+            continue;
+        }
         e = launch_march<S>(h->stream, P, h->ctl, slot, 1, U0, nullptr, R, h->B, 0, h->ghosts_settled() ? 1 : 0);
-        if (h->fused == KV_HYBRID) continue;
-        if (e == hipSuccess) e = launch_march<S>(h->stream, P, h->ctl, slot, 2, U0, R, Us, h->B);   // not closing
+        if (kind == TUNE_STEPS && e == hipSuccess) e = launch_march<S>(h->stream, P, h->ctl, slot, 2, U0, R, Us, h->B);
     }
     return e;
 }
@@ -297,32 +301,32 @@ bool autotune_enabled() {
     return !(e && e[0] == '0');
 }
 
-int cached_march_rows(sfv_handle* h) {
-    if (h->march_rows > 0) return h->march_rows;
-    const TuneKey key{h->device, h->cfg.precision, size_bucket(h->cfg.nx), size_bucket(h->cfg.ny),
-                      h->fused == KV_HYBRID ? 1 : 0};
-    std::lock_guard<std::mutex> lk(g_tune_mu);
-    auto it = g_tuned.find(key);
-    if (it == g_tuned.end()) return 0;
-    h->march_rows = it->second;
-    h->P.rows = it->second;
-    return it->second;
-}
-
-int tune_march_rows(sfv_handle* h, std::string& why) {
-    if ((h->fused != KV_MARCH && h->fused != KV_HYBRID) || h->march_rows > 0) return SFV_OK;
+int tune_march_rows(sfv_handle* h, bool piped, std::string& why) {
+    if (h->fused != KV_MARCH && h->fused != KV_HYBRID) return SFV_OK;
+    const int kind = h->fused == KV_MARCH ? TUNE_STEPS : piped ? TUNE_STAGE3 : TUNE_STAGE1;
+    // a height measured for single ForwardEuler steps is measured again for loops
+    if (h->march_rows > 0 && (h->rows_forced || kind != TUNE_STAGE3 || h->tuned_kind != TUNE_STAGE1)) return SFV_OK;
+    h->tuned_kind = kind;
     // (the hybrid kernels' launches choose by the grid alone)
     const bool block = (h->fused == KV_HYBRID || !h->variant_forced) && block_suits(h->P);
-    const int fallback = march_rows_per_wave(h->P, 1, h->cfg.precision == SFV_F64 ? 0 : 1);
+    const int fallback = march_rows_per_wave(h->P, kind == TUNE_STAGE3 ? 3 : 1, h->cfg.precision == SFV_F64 ? 0 : 1);
     if (block || !autotune_enabled()) {
         h->march_rows = fallback;
         h->P.rows = fallback;
         if (block && h->fused == KV_MARCH) h->fused = KV_TILED;
         return SFV_OK;
     }
-    if (cached_march_rows(h) > 0) return SFV_OK;
-    const TuneKey key{h->device, h->cfg.precision, size_bucket(h->cfg.nx), size_bucket(h->cfg.ny),
-                      h->fused == KV_HYBRID ? 1 : 0};
+    const TuneKey key{h->device, h->cfg.precision, size_bucket(h->cfg.nx), size_bucket(h->cfg.ny), kind};
+    {
+        std::lock_guard<std::mutex> lk(g_tune_mu);
+        auto it = g_tuned.find(key);
+        if (it != g_tuned.end()) {
+            h->march_rows = it->second;
+            h->P.rows = it->second;
+            return SFV_OK;
+        }
+    }
+    h->march_rows = 0;
     std::vector<int> cand;
     for (int c : {1, 2, 3, 4, 6, 8, 12, 16, 24})
         if (c <= h->cfg.ny) cand.push_back(c);
@@ -345,13 +349,18 @@ int tune_march_rows(sfv_handle* h, std::string& why) {
     if (e == hipSuccess) e = hipEventCreate(&e1);
     if (e == hipSuccess)
         e = launch_prepare(h->stream, h->P, h->ctl, slot, 0.0, NAN, 0, 0, 0.0, -1, 0, h->cfg.precision);
+    // stage 3 starts from a right-hand side and its wave speeds
+    if (e == hipSuccess && kind == TUNE_STAGE3) {
+        h->P.rows = fallback;
+        e = f64 ? tune_steps<double>(h, TUNE_STAGE1, slot, 1) : tune_steps<float>(h, TUNE_STAGE1, slot, 1);
+    }
     // time n steps with `rows`; the first call also sizes n so one
     // measurement covers about a millisecond
     auto timed = [&](int rows, int n, double& ms_out) -> hipError_t {
         h->P.rows = rows;
-        hipError_t r = f64 ? tune_steps<double>(h, slot, 1) : tune_steps<float>(h, slot, 1);  // warm-up
+        hipError_t r = f64 ? tune_steps<double>(h, kind, slot, 1) : tune_steps<float>(h, kind, slot, 1);  // warm-up
         if (r == hipSuccess) r = hipEventRecord(e0, h->stream);
-        if (r == hipSuccess) r = f64 ? tune_steps<double>(h, slot, n) : tune_steps<float>(h, slot, n);
+        if (r == hipSuccess) r = f64 ? tune_steps<double>(h, kind, slot, n) : tune_steps<float>(h, kind, slot, n);
         if (r == hipSuccess) r = hipEventRecord(e1, h->stream);
         if (r == hipSuccess) r = hipEventSynchronize(e1);
         float ms = 0;
@@ -394,7 +403,8 @@ int tune_march_rows(sfv_handle* h, std::string& why) {
     h->march_rows = pick;
     h->P.rows = pick;
     if (const char* dbg = std::getenv("SFV_TUNE_REPORT"); dbg && dbg[0] == '1') {
-        std::fprintf(stderr, "[sfv autotune] %dx%d %s:", h->cfg.nx, h->cfg.ny, f64 ? "f64" : "f32");
+        std::fprintf(stderr, "[sfv autotune] %dx%d %s, %s:", h->cfg.nx, h->cfg.ny, f64 ? "f64" : "f32",
+                     kind == TUNE_STEPS ? "steps" : kind == TUNE_STAGE1 ? "stage 1" : "stage 3");
         for (size_t c = 0; c < cand.size(); ++c) std::fprintf(stderr, " %d:%.4f", cand[c], best[c]);
         std::fprintf(stderr, " -> %d (ms per step, %d steps per timing)\n", pick, n);
     }
@@ -464,22 +474,17 @@ int await_progress(sfv_handle* h, int next_slot, int64_t& done, bool& active) {
 constexpr int64_t AHEAD = 12;
 int run_loop(sfv_handle* h, double t0, double endtime, int match_endtime, int has_max, double max_ts,
              int64_t max_steps, int until_endtime, int64_t* steps_out, double* t_out) {
-    {
-        std::string why;
-        const int rt = sfv::tune_march_rows(h, why);
-        if (rt) return fail(h, rt, why);
-    }
     const bool euler = h->fused == KV_HYBRID && h->cfg.stepper == SFV_FORWARD_EULER && h->ghosts_settled();
     // a second right-hand side is needed; without the memory for it each step
     // takes two launches
     bool piped = euler && max_steps != 1 && h->euler_piped();
-    if (piped) {
-        std::string why;
-        if (h->ensure_scratch(why) != SFV_OK) {
-            (void)hipGetLastError();
-            piped = false;
-        }
+    std::string why;
+    if (piped && h->ensure_scratch(why) != SFV_OK) {
+        (void)hipGetLastError();
+        piped = false;
     }
+    const int rt = sfv::tune_march_rows(h, piped, why);
+    if (rt) return fail(h, rt, why);
     const int slot0 = euler ? 0 : (int)(h->step_parity & 1);
     // a run that is over before it starts launches nothing
     bool active = !until_endtime || t0 < endtime;
@@ -761,7 +766,7 @@ int sfv_time_kernel(sfv_handle* h, const char* which, int32_t n, double* ms_out)
     HIP_TRY(h, hipSetDevice(h->device));
     {
         std::string why;
-        int rc2 = sfv::tune_march_rows(h, why);
+        int rc2 = sfv::tune_march_rows(h, false, why);
         if (!rc2) rc2 = h->ensure_scratch(why);
         if (rc2) return fail(h, rc2, why);
     }
@@ -844,6 +849,7 @@ int sfv_set_march_rows(sfv_handle* h, int32_t rows) {
     if (rows < 0 || rows > 1024) return fail(h, SFV_ERR_ARGUMENT, "rows must be in 0..1024");
     h->march_rows = rows;
     h->rows_forced = rows > 0;
+    h->tuned_kind = 0;
     h->P.rows = rows;
     return SFV_OK;
 }

@@ -108,6 +108,7 @@ struct sfv_handle {
     int fused = KV_MARCH;               // kernel variant, KV_*
     int march_rows = 0;                 // rows per march segment: 0 = not chosen yet (autotuned on first use)
     bool rows_forced = false;           // set by sfv_set_march_rows
+    int tuned_kind = 0;                 // what march_rows was chosen for (sfv_capi.hip)
     bool variant_forced = false;        // set by sfv_set_fused: the tuner keeps the variant
     std::string err;
     bool staging = false;               // holds the process's staging memory (sfv_transfer.hpp)
@@ -309,9 +310,8 @@ namespace sfv {
 int create_handle(const sfv_config* cfg, DevicePool* pool, sfv_handle** out, std::string& why);
 // Choose the march kernels' segment height for a handle (measured on the
 // handle's current state, cached per grid size class); a no-op once chosen.
-int tune_march_rows(sfv_handle* h, std::string& why);
-// The cached height for the handle's size class, without measuring (0: none yet).
-int cached_march_rows(sfv_handle* h);
+// piped: for a ForwardEuler loop of one launch a step (U[2] is there).
+int tune_march_rows(sfv_handle* h, bool piped, std::string& why);
 // False when SFV_AUTOTUNE=0 is set in the environment: no height is measured.
 bool autotune_enabled();
 }  // namespace sfv

@@ -549,6 +549,11 @@ int march_mode(const KParams& P) {
     return !fast ? MODE_GENERAL : P.dx_pow2 && P.dy_pow2 ? MODE_POW2 : MODE_FAST;
 }
 
+// The kernels of a stage: the ones that write ghosts are the general ones.
+static int stage_mode(const KParams& P, int stage) {
+    return stage == 3 && P.ghost_self ? MODE_GENERAL : march_mode(P);
+}
+
 // Rows per wave segment for this grid.  With w waves on each SIMD a launch
 // lasts about w (my + 4) / f(w): every wave marches my + 4 rows, the SIMD's
 // issue is shared, and fewer than four waves leave part of it idle.  Measured
@@ -564,7 +569,7 @@ static int march_resident_blocks() {
 }
 int march_rows_per_wave(const KParams& P, int stage, int precision) {
     if (SFV_MARCH_ROWS > 0) return SFV_MARCH_ROWS;
-    static int cus = 0, bpc[2][2][3];       // [precision][stage - 1][mode]
+    static int cus = 0, bpc[2][3][3];       // [precision][stage - 1][mode]
     static std::once_flag once;
     std::call_once(once, [] {
         int dev = 0;
@@ -572,7 +577,7 @@ int march_rows_per_wave(const KParams& P, int stage, int precision) {
         if (hipGetDevice(&dev) == hipSuccess && hipGetDeviceProperties(&prop, dev) == hipSuccess)
             cus = prop.multiProcessorCount;
         if (cus <= 0) cus = 256;
-        auto fill = [](auto s, int (&b)[2][3]) {
+        auto fill = [](auto s, int (&b)[3][3]) {
             using S = decltype(s);
             b[0][0] = march_resident_blocks<S, 1, 0>();
             b[0][1] = march_resident_blocks<S, 1, 1>();
@@ -580,12 +585,15 @@ int march_rows_per_wave(const KParams& P, int stage, int precision) {
             b[1][0] = march_resident_blocks<S, 2, 0>();
             b[1][1] = march_resident_blocks<S, 2, 1>();
             b[1][2] = march_resident_blocks<S, 2, 2>();
+            b[2][0] = march_resident_blocks<S, 3, 0>();
+            b[2][1] = march_resident_blocks<S, 3, 1>();
+            b[2][2] = march_resident_blocks<S, 3, 2>();
         };
         fill(double(), bpc[0]);
         fill(float(), bpc[1]);
     });
     // a workgroup puts one wave on each SIMD of its CU
-    const long resident = bpc[precision ? 1 : 0][stage == 1 ? 0 : 1][march_mode(P)];
+    const long resident = bpc[precision ? 1 : 0][std::min(stage, 3) - 1][stage_mode(P, stage)];
     const long strips = (P.nx + MX - 1) / MX;
     static const double f[5] = {1.0, 0.43, 0.70, 0.92, 1.0};
     auto round_time = [&](long w) { return (double)w / f[std::min(w, 4L)]; };
@@ -607,7 +615,7 @@ hipError_t launch_march(hipStream_t st, const KParams& P, StepCtl* ctl, int slot
     const int my = P.rows > 0 ? P.rows : march_rows_per_wave(P, stage, std::is_same<S, float>::value ? 1 : 0);
     const int segs = (P.ny + my - 1) / my;
     const int strips = (P.nx + MX - 1) / MX;
-    by_stage_mode<LAUNCH_STAGES<S>>(stage, stage == 3 && P.ghost_self ? MODE_GENERAL : march_mode(P), [&](auto stg, auto mode) {
+    by_stage_mode<LAUNCH_STAGES<S>>(stage, stage_mode(P, stage), [&](auto stg, auto mode) {
         hipLaunchKernelGGL((k_march<S, decltype(stg)::value, decltype(mode)::value>), dim3(march_blocks(strips, segs) + (decltype(stg)::value >= 2 ? 1 : 0)),
                            dim3(MW * MWAVES), 0, st, P, ctl, slot, my, strips, segs, U0, RHS1, OUT, UO, B, close,
                            remap_halo);

@@ -4,8 +4,9 @@
 // captured once in a HIP graph and replayed.
 //
 // Each member keeps its own buffers; the batch owns the member table the
-// kernels read, the members' step-control blocks (one contiguous array, so a
-// single copy reads every member's progress) and the graph.  Results are
+// kernels read, the members' step-control blocks (one array), the reports a
+// kernel writes of them to pinned memory after the replays, and the graph.
+// Results are
 // bitwise those of stepping each member alone: the kernels are the same
 // per-wave tile code, only the block-to-tile map differs.
 #include <hip/hip_runtime.h>
@@ -275,9 +276,9 @@ std::vector<long long> BatchEngine::signature() const {
 // else line up the timed trials: the rule's height, the next lower and the
 // two next higher candidates, the least height at which the batch's segments
 // fit the resident wave slots in one round (in place of a third higher
-// candidate; 16 grids of 128 to 1024 squared: 55.8 ms a run at 20 rows, 59.2 at
-// 12, whose one and a half rounds leave half the slots idle at the end), the
-// rule's height again.
+// candidate; 16 grids of 128 to 1024 squared, where that is 19 rows: 55.8 ms a
+// run at 20, 59.2 at 12, whose one and a half rounds leave half the slots idle
+// at the end), the rule's height again.
 void BatchEngine::plan_tuning() {
     trials_.clear();
     trial_ms_.clear();
@@ -327,9 +328,9 @@ int BatchEngine::upload_table(std::string& why) {
     return SFV_OK;
 }
 
-// graph_steps RK2 steps (stage 1, then stage 2, which also fills the ghosts
-// and closes each member's step), launch parity alternating 0, 1, ... on the
-// engine's stream.
+// graph_steps RK2 steps (stage 1, then stage 2, which also closes each
+// member's step; ghosts are filled when a member leaves, remove), launch parity
+// alternating 0, 1, ... on the engine's stream.
 int BatchEngine::capture(std::string& why) {
     ETRY(hipStreamBeginCapture(stream_, hipStreamCaptureModeThreadLocal));
     hipError_t e = hipSuccess;

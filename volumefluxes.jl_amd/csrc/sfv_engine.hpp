@@ -52,11 +52,11 @@ public:
     // steps into the handle (buffer parity, last dt).
     void remove(int slot);
 
-    // Replay the graph `k` times (k * graph_steps launched steps), then copy
-    // every slot's step control to the host and wait.
+    // Replay the graph `k` times (k * graph_steps launched steps), then have
+    // every member's report written to the host and wait.
     int replay(int k, std::string& why);
     // The same in two halves, so the host can work while the device steps:
-    // replay_begin queues the replays and the step-control copy; replay_end
+    // replay_begin queues the replays and the report launch; replay_end
     // waits for them.  Between the two, add / remove / finished / report must
     // not be called (they use the table and the members' reports).
     int replay_begin(int k, std::string& why);

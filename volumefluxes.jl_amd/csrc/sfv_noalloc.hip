@@ -21,7 +21,9 @@
 
 namespace {
 
-constexpr size_t CTL_BYTES = 256;                // ahead of the right-hand side (unused)
+// Left free ahead of the right-hand side: the documented cell limits are those
+// of an array that also held a control block of this size.
+constexpr size_t RESERVED = 256;
 constexpr size_t CTL_ARRAY = 4096;
 static_assert(sizeof(sfv::StepCtl) <= CTL_ARRAY, "StepCtl outgrew its array");
 
@@ -42,11 +44,11 @@ int fail(int code, const std::string& msg) {
     return code;
 }
 
-// Largest nxT*nyT whose right-hand side and second state fit the array
-// beside the control block (each rounded up to 256 bytes).
+// Largest nxT*nyT whose right-hand side and second state fit the array (each
+// rounded up to 256 bytes).
 int64_t max_cells(int32_t precision) {
     const size_t elem = precision == SFV_F32_STORAGE ? 4 : 8;
-    return (int64_t)((SFV_NOALLOC_SCRATCH_BYTES - CTL_BYTES - 512) / (2 * 3 * elem));
+    return (int64_t)((SFV_NOALLOC_SCRATCH_BYTES - RESERVED - 512) / (2 * 3 * elem));
 }
 
 size_t round_up(size_t b) { return (b + 255) / 256 * 256; }
@@ -78,7 +80,7 @@ int advance(const sfv::KParams& P, hipStream_t st, const Scratch& scr, const dou
     using namespace sfv;
     const size_t n3 = 3 * (size_t)P.nxT * P.nyT;
     StepCtl* ctl = (StepCtl*)scr.ctl;
-    S* RHS = (S*)((unsigned char*)scr.state + CTL_BYTES);
+    S* RHS = (S*)((unsigned char*)scr.state + RESERVED);
     S* other = (S*)((unsigned char*)RHS + round_up(n3 * sizeof(S)));
     S* buf[2] = {U, other};
     // the step control is armed by a kernel (no memset): every field a step

@@ -149,6 +149,15 @@ __device__ __forceinline__ int batch_find(const BatchMember* __restrict__ mem, i
     return lo;
 }
 
+__device__ __forceinline__ unsigned long long wave_max_u64(unsigned long long v) {
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+        const unsigned long long o = __shfl_xor(v, off, 64);
+        v = o > v ? o : v;
+    }
+    return v;
+}
+
 // Raise the slot's maximum speeds to at least (mx, my): one thread per block
 // calls it with its block's maxima.  Device-wide atomics on one address are
 // carried out one after the other, so hundreds of blocks that end together

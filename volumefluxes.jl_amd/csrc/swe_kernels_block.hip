@@ -336,17 +336,23 @@ static int block_height(const KParams& P) {
 
 // These kernels against the wave-march kernels, us per step (f64, same box):
 // 64x48 15.1 and 22.1, 256^2 18.3 and 23.6, 420^2 22.8 and 28.0, 512^2 31 and 35,
-// 700^2 (36 rows per workgroup) 46 and 44, 1024^2 86 and 74.  A workgroup's
-// eight or more rows in flight beat a wave's one after the other until a
-// CU's rows are more than about 24, the four-rows-in-flight limit per SIMD of
-// either kernel.
+// 700^2 (36 rows per workgroup) 46 and 44, 1024^2 86 and 74.  A workgroup's 6,
+// 10 or 16 rows in flight beat a wave's one after the other until a CU's rows are
+// more than about 24, the four-rows-in-flight limit per SIMD of either kernel.
+// Near the limit the order depends on the grid more than on the type, options
+// or stage (f64; f32 storage; general options; ForwardEuler, where the launch is
+// stage 3): at 19 rows 30.5 and 34.6; 29.8 and 34.7; 32.0 and 37.4; 18.7 and 20.1;
+// at 24 rows (600^2) 36.9 and 36.1; 38.5 and 36.3; 40.1 and 39.0; 21.0 and 20.6;
+// at 27 rows (619x610) 37.1 and 41.1; 41.8 and 43.9; 43.0 and 46.1; 25.2 and 25.7,
+// but (4000x80) 43.4 and 38.9; 41.9 and 38.7; 44.7 and 42.2; 25.1 and 23.4.
 bool block_suits(const KParams& P) {
     const int H = block_height(P);
     return P.gc >= 2 && H > 0 && H <= BLOCK_MAX_ROWS;
 }
 
 // A chunk of BW rows takes about 9 + BW units of time (two launches of one
-// chunk each: 15.0 us at 6 rows, 17.5 at 10, 22 at 16).
+// chunk each: 15.0 us at 6 rows, 17.5 at 10, 22 at 16).  Three sizes, so that
+// each stage and mode is built three times; sizes between were not measured.
 template <class F>
 static void by_waves(int H, F&& go) {
     int best = 6, cost = 1 << 30;

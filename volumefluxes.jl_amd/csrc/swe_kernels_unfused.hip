@@ -2,22 +2,14 @@
 // per cell.  They keep the reference's pass boundaries (flux/sources → RK
 // update + friction + clamp → boundary condition) and are the device-side
 // parity reference for the fused stage kernels (swe_kernels_march.hip,
-// swe_kernels_block.hip); the
-// Forward-Euler stepper and the boundary condition always use them.
+// swe_kernels_block.hip).  They run on request and for gc < 2; k_finish is also
+// the update of RungeKutta2 with NeumannBC and of a ForwardEuler loop's last
+// step.
 #include "swe_kernels.hpp"
 
 namespace sfv {
 
 // ---------------------------------------------------------------- reductions
-__device__ __forceinline__ unsigned long long wave_max_u64p(unsigned long long v) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-        const unsigned long long o = __shfl_xor(v, off, 64);
-        v = o > v ? o : v;
-    }
-    return v;
-}
-
 // Block max of two values, then one atomic per block into the step slot.
 // Speeds are >= +0.0 or NaN, whose bit patterns order like the values (and a
 // NaN orders above +Inf), so an unsigned max of the bits is max() with NaN
@@ -27,8 +19,8 @@ __device__ void block_max_to_slot(unsigned long long sx, unsigned long long sy, 
     const int tid = threadIdx.x + blockDim.x * threadIdx.y;
     const int lane = tid & 63, wid = tid >> 6;
     const int nw = (blockDim.x * blockDim.y + 63) >> 6;
-    sx = wave_max_u64p(sx);
-    sy = wave_max_u64p(sy);
+    sx = wave_max_u64(sx);
+    sy = wave_max_u64(sy);
     if (lane == 0) { red[0][wid] = sx; red[1][wid] = sy; }
     __syncthreads();
     if (tid == 0) {

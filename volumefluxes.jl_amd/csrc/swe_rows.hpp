@@ -13,9 +13,8 @@ namespace sfv {
 // VALU latency instead of an LDS round trip): lane i receives lane i-1
 // (shfl_up1) or lane i+1 (shfl_dn1).  Lane 0 (shfl_up1) / lane 63
 // (shfl_dn1) have no source lane and read zero; both are halo lanes whose
-// shifted values feed no output (the one exception, the corner column lane
-// 63 needs, is supplied separately by next_col).  With no old value to keep,
-// each shift is a single DPP move into a fresh register.
+// shifted values feed no output.  With no old value to keep, each shift is a
+// single DPP move into a fresh register.
 template <int CTRL>
 __device__ __forceinline__ int dpp_shift(int v) {
     return __builtin_amdgcn_mov_dpp(v, CTRL, 0xf, 0xf, true);
@@ -34,15 +33,6 @@ template <class T>
 __device__ __forceinline__ T shfl_up1(T v) { return dpp_shift<DPP_WAVE_SHR1>(v); }
 template <class T>
 __device__ __forceinline__ T shfl_dn1(T v) { return dpp_shift<DPP_WAVE_SHL1>(v); }
-
-__device__ __forceinline__ unsigned long long wave_max_u64(unsigned long long v) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-        const unsigned long long o = __shfl_xor(v, off, 64);
-        v = o > v ? o : v;
-    }
-    return v;
-}
 
 __device__ __forceinline__ double Bload(const KParams& P, const double* __restrict__ B, int i, int j) {
     return (i <= P.nxT && j <= P.nyT) ? B[(size_t)i + (size_t)(P.nxT + 1) * j] : 0.0;

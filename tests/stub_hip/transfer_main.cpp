@@ -51,7 +51,7 @@ int pageable() {
 }
 
 // Memory the runtime knows is written by one copy of its own.
-int known_destination(char* dst, bool device) {
+int known_destination(char* dst) {
     sfv::staging_retain();
     Source s(20 * MB);
     StubStream st;
@@ -63,15 +63,14 @@ int known_destination(char* dst, bool device) {
     int differs = 0;
     stub::with_access(dst, s.n, [&] { differs = std::memcmp(dst, s.want.data(), s.n); });
     CHECK(differs == 0);
-    (void)device;
     sfv::staging_release();
     return 0;
 }
-int device_destination() { return known_destination(stub::device_alloc(20 * MB), true); }
+int device_destination() { return known_destination(stub::device_alloc(20 * MB)); }
 int pinned_destination() {
     void* p = nullptr;
     CHECK(hipHostMalloc(&p, 20 * MB, hipHostMallocDefault) == hipSuccess);
-    return known_destination((char*)p, false);
+    return known_destination((char*)p);
 }
 
 // The caller's stream only waits: the copies run on another.

@@ -1,7 +1,7 @@
 // sfv_transfer.hip — device-to-host copies into pageable memory.
 //
 // hipMemcpy to pageable memory runs at 18 GB/s where the destination's pages
-// are mapped and at 4.4 GB/s where they are fresh (a new array's pages are
+// are mapped and at 4 to 10 GB/s where they are fresh (a new array's pages are
 // mapped one fault at a time), against 57 GB/s into pinned memory.  A copy
 // here goes through a ring of pinned slots: the calling thread queues the DMA
 // of the next chunks while worker threads empty the slots that have arrived,
@@ -16,9 +16,10 @@
 // runtime's own and one below MIN_STAGED: 6 MB gain 0.1 ms at most.
 //
 // A copy leaves nothing behind on the caller's stream, and no mapping of the
-// process changes: the runtime gives the queue of a destroyed stream to the next
-// one only if it is idle for good, and a new queue costs 1.1 ms and its first
-// uploads run at 2.6 GB/s.  With the DMAs on the caller's stream, or with
+// process changes.  A handle's stream is destroyed with it, and the next
+// handle's is as good as free where the runtime has that queue ready again;
+// where it has not (the same times come where streams are never destroyed),
+// a new queue costs 1.1 ms and its first uploads run at 2.6 GB/s.  With the DMAs on the caller's stream, or with
 // default-size stacks for eight threads (64 MB, more than the C library keeps
 // for reuse, so that every copy unmapped some), that met most handles made
 // after one was read and destroyed; making the lane again cost as much.  For a
